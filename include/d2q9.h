@@ -257,6 +257,44 @@ int d2q9_fused_step2(const d2q9_lattice* L, const d2q9_lattice* L_rim_a,
 /* Rows of a deep tile of d2q9_fused_step2. */
 int d2q9_deep_rows(void);
 
+/*
+ * Tiled sweep: n fused steps (as n calls of d2q9_fused_step, bitwise in every
+ * storage form), up to `steps` of them per launch.  A workgroup holds a
+ * region of rows x width cells in LDS (width 16, 32 or 64; at most 1024
+ * cells, one per thread) and stores what K steps leave valid of it, (rows -
+ * 2 K) x (width - 2 K) cells.  Every kind of cell is swept, so a launch is
+ * one kernel on `stream`.
+ *
+ * cells [plane] holds each cell's flags in bits 0..7 and, for a cell flagged
+ * D2Q9_CELL_NEAR_SOLID or D2Q9_CELL_BC, the number of its record above.
+ * codes holds four uint32 per record (16-byte aligned).  Bytes 0..7: where
+ * directions 1..8 stream from, (dr + 1) | (dc + 1) << 2 | k << 4 for
+ * population k of the cell at (i + dr, j + dc), dr and dc in -1..1 (never 0).
+ * Word 2: bit d - 1 set when direction d is a moving wall's or a
+ * fixed-pressure node's (its byte then names the cell's own opposite
+ * population), of boundary element bits 16..23, or of element bits 24..31
+ * when bit 7 + d is set too; has_vel and has_pres: some such element is of
+ * type D2Q9_RULE_VEL, D2Q9_RULE_PRES.  n_elems (at most 32) boundary
+ * elements are in bc_elems.  The solids must be at rest.
+ *
+ * The steps go f_a -> f_b -> f_a ... once per launch, ceil(n / steps)
+ * launches (the last one's target holds the result), the moments alike.
+ * collide_first: the first step is a d2q9_collide (no streaming).
+ * mom_steps (nullable): rho/u of every fluid cell after step s (0-based) at
+ * mom_steps + s * mom_stride elements, three planes each; mom_b is then not
+ * written.  mom_a holds rho/u of the step before, as for d2q9_fused_step.
+ */
+typedef struct d2q9_tiled_desc {
+  int32_t rows, width, steps;
+  int32_t n_elems, has_vel, has_pres;
+  const uint32_t* cells;
+  const uint32_t* codes;
+} d2q9_tiled_desc;
+
+int d2q9_tiled_steps(const d2q9_lattice* L, const d2q9_tiled_desc* D, void* f_a, void* f_b,
+                     void* mom_a, void* mom_b, int32_t n, int collide_first,
+                     int write_moments, void* mom_steps, int64_t mom_stride, void* stream);
+
 /* rho/u of the populations f (e.g. pop_new) on every fluid cell. */
 int d2q9_moments(const d2q9_lattice* L, const void* f, void* mom,
                  void* stream);

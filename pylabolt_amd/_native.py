@@ -97,6 +97,18 @@ class BatchItem(ctypes.Structure):
     _fields_ = [("lattice", ctypes.c_int32), ("code", ctypes.c_int32)]
 
 
+class TiledDesc(ctypes.Structure):
+    """Mirror of ``d2q9_tiled_desc``."""
+    _fields_ = [("rows", ctypes.c_int32), ("width", ctypes.c_int32),
+                ("steps", ctypes.c_int32), ("n_elems", ctypes.c_int32),
+                ("has_vel", ctypes.c_int32), ("has_pres", ctypes.c_int32),
+                ("cells", ctypes.c_void_p), ("codes", ctypes.c_void_p)]
+
+
+# boundary elements a launch of the tiled sweep holds (d2q9_tiled_desc)
+TILED_MAX_ELEMS = 32
+
+assert ctypes.sizeof(TiledDesc) == 40
 assert ctypes.sizeof(BcElem) == 40 and ctypes.sizeof(BcNode) == 20
 
 _P = ctypes.c_void_p
@@ -111,6 +123,9 @@ SIGNATURES = {
                                         ctypes.c_int32, _P, _P, _P, _P, _P,
                                         _P, ctypes.c_int, _P]),
     "d2q9_deep_rows": (ctypes.c_int, []),
+    "d2q9_tiled_steps": (ctypes.c_int, [_LP, ctypes.POINTER(TiledDesc), _P, _P,
+                                        _P, _P, ctypes.c_int32, ctypes.c_int,
+                                        ctypes.c_int, _P, ctypes.c_int64, _P]),
     "d2q9_moments": (ctypes.c_int, [_LP, _P, _P, _P]),
     "d2q9_reduce_work_len": (ctypes.c_int64, [_LP]),
     "d2q9_mass_fp64": (ctypes.c_int, [_LP, _P, _P, _P, _P]),

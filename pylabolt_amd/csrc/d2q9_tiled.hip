@@ -1,0 +1,78 @@
+// C-ABI entry of the tiled sweep (kernel in d2q9_tiled.h, one translation
+// unit per storage form).
+#include <hip/hip_runtime.h>
+
+#include "d2q9_reduce.h"
+#include "d2q9_tiled.h"
+
+using namespace d2q9;
+
+namespace {
+
+int tfail(int code, const char* what) {
+  set_error(what);
+  return code;
+}
+
+}  // namespace
+
+extern "C" int d2q9_tiled_steps(const d2q9_lattice* L, const d2q9_tiled_desc* D, void* f_a,
+                                void* f_b, void* mom_a, void* mom_b, int32_t n,
+                                int collide_first, int write_moments, void* mom_steps,
+                                int64_t mom_stride, void* stream) {
+  if (int r = validate_lattice(L)) return r;
+  if (!D || !f_a || !f_b || !mom_a || !mom_b)
+    return tfail(D2Q9_E_ARG, "tiled steps: null buffer");
+  if (f_a == f_b || mom_a == mom_b)
+    return tfail(D2Q9_E_ARG, "tiled steps: the two buffers must differ");
+  if (n < 0 || D->steps < 1 || (D->width != 16 && D->width != 32 && D->width != 64) ||
+      2 * (int64_t)D->steps >= D->width || 2 * (int64_t)D->steps >= D->rows)
+    return tfail(D2Q9_E_ARG, "tiled steps: bad region or step count");
+  if (D->n_elems < 0 || D->n_elems > tiled::MAX_ELEMS || (D->n_elems > 0 && !L->bc_elems) ||
+      !D->cells || !D->codes)
+    return tfail(D2Q9_E_ARG, "tiled steps: bad special-cell tables");
+  const size_t elem = L->storage == D2Q9_STORE_F64 ? 8 : 4;
+  const size_t raw = L->storage == D2Q9_STORE_F64 ? 8 : (L->storage == D2Q9_STORE_F32 ? 4 : 2);
+  if ((int64_t)D->rows * D->width > tiled::MAX_CELLS)
+    return tfail(D2Q9_E_TOO_LARGE, "tiled steps: the region does not fit a workgroup");
+  // cells are addressed by 32-bit byte offsets
+  if ((uint64_t)L->pop_len * raw > 0xffffffffull || L->plane > 0x7fffffffll)
+    return tfail(D2Q9_E_TOO_LARGE, "tiled steps: lattice over 4 GiB");
+  if (n == 0) return 0;
+  // launches of nearly equal length: the work on grown cells rises with the
+  // steps of a launch
+  const int launches = (n + D->steps - 1) / D->steps;
+  const int base = n / launches, longer = n % launches;
+  void* f[2] = {f_a, f_b};
+  void* m[2] = {mom_a, mom_b};
+  char* const per_step = static_cast<char*>(mom_steps);
+  const int64_t step_bytes = mom_stride * (int64_t)elem;
+  tiled::Launch A;
+  A.stream = static_cast<hipStream_t>(stream);
+  A.msrc = mom_a;
+  A.mom_stride = mom_stride;
+  int done = 0;
+  for (int a = 0; a < launches; ++a) {
+    A.K = base + (a < longer ? 1 : 0);
+    A.collide_first = a == 0 && collide_first;
+    A.write_mom = a == launches - 1 && write_moments;
+    A.fsrc = f[a & 1];
+    A.fdst = f[1 - (a & 1)];
+    A.mdst = m[1 - (a & 1)];
+    A.mom_steps = per_step ? per_step + done * step_bytes : nullptr;
+    hipError_t e = hipErrorInvalidValue;
+    switch (L->storage) {
+      case D2Q9_STORE_F64: e = tiled::launch<D2Q9_STORE_F64>(L, D, A); break;
+      case D2Q9_STORE_F32: e = tiled::launch<D2Q9_STORE_F32>(L, D, A); break;
+      case D2Q9_STORE_F16DEV: e = tiled::launch<D2Q9_STORE_F16DEV>(L, D, A); break;
+      case D2Q9_STORE_BF16DEV: e = tiled::launch<D2Q9_STORE_BF16DEV>(L, D, A); break;
+    }
+    if (e != hipSuccess) {
+      set_error(hipGetErrorString(e));
+      return (int)e;
+    }
+    done += A.K;
+    A.msrc = per_step ? per_step + (done - 1) * step_bytes : A.mdst;
+  }
+  return 0;
+}

@@ -28,6 +28,7 @@ the stream-only sweep when ``pop_new[n]`` is wanted.  The values are the
 reference's either way.
 """
 import ctypes
+import functools
 import math
 import warnings
 from types import SimpleNamespace
@@ -50,6 +51,7 @@ _TORCH_DTYPES = {
 # D2Q9 directions (reference base/lattice.py:50-59)
 CX = np.array([0, 1, 0, -1, 0, 1, -1, -1, 1])
 CY = np.array([0, 0, 1, 0, -1, 1, 1, -1, -1])
+INV = np.array([0, 3, 4, 1, 2, 7, 8, 5, 6])
 _KIND = {"bounce_back": nt.RULE_BB, "fixed_velocity": nt.RULE_VEL,
          "fixed_pressure": nt.RULE_PRES, "zero_gradient": nt.RULE_ZG}
 
@@ -326,6 +328,77 @@ class CaseTables:
             self.n_fix = int(self.fix_cells.size)
         return self.tile_class
 
+    def special_codes(self):
+        """Tables of the tiled sweep (d2q9_tiled_steps): for every fluid
+        cell with a solid neighbour or a boundary rule, where the value
+        streamed into each direction comes from.
+
+        Returns (cells [nx+2, ny+2] uint32, codes [n, 4] uint32, has_vel,
+        has_pres), or None when the tables cannot express the case: more
+        boundary elements than the kernel holds, a zero-gradient node beside
+        a cell that is not fluid, or a cell with moving-wall and
+        fixed-pressure directions of more than two elements.  The order is
+        that of the general path: a solid pull neighbour (by its own index,
+        not its periodic image) gives the cell's own opposite population,
+        and a boundary rule replaces the direction after that.  Valid for
+        solids at rest."""
+        if len(self.elems) > nt.TILED_MAX_ELEMS:
+            return None
+        solid = (self.flags_pad & nt.CELL_SOLID) != 0
+        fluid = self.fluid_pad
+        special = fluid & ((self.flags_pad & (nt.CELL_NEAR_SOLID |
+                                              nt.CELL_BC)) != 0)
+        ii, jj = np.nonzero(special)
+        n = ii.size
+        if n >= 1 << 24:
+            return None
+        cells = self.flags_pad.astype(np.uint32)
+        cells[ii, jj] |= np.arange(n, dtype=np.uint32) << np.uint32(8)
+        codes = np.zeros((max(1, n), 4), dtype=np.uint32)
+
+        def source(dr, dc, k):
+            return (dr + 1) | (dc + 1) << 2 | k << 4
+
+        bc = (self.flags_pad[ii, jj] & nt.CELL_BC) != 0
+        node = self.bc_slot_pad[ii, jj]
+        normal = np.array([[int(v) for v in e["normal"]]
+                           for _, e in self.elems] or [[0, 0]])
+        has_vel = has_pres = False
+        first = np.full(n, -1)
+        second = np.full(n, -1)
+        arith = np.zeros(n, dtype=np.int64)
+        for d in range(1, 9):
+            back = source(0, 0, int(INV[d]))
+            code = np.where(solid[ii - CX[d], jj - CY[d]], back,
+                            source(-CX[d], -CY[d], d))
+            rule = np.where(bc, self.bc_nodes[node, d].astype(np.int64), 0)
+            kind, elem = rule & 15, rule >> 4
+            moving = (kind == nt.RULE_VEL) | (kind == nt.RULE_PRES)
+            has_vel |= bool((kind == nt.RULE_VEL).any())
+            has_pres |= bool((kind == nt.RULE_PRES).any())
+            code = np.where((kind == nt.RULE_BB) | moving, back, code)
+            first = np.where(moving & (first < 0), elem, first)
+            other = moving & (elem != first)
+            if np.any(other & (second >= 0) & (second != elem)):
+                return None
+            second = np.where(other, elem, second)
+            arith |= moving.astype(np.int64) << (d - 1)
+            arith |= other.astype(np.int64) << (d + 7)
+            zg = np.nonzero(kind == nt.RULE_ZG)[0]
+            if zg.size:
+                n0, n1 = normal[elem[zg]].T
+                bi, bj = ii[zg] + n0, jj[zg] + n1
+                if not fluid[bi, bj].all():
+                    return None
+                # the neighbour is interior, so its own are in range
+                code[zg] = np.where(solid[bi - CX[d], bj - CY[d]],
+                                    source(n0, n1, int(INV[d])),
+                                    source(n0 - CX[d], n1 - CY[d], d))
+            codes[:n, (d - 1) >> 2] |= code.astype(np.uint32) << np.uint32(
+                8 * ((d - 1) & 3))
+        arith |= np.maximum(first, 0) << 16 | np.maximum(second, 0) << 24
+        codes[:n, 2] = np.where(first >= 0, arith, 0)
+        return cells, codes, has_vel, has_pres
 
     def deep_split(self, rows):
         """Deep tiles of the two-step sweep (d2q9_fused_step2) and the rim
@@ -505,6 +578,48 @@ class CaseTables:
             n_fix_b=nfb)
 
 
+# Cost model of a launch of the tiled sweep, microseconds on an MI355X, per
+# compute width and forcing: a wave's loads, a wave's step; a launch and its
+# loads take 4 us, a step's latency half a microsecond.  FP64 without a force
+# runs two workgroups of 768 threads per CU, so larger regions lose
+# (2048x1024: 27.7 us per step with 24 x 32 cells, 38.9 with 32 x 32).
+_TILED_LAUNCH, _TILED_LATENCY = 4.0, 0.5
+_TILED_COST = {(8, False): (0.13, 0.11, 768), (8, True): (0.13, 0.16, 1024),
+               (4, False): (0.05, 0.06, 1024), (4, True): (0.05, 0.07, 1024)}
+_TILED_CUS = 256
+
+
+@functools.lru_cache(maxsize=256)
+def tiled_shape(nx, ny, double, forced):
+    """(rows, width, steps) of the tiled sweep's region for a lattice.
+
+    More steps per launch share its latency but grow the work on cells that
+    several tiles compute; smaller regions spread a small lattice over more
+    CUs.  The choice minimises a cost model (launch + steps + the waves of
+    the busiest CU) over the regions of up to 1024 cells.  Against a sweep
+    of regions and steps on nine lattices from 128 x 128 to 4096 x 1024 it
+    picks the fastest region or one within 5 % of it, 14 % on one."""
+    load, step, most = _TILED_COST[8 if double else 4, bool(forced)]
+    best = None
+    for width in (16, 32, 64):
+        for steps in (4, 6, 8):
+            cols = width - 2 * steps
+            if cols <= 0:
+                continue
+            for rows in range(2 * steps + 2, most // width + 1, 2):
+                tiles = -(-nx // (rows - 2 * steps)) * -(-ny // cols)
+                # a last round that is partly empty matters for few rounds
+                per_cu = (-(-tiles // _TILED_CUS) if tiles <= 4 * _TILED_CUS
+                          else tiles / _TILED_CUS + 0.5)
+                active = sum(rows - 2 * s for s in range(1, steps + 1)) \
+                    * width / 64.0
+                cost = (_TILED_LAUNCH + _TILED_LATENCY * steps + per_cu *
+                        (load * -(-rows * width // 64) + step * active)) / steps
+                if best is None or cost < best[0]:
+                    best = (cost, rows, width, steps)
+    return best[1:]
+
+
 def force_tables(nx, ny, groups):
     """Device-ready node and group records for d2q9_momentum_exchange.
 
@@ -565,9 +680,13 @@ class D2Q9Engine:
     ``two_step`` advances pairs of steps with one sweep over the deep
     interior (d2q9_fused_step2) when deep tiles fit; by default for FP64
     and FP32 storage when the two population buffers exceed
-    ``TWO_STEP_MIN_BYTES`` (the results are bitwise those of single
-    steps), for 16-bit storage only when asked (its intermediate step stays
-    in FP32, which changes the rounding).
+    ``TWO_STEP_MIN_BYTES`` and it is the faster sweep (``_two_step_wins``;
+    the results are bitwise those of single steps), for 16-bit storage only
+    when asked (its intermediate step stays in FP32, which changes the
+    rounding).  Otherwise steps go through the tiled sweep
+    (d2q9_tiled_steps, several steps per launch, bitwise single steps in
+    every storage form), or single sweeps where the case cannot be
+    expressed in its tables or a solid moves.
     """
 
     def __init__(self, nx, ny, solid_pad, density, velocity, elements,
@@ -691,9 +810,12 @@ class D2Q9Engine:
         self._upload_tiles()
         self.graph_steps = max(2, int(graph_steps) // 2 * 2)
         self._graphs = {}
-        # pairs of steps with one sweep over the deep interior, by default
-        # for lattices whose two population buffers exceed
-        # TWO_STEP_MIN_BYTES
+        # several steps per launch: the tiled sweep's tables, where the case
+        # can be expressed in them
+        self._codes = (self.tables.special_codes()
+                       if min(self.nx, self.ny) >= 2 and
+                       self.f[0].numel() * self.f[0].element_size() < 1 << 32
+                       else None)
         if two_step is None:
             # FP64 and FP32 give the same bits either way; in 16-bit
             # storage the two-step sweep keeps the intermediate step in FP32
@@ -701,13 +823,14 @@ class D2Q9Engine:
             # may do
             two_step = (self.storage in (nt.STORE_F64, nt.STORE_F32) and
                         2 * self.f[0].numel() * self.f[0].element_size()
-                        > TWO_STEP_MIN_BYTES)
+                        > TWO_STEP_MIN_BYTES and self._two_step_wins())
         self._two_step_req = bool(two_step)
         self.two_step = False
         self._setup_two_step()
-        self.time_step = 0
         self._init_density = np.asarray(density, dtype=np.float64)
         self._init_velocity = np.asarray(velocity, dtype=np.float64)
+        self._setup_tiled()
+        self.time_step = 0
         self.initialize()
 
     def _upload_tiles(self):
@@ -796,6 +919,74 @@ class D2Q9Engine:
         # return to their roles
         self.graph_steps = max(4, self.graph_steps // 4 * 4)
 
+    def _two_step_wins(self):
+        """Whether the two-step sweep is the faster one for a lattice of
+        more than TWO_STEP_MIN_BYTES.
+
+        It is where it has no rim (a channel periodic in x with straight
+        walls at y, whole blocks and tile heights: us per step against the
+        tiled sweep's, FP32 2048x1024 16.3 / 18.2, FP64 1024x1024 19.6 /
+        23.8, 4096x1024 67 / 80) and for forced FP64 at large sizes, whose
+        tiled kernel is short of registers.  Elsewhere the rim's kernels and
+        its fork and join cost more than the tiled sweep's repeated cells:
+        FP64 cylinder 1001x413 7.4 us tiled, 25 two-step, 8192x2048 220 /
+        235; FP32 cylinder 2999x1111 22.6 / 34, 8192x2048 112 / 122."""
+        if self._codes is None:
+            return True
+        if (self.storage == nt.STORE_F64 and self.forcing is not None and
+                self.nx * self.ny > 1 << 20):
+            return True
+        t = self.tables
+        plain = not (t.flags_pad & nt.CELL_NEAR_SOLID).any()
+        return bool(plain and t.x_periodic and not t.y_periodic and
+                    self.nx % self.tile_i == 0 and self.ny % self.B == 0 and
+                    t.wall_inline_wrap[:, [0, -1]].all())
+
+    def _setup_tiled(self):
+        """Tables of the tiled sweep on the device, where the lattice takes
+        it."""
+        self.tiled = None
+        self._tiled_arrays = None
+        t, tables = self.tables, self._codes
+        self._codes = None
+        if self.two_step or tables is None:
+            return
+        cells, codes, has_vel, has_pres = tables
+        rows, width, steps = tiled_shape(
+            self.nx, self.ny, self.storage == nt.STORE_F64,
+            self.forcing is not None)
+        with torch.cuda.stream(self.stream):
+            dev = {"cells": self._upload_plane(cells, torch.int32),
+                   "codes": torch.from_numpy(codes.view(np.int32)).to(
+                       self.device)}
+        D = nt.TiledDesc()
+        D.rows, D.width, D.steps = rows, width, steps
+        D.n_elems = len(t.elems)
+        D.has_vel, D.has_pres = int(has_vel), int(has_pres)
+        D.cells, D.codes = dev["cells"].data_ptr(), dev["codes"].data_ptr()
+        self._tiled_arrays = dev
+        self._tiled_solid = np.flatnonzero(
+            (t.flags_pad & nt.CELL_SOLID).ravel())
+        self.tiled = D
+        self._tiled_p = ctypes.byref(D)
+
+    def _advance_tiled(self, n, write_moments):
+        """``n`` steps through the tiled sweep; the first one collides
+        ``pop_new`` where that is in memory."""
+        first = self.i_pop_new is not None
+        a = self.i_pop_new if first else self.i_pop
+        m = self.i_mom
+        nt.check(self.lib.d2q9_tiled_steps(
+            self._Lp, self._tiled_p, nt.ptr(self.f[a]), nt.ptr(self.f[1 - a]),
+            nt.ptr(self.mom[m]), nt.ptr(self.mom[1 - m]), n, int(first),
+            int(write_moments), None, 0, self._stream_ptr),
+            "d2q9_tiled_steps")
+        flip = -(-n // self.tiled.steps) & 1
+        self.i_pop, self.i_mom = a ^ flip, m ^ flip
+        self.i_pop_new = None
+        self.mom_full = bool(write_moments)
+        self.time_step += n
+
     def set_tile_rows(self, tile_i):
         """Re-tile with ``tile_i`` rows per tile (workgroup 64 x tile_i);
         drops captured graphs, which hold the old tile tables."""
@@ -842,6 +1033,10 @@ class D2Q9Engine:
     # ---- lifecycle ------------------------------------------------------
     def initialize(self):
         """pop = pop_new = feq(rho0, u0) (equilibrium_kernels.py:38-78)."""
+        if self.tiled is not None and np.any(
+                self._init_velocity.reshape(-1, 2)[self._tiled_solid]):
+            # the tiled sweep is for solids at rest
+            self.tiled = None
         with torch.cuda.stream(self.stream):
             m = self._mom_from_host(self._init_density, self._init_velocity)
             self.mom[0].copy_(m)
@@ -912,6 +1107,9 @@ class D2Q9Engine:
 
     def step(self, write_moments=False):
         """Advance one reference time step."""
+        if self.tiled is not None:
+            self._advance_tiled(1, write_moments)
+            return
         if self.i_pop_new is not None:
             # pop_new is in memory: moments + collision only
             src = self.i_pop_new
@@ -932,6 +1130,9 @@ class D2Q9Engine:
         steps replay a captured HIP graph."""
         n = int(n)
         if n <= 0:
+            return
+        if self.tiled is not None:
+            self._advance_tiled(n, write_moments)
             return
         if self.i_pop_new is not None:
             self.step(write_moments and n == 1)
@@ -968,7 +1169,7 @@ class D2Q9Engine:
         """Capture (once) the graph that ``advance`` replays from the
         current buffer roles, without running it; a timed region that
         follows then replays graphs only."""
-        if self.i_pop_new is None:
+        if self.i_pop_new is None and self.tiled is None:
             full = self.mom_full
             self._graph_for_state()
             self.mom_full = full

@@ -430,6 +430,18 @@ int d2q9_adjoint_step(const d2q9_lattice* L, int streamed, const void* lam_src,
                       void* lam_dst, const void* mom, const void* seed_u,
                       void* grad_force, void* stream);
 
+/*
+ * n reverse steps in one launch (1 <= n <= D->steps), as n calls of
+ * d2q9_adjoint_step: the first reads this step's rho/u at mom, the next at
+ * mom - mom_stride elements, and so on back in time; seed_u (nullable) is the
+ * first one's.  last_streamed: the last of them is streamed (it is not when it
+ * is the first time step).  The region, the special cells' records and their
+ * conditions are those of d2q9_tiled_steps.
+ */
+int d2q9_adjoint_steps(const d2q9_lattice* L, const d2q9_tiled_desc* D, int32_t n,
+                       int last_streamed, const void* lam_src, void* lam_dst, const void* mom,
+                       int64_t mom_stride, const void* seed_u, void* grad_force, void* stream);
+
 /* dL/d(rho0, u0) [3][plane] from mu = dL/d(initial equilibrium populations)
  * and mom0 = the initial rho/u. */
 int d2q9_adjoint_init_grad(const d2q9_lattice* L, const void* mu,

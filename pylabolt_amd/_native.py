@@ -142,6 +142,9 @@ SIGNATURES = {
                                        ctypes.c_int]),
     "d2q9_adjoint_step": (ctypes.c_int, [_LP, ctypes.c_int, _P, _P, _P, _P,
                                          _P, _P]),
+    "d2q9_adjoint_steps": (ctypes.c_int, [_LP, ctypes.POINTER(TiledDesc),
+                                          ctypes.c_int32, ctypes.c_int, _P, _P,
+                                          _P, ctypes.c_int64, _P, _P, _P]),
     "d2q9_adjoint_init_grad": (ctypes.c_int, [_LP, _P, _P, _P, _P]),
     "d2q9_batched_step": (ctypes.c_int, [_P, _P, _P, _P] + [ctypes.c_int] * 9
                           + [_P]),

@@ -81,7 +81,8 @@ class FlowRollout:
             st.boundary.y_periodic, "BGK", co.forcing_fluid, co.omega_fluid,
             (0.0, 0.0), lat.inv_cs_2, lat.inv_cs_4, lat.weights,
             st.control.float_min, storage="f64",
-            force_field=np.zeros((size, 2)), device=device)
+            force_field=np.zeros((size, 2)), device=device,
+            two_step=False)
         self._check_permutation()
         eng = self.eng
         dev = eng.device
@@ -94,7 +95,9 @@ class FlowRollout:
             nck = self.nseg if self.mode == "sqrt" else 1
             self.ck = [torch.zeros(L, **z) for _ in range(nck)]
             self.work = [torch.zeros(L, **z) for _ in range(2)]
-            self.ring = [torch.zeros(3 * P, **z) for _ in range(self.K)]
+            # rho/u of the steps of a segment, one after another
+            moments = torch.zeros(self.K, 3 * P, **z)
+            self.ring = list(moments)
             self.mscratch = [torch.zeros(3 * P, **z) for _ in range(2)]
             self.mom0 = torch.zeros(3 * P, **z)
             self.lam = [torch.zeros(L, **z) for _ in range(2)]
@@ -170,28 +173,51 @@ class FlowRollout:
         if rc:
             raise nt.NativeError(e.lib.d2q9_last_error().decode())
 
-    def _forward_ops(self):
-        """The forward pass as a list of sweeps (captured in one graph)."""
-        N, K = self.steps, self.K
+    def _sweeps(self, src, dst, msrc, mdst, first, steps, every):
+        """``steps`` steps from ``src`` into ``dst`` in one launch (one step
+        where the engine has no tiled sweep).  ``every``: rho/u after each
+        step go to consecutive ring slots from ``mdst`` on; otherwise only
+        the last step's, to ``mdst`` (None: nowhere that matters)."""
         e = self.eng
+        if e.tiled is None:
+            self._sweep(src, dst, msrc, mdst if mdst is not None else
+                        self.mscratch[1], first, mdst is not None)
+            return
+        nt.check(e.lib.d2q9_tiled_steps(
+            e._Lp, e._tiled_p, nt.ptr(src), nt.ptr(dst), nt.ptr(msrc),
+            nt.ptr(self.mscratch[1] if mdst is None or every else mdst),
+            steps, int(first), int(mdst is not None),
+            nt.ptr(mdst) if every else None, 3 * e.plane, e._stream_ptr),
+            "d2q9_tiled_steps")
+
+    def _per_launch(self, n):
+        """``n`` steps cut into launches of nearly equal length."""
+        most = self.eng.tiled.steps if self.eng.tiled is not None else 1
+        k = -(-n // most)
+        return [n // k + (1 if q < n % k else 0) for q in range(k)]
+
+    def _forward_ops(self):
+        """The forward pass as a list of sweeps (captured in one graph):
+        (src, dst, msrc, mdst, first, steps, every) as for ``_sweeps``.
+        The supported rules read no moments of the step before, so every
+        launch may name the same msrc."""
+        N, K = self.steps, self.K
         ops = []
         # g_0 = feq(rho0, u0) lives in ck[0]; work[1] also receives it
-        prev = self.ck[0]
-        for n in range(1, N + 1):
-            ckpt = self.mode == "sqrt" and n % K == 0 and n // K < self.nseg
-            dst = self.ck[n // K] if ckpt else self.work[n % 2]
-            if dst is prev:
-                dst = self.work[(n + 1) % 2]
-            if self.mode == "moments":
-                msrc = self.ring[n - 2] if n >= 2 else self.mscratch[0]
-                mdst = self.ring[n - 1]
-            else:
-                msrc = self.mscratch[(n - 1) % 2]
-                mdst = self.mscratch[n % 2]
-            ops.append((prev, dst, msrc, mdst, n == 1, n == N or
-                        self.mode == "moments"))
-            prev = dst
-        self._last_moments = ops[-1][3]
+        prev, n = self.ck[0], 0
+        every = self.mode == "moments"
+        while n < N:
+            seg = min(K, N - n)
+            for q, m in enumerate(self._per_launch(seg)):
+                end = n + m
+                ckpt = not every and end % K == 0 and end // K < self.nseg
+                dst = (self.ck[end // K] if ckpt else
+                       self.work[1] if prev is self.work[0] else self.work[0])
+                mdst = (self.ring[n] if every else
+                        self.mscratch[0] if end == N else None)
+                ops.append((prev, dst, self.mom0, mdst, n == 0, m, every))
+                prev, n = dst, end
+        self._last_moments = self.ring[N - 1] if every else self.mscratch[0]
         return ops
 
     def _capture(self, issue):
@@ -215,7 +241,7 @@ class FlowRollout:
                                     nt.ptr(self.work[1]), nt.ptr(self.mom0),
                                     e._stream_ptr), "d2q9_init_eq")
         for op in self._forward_ops():
-            self._sweep(*op)
+            self._sweeps(*op)
 
     def _issue_backward(self):
         e = self.eng
@@ -232,22 +258,31 @@ class FlowRollout:
                     prev = self.work[0]
                 else:
                     prev = self.ck[s]
-                for n in range(n0, n1 + 1):
+                n = n0
+                for m in self._per_launch(n1 - n0 + 1):
                     dst = self.work[1] if prev is self.work[0] else self.work[0]
-                    slot = n - n0
-                    msrc = self.ring[slot - 1] if slot else self.mscratch[0]
-                    self._sweep(prev, dst, msrc, self.ring[slot], n == 1, True)
-                    prev = dst
-            for n in range(n1, n0 - 1, -1):
+                    self._sweeps(prev, dst, self.mom0, self.ring[n - n0],
+                                 n == 1, m, True)
+                    prev, n = dst, n + m
+            n = n1
+            for m in self._per_launch(n1 - n0 + 1):
                 slot = (n - n0) if self.mode == "sqrt" else n - 1
                 seed = self.seed if n == N else None
-                rc = e.lib.d2q9_adjoint_step(
-                    e._Lp, int(n >= 2), nt.ptr(lam_cur), nt.ptr(lam_nxt),
-                    nt.ptr(self.ring[slot]), nt.ptr(seed),
-                    nt.ptr(self.grad_f), e._stream_ptr)
+                if e.tiled is None:
+                    rc = e.lib.d2q9_adjoint_step(
+                        e._Lp, int(n >= 2), nt.ptr(lam_cur), nt.ptr(lam_nxt),
+                        nt.ptr(self.ring[slot]), nt.ptr(seed),
+                        nt.ptr(self.grad_f), e._stream_ptr)
+                else:
+                    rc = e.lib.d2q9_adjoint_steps(
+                        e._Lp, e._tiled_p, m, int(n - m >= 1),
+                        nt.ptr(lam_cur), nt.ptr(lam_nxt),
+                        nt.ptr(self.ring[slot]), 3 * e.plane, nt.ptr(seed),
+                        nt.ptr(self.grad_f), e._stream_ptr)
                 if rc:
                     raise nt.NativeError(e.lib.d2q9_last_error().decode())
                 lam_cur, lam_nxt = lam_nxt, lam_cur
+                n -= m
         nt.check(e.lib.d2q9_adjoint_init_grad(
             e._Lp, nt.ptr(lam_cur), nt.ptr(self.mom0), nt.ptr(self.grad_init),
             e._stream_ptr), "d2q9_adjoint_init_grad")

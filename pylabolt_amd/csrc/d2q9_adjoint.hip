@@ -25,7 +25,7 @@
 
 #include <string>
 
-#include "d2q9_device.h"
+#include "d2q9_tiled.h"
 
 using namespace d2q9;
 
@@ -37,6 +37,65 @@ int afail(int code, const char* what) {
 }
 
 constexpr int B64 = 64;
+
+// The collision's transpose at one cell, in place: lam' -> mu, and this step's
+// contribution to dL/dF.  The sums over k reduce to the weighted moments of
+// lam' up to second order (w_k lam'_k against 1, c, cc), since feq and Fbar
+// are quadratic in c: about 110 FP64 operations against 390 direction by
+// direction.
+struct AdjointConsts {
+  double om, a, i4, fmin, w0, w1, w5;
+};
+
+__device__ __forceinline__ AdjointConsts adjoint_consts(const d2q9_lattice& L) {
+  return {L.omega, L.inv_cs_2, L.inv_cs_4, L.float_min, L.w[0], L.w[1], L.w[5]};
+}
+
+template <int FORCING>
+__device__ __forceinline__ void collide_transpose(const AdjointConsts& K, double (&g)[9],
+                                                  double rho, double ux, double uy, double fx,
+                                                  double fy, double seed_x, double seed_y,
+                                                  double& gfx, double& gfy) {
+  const double om = K.om, a = K.a, i4 = K.i4;
+  const double inv = 1.0 / (rho + K.fmin);
+  const double s13 = g[1] + g[3], s24 = g[2] + g[4], d13 = g[1] - g[3], d24 = g[2] - g[4];
+  const double s57 = g[5] + g[7], s68 = g[6] + g[8], d57 = g[5] - g[7], d68 = g[6] - g[8];
+  const double diag = K.w5 * (s57 + s68);
+  const double mxx = K.w1 * s13 + diag, myy = K.w1 * s24 + diag, mxy = K.w5 * (s57 - s68);
+  const double m0 = K.w0 * g[0] + (K.w1 * (s13 + s24) + diag);
+  const double mx = K.w1 * d13 + K.w5 * (d57 - d68), my = K.w1 * d24 + K.w5 * (d57 + d68);
+  // c . u against c, twice over: sum w lam (c . u) c
+  const double cux = ux * mxx + uy * mxy, cuy = ux * mxy + uy * myy;
+  const double a_rho =
+      om * (m0 * (1.0 - (0.5 * a) * (ux * ux + uy * uy)) + a * (ux * mx + uy * my) +
+            (0.5 * i4) * (ux * cux + uy * cuy));
+  const double omr = om * rho, cf = 1.0 - 0.5 * om;
+  double aux = omr * (a * (mx - ux * m0) + i4 * cux);
+  double auy = omr * (a * (my - uy * m0) + i4 * cuy);
+  gfx = gfy = 0.0;
+  if constexpr (FORCING == D2Q9_GUO_LINEAR) {
+    gfx = cf * (a * mx);
+    gfy = cf * (a * my);
+  } else if constexpr (FORCING == D2Q9_GUO_SECOND_ORDER) {
+    aux += cf * (i4 * (fx * mxx + fy * mxy) - a * (fx * m0));
+    auy += cf * (i4 * (fx * mxy + fy * myy) - a * (fy * m0));
+    gfx = cf * (a * (mx - ux * m0) + i4 * cux);
+    gfy = cf * (a * (my - uy * m0) + i4 * cuy);
+  }
+  aux += seed_x;
+  auy += seed_y;
+  const double ax = inv * aux, ay = inv * auy;
+  gfx += 0.5 * ax;
+  gfy += 0.5 * ay;
+  const double base = a_rho - (ux * ax + uy * ay);
+#pragma unroll
+  for (int k = 0; k < 9; ++k) {
+    double v = base;
+    if (CX[k] != 0) v = CX[k] > 0 ? v + ax : v - ax;
+    if (CY[k] != 0) v = CY[k] > 0 ? v + ay : v - ay;
+    g[k] = (1.0 - om) * g[k] + v;
+  }
+}
 
 template <int FORCING, bool SCATTER>
 __global__ __launch_bounds__(256) void k_adjoint(
@@ -51,53 +110,16 @@ __global__ __launch_bounds__(256) void k_adjoint(
   const uint8_t fl = L.flags[c];
   if (!(fl & D2Q9_CELL_FLUID)) return;
   const int64_t P = L.plane;
-  const double om = L.omega, a = L.inv_cs_2, i4 = L.inv_cs_4;
-  const double b = 0.5 * i4, c0 = 0.5 * a;
   const double* F = static_cast<const double*>(L.force_field);
-  const double fx = F[c], fy = F[P + c];
-  const double rho = mom[c], ux = mom[P + c], uy = mom[2 * P + c];
-  const double inv = 1.0 / (rho + L.float_min);
-  const double u2 = ux * ux + uy * uy;
-  double lam[9];
-#pragma unroll
-  for (int k = 0; k < 9; ++k) lam[k] = lam_src[pop_index<B64>(L, i, j, k)];
-  double a_rho = 0.0, aux = 0.0, auy = 0.0, gfx = 0.0, gfy = 0.0;
-#pragma unroll
-  for (int k = 0; k < 9; ++k) {
-    const double cx = CX[k], cy = CY[k], w = L.w[k];
-    const double cu = cx * ux + cy * uy;
-    // d feq / d rho at fixed u, d feq / d u
-    const double dfr = w * (1.0 + a * cu + b * cu * cu - c0 * u2);
-    const double dfu_x = w * rho * (a * cx + 2.0 * b * cu * cx - 2.0 * c0 * ux);
-    const double dfu_y = w * rho * (a * cy + 2.0 * b * cu * cy - 2.0 * c0 * uy);
-    a_rho += lam[k] * om * dfr;
-    aux += lam[k] * om * dfu_x;
-    auy += lam[k] * om * dfu_y;
-    if constexpr (FORCING == D2Q9_GUO_LINEAR) {
-      const double h = (1.0 - 0.5 * om) * lam[k] * w * a;
-      gfx += h * cx;
-      gfy += h * cy;
-    } else if constexpr (FORCING == D2Q9_GUO_SECOND_ORDER) {
-      const double h = (1.0 - 0.5 * om) * lam[k] * w;
-      const double cf = cx * fx + cy * fy;
-      // dFbar/du = w (-a F + i4 (c.F) c)
-      aux += h * (-a * fx + i4 * cf * cx);
-      auy += h * (-a * fy + i4 * cf * cy);
-      // dFbar/dF = w (a (c - u) + i4 (c.u) c)
-      gfx += h * (a * (cx - ux) + i4 * cu * cx);
-      gfy += h * (a * (cy - uy) + i4 * cu * cy);
-    }
-  }
-  if (seed_u) {
-    aux += seed_u[c];
-    auy += seed_u[P + c];
-  }
-  grad_f[c] += gfx + 0.5 * inv * aux;
-  grad_f[P + c] += gfy + 0.5 * inv * auy;
   double mu[9];
 #pragma unroll
-  for (int k = 0; k < 9; ++k)
-    mu[k] = (1.0 - om) * lam[k] + a_rho + inv * ((CX[k] - ux) * aux + (CY[k] - uy) * auy);
+  for (int k = 0; k < 9; ++k) mu[k] = lam_src[pop_index<B64>(L, i, j, k)];
+  double gfx, gfy;
+  collide_transpose<FORCING>(adjoint_consts(L), mu, mom[c], mom[P + c], mom[2 * P + c], F[c],
+                             F[P + c], seed_u ? seed_u[c] : 0.0, seed_u ? seed_u[P + c] : 0.0,
+                             gfx, gfy);
+  grad_f[c] += gfx;
+  grad_f[P + c] += gfy;
   if constexpr (!SCATTER) {
 #pragma unroll
     for (int k = 0; k < 9; ++k) lam_dst[pop_index<B64>(L, i, j, k)] = mu[k];
@@ -131,6 +153,121 @@ __global__ __launch_bounds__(256) void k_adjoint(
       if (xn < 1 || xn > L.nx || yn < 1 || yn > L.ny) continue;  // from a ghost: no dependence
       lam_dst[pop_index<B64>(L, xn, yn, d)] = mu[d];
     }
+  }
+}
+
+// K reverse steps of an output tile per launch, as the tiled forward sweep
+// (d2q9_tiled.h: the same regions, special-cell records and LDS layout).  A
+// reverse step is local up to its streaming: mu goes to LDS and the transpose
+// of the pull gathers it back, lam_d(x) = mu_d(x + c_d), or the cell's own
+// mu_{inv d} where the population p_d bounces back to it -- the directions
+// whose record names the cell itself.  rho/u of a region cell are loaded a
+// step ahead.  grad_f is read and written once per launch.
+template <int FORCING, int W>
+__global__ __launch_bounds__(tiled::MAX_CELLS) void k_adjoint_tiled(
+    const d2q9_lattice L, const d2q9_tiled_desc D, int ntiles, int ntj, int K, int rows,
+    int last_streamed, const double* __restrict__ lam_src, double* __restrict__ lam_dst,
+    const double* __restrict__ mom, int64_t mom_stride, const double* __restrict__ seed_u,
+    double* __restrict__ grad_f) {
+  extern __shared__ __align__(16) char smem[];
+  double* const s = reinterpret_cast<double*>(smem);
+  const int tile = xcd_remap((int)blockIdx.x, ntiles);
+  const int e = (int)threadIdx.x, r = e / W, c = e % W;
+  const int i0 = 1 + (tile / ntj) * (rows - 2 * K) - K;
+  const int j0 = 1 + (tile % ntj) * (W - 2 * K) - K;
+  int i = i0 + r, j = j0 + c;
+  bool own = i <= L.nx && j <= L.ny;
+  if (L.x_periodic) {
+    while (i < 1) i += L.nx;
+    while (i > L.nx) i -= L.nx;
+  }
+  if (L.y_periodic) {
+    while (j < 1) j += L.ny;
+    while (j > L.ny) j -= L.ny;
+  }
+  const AdjointConsts Kc = adjoint_consts(L);
+  int depth = -1;           // the last reverse step the cell collides in
+  uint32_t pop = 0, bounce = 0;
+  int32_t cell = 0;
+  double g[9], fx = 0.0, fy = 0.0, gx = 0.0, gy = 0.0, sx = 0.0, sy = 0.0;
+  double rho = 1.0, ux = 0.0, uy = 0.0;
+#pragma unroll
+  for (int k = 0; k < 9; ++k) g[k] = 0.0;
+  if (r < rows && i >= 1 && i <= L.nx && j >= 1 && j <= L.ny) {
+    const unsigned jj = (unsigned)(j + B64 - 1);
+    pop = ((unsigned)i * (unsigned)L.nbj + jj / B64) * (9u * B64) + jj % B64;
+    cell = L.origin + i * L.pitch + j;
+    const uint32_t info = D.cells[cell];
+    if (info & D2Q9_CELL_FLUID) {
+      depth = min(min(r, rows - 1 - r), min(c, W - 1 - c));
+      const double* F = static_cast<const double*>(L.force_field);
+#pragma unroll
+      for (int k = 0; k < 9; ++k) g[k] = lam_src[pop + (unsigned)(k * B64)];
+      fx = F[cell];
+      fy = F[L.plane + cell];
+      rho = mom[cell];
+      ux = mom[L.plane + cell];
+      uy = mom[2 * L.plane + cell];
+      if (seed_u) {
+        sx = seed_u[cell];
+        sy = seed_u[L.plane + cell];
+      }
+      if (info & (D2Q9_CELL_NEAR_SOLID | D2Q9_CELL_BC)) {
+        const uint4 v = reinterpret_cast<const uint4*>(D.codes)[info >> 8];
+#pragma unroll
+        for (int d = 1; d < 9; ++d) {
+          const uint32_t w = ((d < 5 ? v.x : v.y) >> (8 * ((d - 1) & 3))) & 0xffu;
+          if ((w & 0xfu) == 5u) bounce |= 1u << INV[d];  // from the cell itself
+        }
+      }
+    }
+  }
+  own = own && depth >= K;
+  if (own) {
+    gx = grad_f[cell];
+    gy = grad_f[L.plane + cell];
+  }
+#pragma unroll 1
+  for (int st = 0; st < K; ++st) {
+    // a step ahead: rho/u of the step before (in time)
+    double rho1 = 1.0, ux1 = 0.0, uy1 = 0.0;
+    if (st + 1 < K && depth > st) {
+      const double* const m = mom - (int64_t)(st + 1) * mom_stride + cell;
+      rho1 = m[0];
+      ux1 = m[L.plane];
+      uy1 = m[2 * L.plane];
+    }
+    if (depth >= st) {
+      double gfx, gfy;
+      collide_transpose<FORCING>(Kc, g, rho, ux, uy, fx, fy, sx, sy, gfx, gfy);
+      gx += gfx;
+      gy += gfy;
+    }
+    sx = sy = 0.0;
+    if (st + 1 < K || last_streamed) {
+      if (r < rows) {
+#pragma unroll
+        for (int k = 0; k < 9; ++k) s[e * 9 + k] = g[k];
+      }
+      __syncthreads();
+      if (depth > st) {
+        const double* const p = s + (e - W - 1) * 9;
+#pragma unroll
+        for (int d = 1; d < 9; ++d)
+          g[d] = (bounce >> d) & 1u ? s[e * 9 + INV[d]]
+                                    : p[((1 + CX[d]) * W + 1 + CY[d]) * 9 + d];
+      }
+      __syncthreads();
+    }
+    rho = rho1;
+    ux = ux1;
+    uy = uy1;
+  }
+  if (own) {
+#pragma unroll
+    for (int k = 0; k < 9; ++k) lam_dst[pop + (unsigned)(k * B64)] = g[k];
+    grad_f[cell] = gx;
+    grad_f[L.plane + cell] = gy;
   }
 }
 
@@ -213,6 +350,59 @@ int d2q9_adjoint_step(const d2q9_lattice* L, int streamed, const void* lam_src,
   }
 #undef D2Q9_ADJ
   hipError_t e = hipGetLastError();
+  if (e != hipSuccess) {
+    set_error(hipGetErrorString(e));
+    return (int)e;
+  }
+  return 0;
+}
+
+int d2q9_adjoint_steps(const d2q9_lattice* L, const d2q9_tiled_desc* D, int32_t n,
+                       int last_streamed, const void* lam_src, void* lam_dst, const void* mom,
+                       int64_t mom_stride, const void* seed_u, void* grad_force, void* stream) {
+  if (int r = check(L)) return r;
+  if (int r = validate_lattice(L)) return r;
+  if (!D || !lam_src || !lam_dst || !mom || !grad_force || lam_src == lam_dst)
+    return afail(D2Q9_E_ARG, "adjoint steps: buffers null or aliased");
+  if (int r = tiled::check_desc(L, D)) return r;
+  if (n < 1 || n > D->steps) return afail(D2Q9_E_ARG, "adjoint steps: 1 .. steps per launch");
+  const int rows = D->rows - 2 * (D->steps - n);
+  const int tr = rows - 2 * n, tc = D->width - 2 * n;
+  const int ntj = (L->ny + tc - 1) / tc, tiles = (L->nx + tr - 1) / tr * ntj;
+  const dim3 grid((unsigned)tiles), block((unsigned)((rows * D->width + 63) / 64 * 64));
+  const size_t lds = (size_t)rows * D->width * 9 * sizeof(double);
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  auto ls = static_cast<const double*>(lam_src);
+  auto ld = static_cast<double*>(lam_dst);
+  auto m = static_cast<const double*>(mom);
+  auto su = static_cast<const double*>(seed_u);
+  auto gf = static_cast<double*>(grad_force);
+  hipError_t e = hipErrorInvalidValue;
+#define D2Q9_ADJ_ONE(FO, WV)                                                                   \
+  case WV: {                                                                                   \
+    auto kern = k_adjoint_tiled<FO, WV>;                                                       \
+    static const hipError_t limit =                                                            \
+        hipFuncSetAttribute(reinterpret_cast<const void*>(kern),                               \
+                            hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);           \
+    if ((e = limit) != hipSuccess) break;                                                      \
+    hipLaunchKernelGGL(kern, grid, block, lds, s, *L, *D, tiles, ntj, n, rows, last_streamed,  \
+                       ls, ld, m, mom_stride, su, gf);                                         \
+    e = hipGetLastError();                                                                     \
+    break;                                                                                     \
+  }
+#define D2Q9_ADJ_TILED(FO)                                                                     \
+  switch (D->width) {                                                                          \
+    D2Q9_ADJ_ONE(FO, 16)                                                                       \
+    D2Q9_ADJ_ONE(FO, 32)                                                                       \
+    D2Q9_ADJ_ONE(FO, 64)                                                                       \
+  }
+  switch (L->forcing) {
+    case D2Q9_GUO_LINEAR: D2Q9_ADJ_TILED(D2Q9_GUO_LINEAR) break;
+    case D2Q9_GUO_SECOND_ORDER: D2Q9_ADJ_TILED(D2Q9_GUO_SECOND_ORDER) break;
+    default: return afail(D2Q9_E_UNSUPPORTED, "adjoint steps: a Guo forcing is needed");
+  }
+#undef D2Q9_ADJ_TILED
+#undef D2Q9_ADJ_ONE
   if (e != hipSuccess) {
     set_error(hipGetErrorString(e));
     return (int)e;

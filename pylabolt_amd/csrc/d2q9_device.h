@@ -46,6 +46,10 @@ namespace d2q9 {
 // d2q9_step.hip.
 void set_error(const char* what);
 
+// The argument checks of every single-lattice entry point (d2q9_step.hip):
+// 0, or D2Q9_E_ARG with the error text set.
+int validate_lattice(const d2q9_lattice* L);
+
 // Velocity set, reference ordering (base/lattice.py:50-59).
 __device__ constexpr int CX[9] = {0, 1, 0, -1, 0, 1, -1, -1, 1};
 __device__ constexpr int CY[9] = {0, 0, 1, 0, -1, 1, 1, -1, -1};

@@ -310,6 +310,10 @@ __global__ __launch_bounds__(MAX_CELLS, (waves_per_simd<S, FORCING>())) void k_t
                                  mom_stride);
 }
 
+// The checks of a descriptor every entry point makes (d2q9_tiled.hip): 0, or
+// a D2Q9_E_* code with the error text set.
+int check_desc(const d2q9_lattice* L, const d2q9_tiled_desc* D);
+
 // Arguments of one launch.
 struct Launch {
   int K, collide_first, write_mom;

@@ -2,7 +2,6 @@
 // unit per storage form).
 #include <hip/hip_runtime.h>
 
-#include "d2q9_reduce.h"
 #include "d2q9_tiled.h"
 
 using namespace d2q9;
@@ -16,6 +15,22 @@ int tfail(int code, const char* what) {
 
 }  // namespace
 
+int d2q9::tiled::check_desc(const d2q9_lattice* L, const d2q9_tiled_desc* D) {
+  if (D->steps < 1 || (D->width != 16 && D->width != 32 && D->width != 64) ||
+      2 * (int64_t)D->steps >= D->width || 2 * (int64_t)D->steps >= D->rows)
+    return tfail(D2Q9_E_ARG, "tiled sweep: bad region or step count");
+  if (D->n_elems < 0 || D->n_elems > tiled::MAX_ELEMS || (D->n_elems > 0 && !L->bc_elems) ||
+      !D->cells || !D->codes)
+    return tfail(D2Q9_E_ARG, "tiled sweep: bad special-cell tables");
+  if ((int64_t)D->rows * D->width > tiled::MAX_CELLS)
+    return tfail(D2Q9_E_TOO_LARGE, "tiled sweep: the region does not fit a workgroup");
+  // cells are addressed by 32-bit byte offsets
+  const uint64_t raw = L->storage == D2Q9_STORE_F64 ? 8 : (L->storage == D2Q9_STORE_F32 ? 4 : 2);
+  if ((uint64_t)L->pop_len * raw > 0xffffffffull || L->plane > 0x7fffffffll)
+    return tfail(D2Q9_E_TOO_LARGE, "tiled sweep: lattice over 4 GiB");
+  return 0;
+}
+
 extern "C" int d2q9_tiled_steps(const d2q9_lattice* L, const d2q9_tiled_desc* D, void* f_a,
                                 void* f_b, void* mom_a, void* mom_b, int32_t n,
                                 int collide_first, int write_moments, void* mom_steps,
@@ -25,19 +40,9 @@ extern "C" int d2q9_tiled_steps(const d2q9_lattice* L, const d2q9_tiled_desc* D,
     return tfail(D2Q9_E_ARG, "tiled steps: null buffer");
   if (f_a == f_b || mom_a == mom_b)
     return tfail(D2Q9_E_ARG, "tiled steps: the two buffers must differ");
-  if (n < 0 || D->steps < 1 || (D->width != 16 && D->width != 32 && D->width != 64) ||
-      2 * (int64_t)D->steps >= D->width || 2 * (int64_t)D->steps >= D->rows)
-    return tfail(D2Q9_E_ARG, "tiled steps: bad region or step count");
-  if (D->n_elems < 0 || D->n_elems > tiled::MAX_ELEMS || (D->n_elems > 0 && !L->bc_elems) ||
-      !D->cells || !D->codes)
-    return tfail(D2Q9_E_ARG, "tiled steps: bad special-cell tables");
+  if (n < 0) return tfail(D2Q9_E_ARG, "tiled steps: negative step count");
+  if (int r = tiled::check_desc(L, D)) return r;
   const size_t elem = L->storage == D2Q9_STORE_F64 ? 8 : 4;
-  const size_t raw = L->storage == D2Q9_STORE_F64 ? 8 : (L->storage == D2Q9_STORE_F32 ? 4 : 2);
-  if ((int64_t)D->rows * D->width > tiled::MAX_CELLS)
-    return tfail(D2Q9_E_TOO_LARGE, "tiled steps: the region does not fit a workgroup");
-  // cells are addressed by 32-bit byte offsets
-  if ((uint64_t)L->pop_len * raw > 0xffffffffull || L->plane > 0x7fffffffll)
-    return tfail(D2Q9_E_TOO_LARGE, "tiled steps: lattice over 4 GiB");
   if (n == 0) return 0;
   // launches of nearly equal length: the work on grown cells rises with the
   // steps of a launch

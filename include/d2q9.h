@@ -414,6 +414,34 @@ int d2q9_batched_step(const d2q9_batch_entry* entries,
                       int write_moments, void* stream);
 
 /*
+ * Batched tiled sweep: n fused steps of many lattices of one storage type
+ * (FP64 or FP32), up to `steps` per launch, as d2q9_tiled_steps on each.  An
+ * entry carries a lattice, its tables (the region's shape is the call's) and
+ * its buffers; at parity p a launch goes from f[p] / mom[p] to f[1-p] /
+ * mom[1-p], and the next launch the other way.  Items list every tile of
+ * every lattice: tile (ti, tj) covers the (rows - 2 steps) x (width - 2 steps)
+ * cells from (1 + ti (rows - 2 steps), 1 + tj (width - 2 steps)) on.  planes:
+ * the most LDS values a cell of any entry needs, 9 + (has_vel ? 1 : 0) +
+ * (has_pres ? 2 : 0).  Entries and items are device memory; every entry must
+ * meet the conditions of d2q9_tiled_steps.
+ */
+typedef struct d2q9_tiled_entry {
+  d2q9_lattice L;
+  d2q9_tiled_desc D;
+  void* f[2];
+  void* mom[2];
+} d2q9_tiled_entry;
+
+typedef struct d2q9_tiled_item {
+  int32_t lattice, ti, tj;
+} d2q9_tiled_item;
+
+int d2q9_tiled_batch(const d2q9_tiled_entry* entries, const d2q9_tiled_item* items,
+                     int32_t n_items, int storage, int32_t rows, int32_t width,
+                     int32_t steps, int32_t planes, int32_t n, int parity,
+                     int collide_first, int write_moments, void* stream);
+
+/*
  * Adjoint of one FP64 step (BGK, Guo forcing, per-cell force field;
  * bounce-back, periodic and static-solid boundaries only, so that streaming
  * permutes the populations).  lam_src = dL/d(post-collision populations of

@@ -105,6 +105,12 @@ class TiledDesc(ctypes.Structure):
                 ("cells", ctypes.c_void_p), ("codes", ctypes.c_void_p)]
 
 
+class TiledEntry(ctypes.Structure):
+    """Mirror of ``d2q9_tiled_entry``."""
+    _fields_ = [("L", Lattice), ("D", TiledDesc), ("f", ctypes.c_void_p * 2),
+                ("mom", ctypes.c_void_p * 2)]
+
+
 # boundary elements a launch of the tiled sweep holds (d2q9_tiled_desc)
 TILED_MAX_ELEMS = 32
 
@@ -148,6 +154,7 @@ SIGNATURES = {
     "d2q9_adjoint_init_grad": (ctypes.c_int, [_LP, _P, _P, _P, _P]),
     "d2q9_batched_step": (ctypes.c_int, [_P, _P, _P, _P] + [ctypes.c_int] * 9
                           + [_P]),
+    "d2q9_tiled_batch": (ctypes.c_int, [_P, _P] + [ctypes.c_int] * 10 + [_P]),
     "d2q9_momentum_exchange": (ctypes.c_int, [_LP, _P, _P, _P, _P,
                                               ctypes.c_int64, _P, ctypes.c_int,
                                               _P, _P, _P]),

@@ -11,6 +11,11 @@ whole, large ones in row-ordered pieces), and a fixed grid of workgroups
 walks them statically or claims them with atomic counters.
 Full chunks of steps replay a captured HIP graph.
 
+Where every lattice has the tables of the tiled sweep (``D2Q9Engine.tiled``),
+``advance`` takes that instead: several steps of all lattices per launch
+(``d2q9_tiled_batch``), bitwise the same; the launch configuration below is
+then that of the persistent kernel for the other cases.
+
 ``BatchAutotuner`` picks the tile shape (rows per workgroup), the register
 budget of the kernel build (waves per SIMD), the queue policy, the grid and
 the claim size by timing candidates on the batch itself, and caches the
@@ -27,7 +32,7 @@ import numpy as np
 import torch
 
 from pylabolt_amd import _native as nt
-from pylabolt_amd.engine import ORIGIN
+from pylabolt_amd.engine import ORIGIN, tiled_shape
 
 N_XCD = 8
 POLICY_STATIC, POLICY_DYNAMIC = 0, 1
@@ -183,6 +188,7 @@ class BatchedLattices:
                 dtype=torch.uint8, device=self.device)
         self._entry_key = None
         self.cells = sum(e.nx * e.ny for e in self.engines)
+        self._setup_tiled()
         self.config = None
         if config is None:
             tuner = tuner if tuner is not None else BatchAutotuner()
@@ -301,6 +307,80 @@ class BatchedLattices:
         self._graphs[self.parity] = handle
         return handle
 
+    # ---- tiled sweep --------------------------------------------------------
+    def _setup_tiled(self):
+        """Region shape, entry table and tile list of the tiled sweep over
+        the whole batch; off where some lattice has no tables for it."""
+        self.tiled = all(e.tiled is not None for e in self.engines)
+        self._tiled_key = None
+        if not self.tiled:
+            return
+        self._tiled_region = tiled_shape(
+            tuple((e.nx, e.ny) for e in self.engines),
+            self.storage == "f64",
+            any(e.forcing is not None for e in self.engines))
+        rows, width, steps = self._tiled_region
+        items = []
+        for l, e in enumerate(self.engines):
+            ti, tj = np.meshgrid(np.arange(-(-e.nx // (rows - 2 * steps))),
+                                 np.arange(-(-e.ny // (width - 2 * steps))),
+                                 indexing="ij")
+            items.append(np.stack([np.full(ti.size, l), ti.ravel(),
+                                   tj.ravel()], axis=1))
+        items = np.concatenate(items).astype(np.int32)
+        self._tiled_count = int(items.shape[0])
+        self._tiled_planes = max(9 + (1 if e.tiled.has_vel else 0) +
+                                 (2 if e.tiled.has_pres else 0)
+                                 for e in self.engines)
+        with torch.cuda.stream(self.stream):
+            self._tiled_items = torch.from_numpy(items.reshape(-1)).to(
+                self.device)
+            self._tiled_entries = torch.zeros(
+                len(self.engines) * ctypes.sizeof(nt.TiledEntry),
+                dtype=torch.uint8, device=self.device)
+
+    def _sync_tiled_entries(self, src):
+        """(Re)write the tiled sweep's entry table so that entry l's
+        f[parity] is buffer ``src[l]`` of engine l."""
+        key = tuple((s ^ self.parity, e.i_mom ^ self.parity)
+                    for s, e in zip(src, self.engines))
+        if key == self._tiled_key:
+            return
+        arr = (nt.TiledEntry * len(self.engines))()
+        p = self.parity
+        for l, (s, e) in enumerate(zip(src, self.engines)):
+            arr[l].L, arr[l].D = e.L, e.tiled
+            arr[l].f[p] = e.f[s].data_ptr()
+            arr[l].f[1 - p] = e.f[1 - s].data_ptr()
+            arr[l].mom[p] = e.mom[e.i_mom].data_ptr()
+            arr[l].mom[1 - p] = e.mom[1 - e.i_mom].data_ptr()
+        host = torch.frombuffer(bytearray(bytes(arr)), dtype=torch.uint8)
+        with torch.cuda.stream(self.stream):
+            self._tiled_entries.copy_(host)
+        self.stream.synchronize()
+        self._tiled_key = key
+
+    def _advance_tiled(self, n, write_moments):
+        """``n`` steps of every lattice; the first one collides ``pop_new``
+        where that is in memory (of every lattice)."""
+        first = self.engines[0].i_pop_new is not None
+        src = [e.i_pop_new if first else e.i_pop for e in self.engines]
+        self._sync_tiled_entries(src)
+        rows, width, steps = self._tiled_region
+        nt.check(self.lib.d2q9_tiled_batch(
+            nt.ptr(self._tiled_entries), nt.ptr(self._tiled_items),
+            self._tiled_count, self.engines[0].storage, rows, width, steps,
+            self._tiled_planes, n, self.parity, int(first),
+            int(write_moments), self._sp), "d2q9_tiled_batch")
+        flip = -(-n // steps) & 1
+        for s, e in zip(src, self.engines):
+            e.i_pop = s ^ flip
+            e.i_mom ^= flip
+            e.i_pop_new = None
+            e.time_step += n
+            e.mom_full = bool(write_moments)
+        self.parity ^= flip
+
     # ---- stepping ---------------------------------------------------------
     @property
     def time_step(self):
@@ -315,7 +395,12 @@ class BatchedLattices:
         t0 = self.engines[0].time_step
         if any(e.time_step != t0 for e in self.engines):
             raise RuntimeError("batched lattices must advance in lockstep")
-        if any(e.i_pop_new is not None for e in self.engines):
+        fresh = sum(e.i_pop_new is not None for e in self.engines)
+        if self.tiled and fresh in (0, len(self.engines)) and all(
+                e.tiled is not None for e in self.engines):
+            self._advance_tiled(n, write_moments)
+            return
+        if fresh:
             # first step after initialisation: collide-only, per lattice
             for e in self.engines:
                 e.step(write_moments and n == 1)

@@ -1,8 +1,8 @@
-// C-ABI entry of the tiled sweep (kernel in d2q9_tiled.h, one translation
-// unit per storage form).
+// C-ABI entries of the tiled sweep (kernels in d2q9_tiled.h and
+// d2q9_tiled_batch.h, one translation unit per storage form).
 #include <hip/hip_runtime.h>
 
-#include "d2q9_tiled.h"
+#include "d2q9_tiled_batch.h"
 
 using namespace d2q9;
 
@@ -78,6 +78,46 @@ extern "C" int d2q9_tiled_steps(const d2q9_lattice* L, const d2q9_tiled_desc* D,
     }
     done += A.K;
     A.msrc = per_step ? per_step + (done - 1) * step_bytes : A.mdst;
+  }
+  return 0;
+}
+
+extern "C" int d2q9_tiled_batch(const d2q9_tiled_entry* entries, const d2q9_tiled_item* items,
+                                int32_t n_items, int storage, int32_t rows, int32_t width,
+                                int32_t steps, int32_t planes, int32_t n, int parity,
+                                int collide_first, int write_moments, void* stream) {
+  if (!entries || !items) return tfail(D2Q9_E_ARG, "tiled batch: null buffer");
+  if (n < 0 || n_items < 0 || (parity != 0 && parity != 1) || planes < 9 || planes > 12 ||
+      steps < 1 || (width != 16 && width != 32 && width != 64) || 2 * (int64_t)steps >= width ||
+      2 * (int64_t)steps >= rows)
+    return tfail(D2Q9_E_ARG, "tiled batch: bad region, steps, planes or parity");
+  if ((int64_t)rows * width > tiled::MAX_CELLS)
+    return tfail(D2Q9_E_TOO_LARGE, "tiled batch: the region does not fit a workgroup");
+  if (storage != D2Q9_STORE_F64 && storage != D2Q9_STORE_F32)
+    return tfail(D2Q9_E_UNSUPPORTED, "tiled batch: FP64 or FP32 storage only");
+  if (n == 0 || n_items == 0) return 0;
+  const int launches = (n + steps - 1) / steps;
+  const int base = n / launches, longer = n % launches;
+  tiled::BatchLaunch A;
+  A.entries = entries;
+  A.items = items;
+  A.n_items = n_items;
+  A.width = width;
+  A.tile_c = width - 2 * steps;
+  A.planes = planes;
+  A.stream = static_cast<hipStream_t>(stream);
+  for (int a = 0; a < launches; ++a) {
+    A.K = base + (a < longer ? 1 : 0);
+    A.rows = rows - 2 * (steps - A.K);
+    A.collide_first = a == 0 && collide_first;
+    A.write_mom = a == launches - 1 && write_moments;
+    A.parity = (parity + a) & 1;
+    const hipError_t e = storage == D2Q9_STORE_F64 ? tiled::launch_batch<D2Q9_STORE_F64>(A)
+                                                   : tiled::launch_batch<D2Q9_STORE_F32>(A);
+    if (e != hipSuccess) {
+      set_error(hipGetErrorString(e));
+      return (int)e;
+    }
   }
   return 0;
 }

@@ -590,8 +590,9 @@ _TILED_CUS = 256
 
 
 @functools.lru_cache(maxsize=256)
-def tiled_shape(nx, ny, double, forced):
-    """(rows, width, steps) of the tiled sweep's region for a lattice.
+def tiled_shape(sizes, double, forced):
+    """(rows, width, steps) of the tiled sweep's region for the lattices of
+    ``sizes``, a tuple of (nx, ny), swept by one launch.
 
     More steps per launch share its latency but grow the work on cells that
     several tiles compute; smaller regions spread a small lattice over more
@@ -607,7 +608,8 @@ def tiled_shape(nx, ny, double, forced):
             if cols <= 0:
                 continue
             for rows in range(2 * steps + 2, most // width + 1, 2):
-                tiles = -(-nx // (rows - 2 * steps)) * -(-ny // cols)
+                tiles = sum(-(-nx // (rows - 2 * steps)) * -(-ny // cols)
+                            for nx, ny in sizes)
                 # a last round that is partly empty matters for few rounds
                 per_cu = (-(-tiles // _TILED_CUS) if tiles <= 4 * _TILED_CUS
                           else tiles / _TILED_CUS + 0.5)
@@ -953,7 +955,7 @@ class D2Q9Engine:
             return
         cells, codes, has_vel, has_pres = tables
         rows, width, steps = tiled_shape(
-            self.nx, self.ny, self.storage == nt.STORE_F64,
+            ((self.nx, self.ny),), self.storage == nt.STORE_F64,
             self.forcing is not None)
         with torch.cuda.stream(self.stream):
             dev = {"cells": self._upload_plane(cells, torch.int32),

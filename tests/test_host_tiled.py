@@ -142,6 +142,6 @@ def test_special_codes_refuse_many_elements():
 @pytest.mark.parametrize("double", [True, False])
 @pytest.mark.parametrize("forced", [True, False])
 def test_tiled_shape_fits_a_workgroup(nx, ny, double, forced):
-    rows, width, steps = tiled_shape(nx, ny, double, forced)
+    rows, width, steps = tiled_shape(((nx, ny),), double, forced)
     assert width in (16, 32, 64) and rows * width <= 1024
     assert steps >= 1 and rows > 2 * steps and width > 2 * steps

@@ -414,6 +414,44 @@ int d2q9_batched_step(const d2q9_batch_entry* entries,
                       int write_moments, void* stream);
 
 /*
+ * Strip sweep: n fused steps, up to 4 per launch, as d2q9_tiled_steps (bitwise
+ * single steps; with round_last, 16-bit storage rounds only the last step of
+ * a launch, which keeps the others in FP32).  d2q9_strip_shape gives the most
+ * steps of a launch, a strip's output columns and a tile's output rows and
+ * columns.
+ *
+ * chunks: `cols` (at most a strip's) columns from j_first on by `rows` rows
+ * from i_first on.  Every cell of a chunk and within `steps` cells of it is
+ * plain fluid (flag D2Q9_CELL_FLUID only; periodic images count), but for the
+ * lattice's first and last column, which may be a straight wall along all those
+ * rows: walls bits 0-1 at j = 1, bits 2-3 at j = ny, 1 zero-gradient, 2
+ * bounce-back; cells beyond such a wall are not read.  tiles: (i_first,
+ * j_first) of tiles whose cells together with the chunks' cover every fluid
+ * cell; a cell in several of them is written with the same bits.  D: the
+ * tables of d2q9_tiled_steps (its region is not used), with their conditions.
+ * The caller guarantees the lists; chunks are device memory, tiles too.
+ */
+typedef struct d2q9_strip_chunk {
+  int32_t i_first, rows, j_first, cols, walls;
+} d2q9_strip_chunk;
+
+typedef struct d2q9_strip_tile {
+  int32_t i_first, j_first;
+} d2q9_strip_tile;
+
+typedef struct d2q9_strip_desc {
+  int32_t n_chunks, n_tiles;
+  const d2q9_strip_chunk* chunks;
+  const d2q9_strip_tile* tiles;
+} d2q9_strip_desc;
+
+int d2q9_strip_shape(int32_t* steps, int32_t* cols, int32_t* tile);
+int d2q9_strip_steps(const d2q9_lattice* L, const d2q9_tiled_desc* D,
+                     const d2q9_strip_desc* P, void* f_a, void* f_b, void* mom_a,
+                     void* mom_b, int32_t n, int write_moments, int round_last,
+                     void* stream);
+
+/*
  * Batched tiled sweep: n fused steps of many lattices of one storage type
  * (FP64 or FP32), up to `steps` per launch, as d2q9_tiled_steps on each.  An
  * entry carries a lattice, its tables (the region's shape is the call's) and

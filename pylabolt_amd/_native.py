@@ -111,6 +111,12 @@ class TiledEntry(ctypes.Structure):
                 ("mom", ctypes.c_void_p * 2)]
 
 
+class StripDesc(ctypes.Structure):
+    """Mirror of ``d2q9_strip_desc``."""
+    _fields_ = [("n_chunks", ctypes.c_int32), ("n_tiles", ctypes.c_int32),
+                ("chunks", ctypes.c_void_p), ("tiles", ctypes.c_void_p)]
+
+
 # boundary elements a launch of the tiled sweep holds (d2q9_tiled_desc)
 TILED_MAX_ELEMS = 32
 
@@ -154,6 +160,11 @@ SIGNATURES = {
     "d2q9_adjoint_init_grad": (ctypes.c_int, [_LP, _P, _P, _P, _P]),
     "d2q9_batched_step": (ctypes.c_int, [_P, _P, _P, _P] + [ctypes.c_int] * 9
                           + [_P]),
+    "d2q9_strip_shape": (ctypes.c_int, [ctypes.POINTER(ctypes.c_int32)] * 3),
+    "d2q9_strip_steps": (ctypes.c_int, [_LP, ctypes.POINTER(TiledDesc),
+                                        ctypes.POINTER(StripDesc), _P, _P, _P,
+                                        _P, ctypes.c_int32, ctypes.c_int,
+                                        ctypes.c_int, _P]),
     "d2q9_tiled_batch": (ctypes.c_int, [_P, _P] + [ctypes.c_int] * 10 + [_P]),
     "d2q9_momentum_exchange": (ctypes.c_int, [_LP, _P, _P, _P, _P,
                                               ctypes.c_int64, _P, ctypes.c_int,

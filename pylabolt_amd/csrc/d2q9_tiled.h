@@ -124,9 +124,9 @@ __device__ __forceinline__ int arith_elem(uint32_t a, int which) {
   return (int)((a >> (which ? 24 : 16)) & 0xffu);
 }
 
-// K steps of the output tile whose first cell is (1 + ti tile_r, 1 + tj
-// tile_c), tile_r = rows - 2 K, tile_c <= W - 2 K: region of `rows` x W cells, a
-// wave holding 64 / W rows, one cell per thread.  LDS element of direction k of region
+// K steps of the output tile of (rows - 2 K) x tile_c cells from (i_first,
+// j_first) on, tile_c <= W - 2 K: region of `rows` x W cells, a wave holding 64 /
+// W rows, one cell per thread.  LDS element of direction k of region
 // cell e: 9 e + k (an odd stride: no bank conflicts, and every neighbour at
 // a constant distance).  mom_steps, when not null, receives rho/u of every
 // owned cell after every step (step s at mom_steps + s * mom_stride), and
@@ -134,8 +134,8 @@ __device__ __forceinline__ int arith_elem(uint32_t a, int which) {
 // collision of the loaded populations alone (no streaming).
 template <int S, int MODEL, int FORCING, int W>
 __device__ __forceinline__ void run_tile(
-    const d2q9_lattice& L, const d2q9_tiled_desc& D, char* __restrict__ smem, int ti, int tj,
-    int tile_c, int K, int rows, int collide_first, const typename Codec<S>::raw* __restrict__ fsrc,
+    const d2q9_lattice& L, const d2q9_tiled_desc& D, char* __restrict__ smem, int i_first,
+    int j_first, int tile_c, int K, int rows, int collide_first, const typename Codec<S>::raw* __restrict__ fsrc,
     typename Codec<S>::raw* __restrict__ fdst, const typename Codec<S>::T* __restrict__ msrc,
     typename Codec<S>::T* __restrict__ mdst, int write_mom,
     typename Codec<S>::T* __restrict__ mom_steps, int64_t mom_stride) {
@@ -150,8 +150,7 @@ __device__ __forceinline__ void run_tile(
   T* const su = srho + (D.has_vel ? area : 0);
   d2q9_bc_elem* const elems = reinterpret_cast<d2q9_bc_elem*>(s + lds_values(D, area));
   const Consts<T> Kc = load_consts<T>(L);
-  const int i0 = 1 + ti * (rows - 2 * K) - K;   // lattice row of region row 0
-  const int j0 = 1 + tj * tile_c - K;
+  const int i0 = i_first - K, j0 = j_first - K;   // the region's first cell
   // the whole region lies in the lattice: nothing to wrap or to leave out
   const bool inside = i0 > 0 && i0 + rows <= L.nx + 1 && j0 > 0 && j0 + W <= L.ny + 1;
   if (D.has_vel || D.has_pres)
@@ -307,7 +306,8 @@ __global__ __launch_bounds__(MAX_CELLS, (waves_per_simd<S, FORCING>())) void k_t
     typename Codec<S>::T* __restrict__ mom_steps, int64_t mom_stride) {
   extern __shared__ __align__(16) char smem[];
   const int tile = xcd_remap((int)blockIdx.x, ntiles);
-  run_tile<S, MODEL, FORCING, W>(L, D, smem, tile / ntj, tile % ntj, W - 2 * K, K, rows,
+  run_tile<S, MODEL, FORCING, W>(L, D, smem, 1 + (tile / ntj) * (rows - 2 * K),
+                                 1 + (tile % ntj) * (W - 2 * K), W - 2 * K, K, rows,
                                  collide_first, fsrc, fdst, msrc, mdst, write_mom, mom_steps,
                                  mom_stride);
 }

@@ -32,8 +32,9 @@ __global__ __launch_bounds__(MAX_CELLS, S == D2Q9_STORE_F64 ? 4 : 8) void k_tile
   auto md = static_cast<typename C::T*>(E.mom[1 - parity]);
 #define D2Q9_TILED_ITEM(KEY, M, F)                                                         \
   case KEY:                                                                                \
-    run_tile<S, M, F, W>(L, D, smem, it.ti, it.tj, tile_c, K, rows, collide_first, fs, fd, \
-                         ms, md, write_mom, nullptr, 0);                                   \
+    run_tile<S, M, F, W>(L, D, smem, 1 + it.ti * (rows - 2 * K), 1 + it.tj * tile_c,       \
+                         tile_c, K, rows, collide_first, fs, fd, ms, md, write_mom,        \
+                         nullptr, 0);                                                      \
     break;
   switch (L.collision * 3 + L.forcing) {
     D2Q9_TILED_ITEM(0, D2Q9_BGK, D2Q9_FORCING_NONE)

@@ -400,6 +400,82 @@ class CaseTables:
         codes[:n, 2] = np.where(first >= 0, arith, 0)
         return cells, codes, has_vel, has_pres
 
+    def strip_split(self, steps, cols, tile, chunk_rows):
+        """Chunks and tiles of the strip sweep (d2q9_strip_steps).
+
+        Strips of ``cols`` columns (the last one moved to end at the last
+        column) are cut along x into chunks of about ``chunk_rows`` rows
+        whose cells, and the cells within ``steps`` of them, are all plain
+        fluid -- or the straight zero-gradient or bounce-back wall of the
+        first or last column, of one kind along those rows.  Periodic sides
+        count as their images.  Every fluid cell in no chunk lies in a tile of
+        ``tile`` x ``tile`` cells.  Returns (chunks [n, 5] int32: first row,
+        rows, first column, columns, walls; tiles [m, 2] int32; the share of
+        the cells in tiles), rows and columns from 1, or None when a strip
+        does not fit."""
+        nx, ny = self.nx, self.ny
+        if ny < cols + 2 * steps or nx < 2 * steps + 1:
+            return None
+        inner = self.flags_pad[1:-1, 1:-1]
+        rough = inner != nt.CELL_FLUID
+        side = self.wall_side_pad[1:-1, 1:-1]
+        inl = self.wall_inline_wrap if self.x_periodic else self.wall_inline
+        lo_kind = np.where(inl[:, 0] & (side[:, 0] == 0), 1,
+                           np.where(inl[:, 0] & (side[:, 0] == 2), 2, -1))
+        hi_kind = np.where(inl[:, -1] & (side[:, -1] == 1), 1,
+                           np.where(inl[:, -1] & (side[:, -1] == 3), 2, -1))
+        starts = list(range(0, ny - cols, cols)) + [ny - cols]
+        chunks = []
+        covered = np.zeros((nx, ny), dtype=bool)
+        for js in starts:
+            c0, c1 = js - steps, js + cols + steps   # region columns
+            if self.y_periodic:
+                bad = np.take(rough, np.arange(c0, c1) % ny,
+                              axis=1).any(axis=1)
+                label = np.where(bad, -1, 0)
+            else:
+                at_lo, at_hi = c0 <= 0, c1 >= ny
+                a, b = max(c0, 1 if at_lo else 0), min(c1, ny - 1 if at_hi
+                                                       else ny)
+                bad = rough[:, a:b].any(axis=1)
+                label = np.zeros(nx, dtype=np.int64)
+                if at_lo:
+                    bad |= lo_kind < 0
+                    label |= np.maximum(lo_kind, 0)
+                if at_hi:
+                    bad |= hi_kind < 0
+                    label |= np.maximum(hi_kind, 0) << 2
+                label[bad] = -1
+            # rows of one label, with the images past a periodic end
+            ext = (np.concatenate([label[-steps:], label, label[:steps]])
+                   if self.x_periodic else label)
+            off = steps if self.x_periodic else 0
+            edges = np.flatnonzero(np.diff(ext)) + 1
+            for s, e in zip(np.concatenate([[0], edges]),
+                            np.concatenate([edges, [ext.size]])):
+                if ext[s] < 0:
+                    continue
+                a = max(s + steps - off, 0)
+                b = min(e - steps - off, nx)
+                if b - a < 2 * tile:
+                    continue
+                n = max(1, int(round((b - a) / chunk_rows)))
+                cut = [a + (b - a) * q // n for q in range(n + 1)]
+                chunks += [(cut[q] + 1, cut[q + 1] - cut[q], js + 1, cols,
+                            int(ext[s])) for q in range(n)]
+                covered[a:b, js:js + cols] = True
+        # neighbouring strips of the same rows next to each other
+        chunks.sort(key=lambda c: (c[0], c[2]))
+        left = ~covered & ((inner & nt.CELL_FLUID) != 0)
+        nti, ntj = -(-nx // tile), -(-ny // tile)
+        pad = np.zeros((nti * tile, ntj * tile), dtype=bool)
+        pad[:nx, :ny] = left
+        ti, tj = np.nonzero(pad.reshape(nti, tile, ntj, tile).any(axis=(1, 3)))
+        tiles = np.stack([1 + ti * tile, 1 + tj * tile], axis=1)
+        return (np.asarray(chunks, dtype=np.int32).reshape(-1, 5),
+                tiles.astype(np.int32), tiles.shape[0] * tile * tile /
+                float(nx * ny))
+
     def deep_split(self, rows):
         """Deep tiles of the two-step sweep (d2q9_fused_step2) and the rim
         tables around them.

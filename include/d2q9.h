@@ -425,7 +425,7 @@ int d2q9_batched_step(const d2q9_batch_entry* entries,
  * plain fluid (flag D2Q9_CELL_FLUID only; periodic images count), but for the
  * lattice's first and last column, which may be a straight wall along all those
  * rows: walls bits 0-1 at j = 1, bits 2-3 at j = ny, 1 zero-gradient, 2
- * bounce-back; cells beyond such a wall are not read.  tiles: (i_first,
+ * bounce-back; cells beyond such a wall are not used, and the wall is a column of the chunk.  tiles: (i_first,
  * j_first) of tiles whose cells together with the chunks' cover every fluid
  * cell; a cell in several of them is written with the same bits.  D: the
  * tables of d2q9_tiled_steps (its region is not used), with their conditions.

@@ -1,19 +1,22 @@
-// Strip sweep: up to STRIP_STEPS fused time steps per pass over the plain
-// interior of a large lattice.
+// Strip sweep: up to STEPS fused time steps per pass over the plain interior
+// of a large lattice.
 //
-// A workgroup sweeps a chunk -- a strip of 64 - 2 STRIP_STEPS output columns
-// by a run of rows -- row by row, one wave per time step: in every iteration
-// wave s - 1 computes one row of step s, two rows behind the wave before it,
-// so that the three rows it pulls from are there.  Steps hand rows on through
-// LDS rings that hold what is still to be pulled: three rows of the
-// directions pulled from the same or the next row, four of those pulled from
-// the row before.  The first wave pulls from the lattice (a row ahead, in
-// registers), the last stores to the other one.
+// A workgroup sweeps a chunk -- a strip of columns by a run of rows -- row by
+// row, one wave per time step: in every iteration wave s - 1 computes one row
+// of step s, two rows behind the wave before it, so that the three rows it
+// pulls from are there.  Steps hand rows on through LDS rings that hold what
+// is still to be pulled: three rows of the directions pulled from the same or
+// the next row, four of those pulled from the row before.  The first wave
+// pulls from the lattice (rows ahead, in registers), the last stores to the
+// other one.  A lane holds one cell, so a row is 64 cells wide, STEPS of them on
+// either side for the neighbouring strips' sake only.  (Two cells a lane for the
+// float forms halve the waves a CU holds: FP32 2999x1111 22 us per step against
+// 18, 8192x2048 97 against 91.)
 //
 // Compared with a tile held in LDS, cells are computed twice only at the sides
-// of a strip (64 lanes for 56 columns) and at the ends of a chunk, and loads,
-// arithmetic and stores of different rows overlap.  Per K steps the lattice is
-// read 64 / 56 times and written once.
+// of a strip (64 for 56 columns) and at the ends of a chunk, and loads,
+// arithmetic and stores of different rows overlap.  Per STEPS steps the lattice
+// is read about 1.15 times and written once.
 //
 // Chunks hold plain cells only, but for a straight zero-gradient or
 // bounce-back wall in the lattice's first or last column; every other cell
@@ -28,27 +31,20 @@ namespace d2q9 {
 namespace strip {
 
 constexpr int STEPS = 4;                     // most steps of a launch
-constexpr int LANES = 64;
-constexpr int COLS = LANES - 2 * STEPS;      // output columns of a strip
 constexpr int THREADS = 64 * STEPS;
+constexpr int COLS = 64 - 2 * STEPS;         // output columns of a strip
 constexpr int TILE_W = 16;                   // region width of the tiles
 constexpr int TILE = TILE_W - 2 * STEPS;     // their output rows and columns
-constexpr int PITCH = LANES + 2;
-// dir-rows of a ring: 3 rows of directions 0,2,4, 3 of 3,6,7, 4 of 1,5,8
+constexpr int AHEAD = 2;                     // rows the first wave loads ahead
+// Rows of a ring, three directions each: 3 of 0,2,4, 3 of 3,6,7, 4 of 1,5,8.
 constexpr int RING_B = 9, RING_C = 18, RING = 30;
 
-// Place of direction k in its group of three, and the group's first dir-row.
+// Place of direction k in its group of three.
 __device__ constexpr int SLOT[9] = {0, 0, 1, 0, 2, 1, 1, 2, 2};
-__device__ constexpr int BASE[9] = {0, RING_C, 0, RING_B, 0, RING_C, RING_B, RING_B, RING_C};
 
-// One stored element as an integer (non-temporal stores take no half types).
-template <size_t BYTES> struct Word;
-template <> struct Word<2> { using type = unsigned short; };
-template <> struct Word<4> { using type = uint32_t; };
-template <> struct Word<8> { using type = uint64_t; };
-
+constexpr int PITCH = 64 + 2;                // values of an LDS row
 template <int S>
-__host__ __device__ constexpr size_t ring_bytes(int steps) {
+constexpr size_t ring_bytes(int steps) {
   return (size_t)(steps - 1) * RING * PITCH * sizeof(typename Codec<S>::T);
 }
 
@@ -65,7 +61,9 @@ __device__ __forceinline__ void run_strip(
   const int st = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6) + 1;  // this wave's step
   const Consts<T> Kc = load_consts<T>(L);
   const int lo = ch.walls & 3, hi = (ch.walls >> 2) & 3;
-  // the lane's column, its neighbours' places in a row
+  // the lane's column; columns past a periodic side are their images, other
+  // ones outside the lattice are clamped and never used
+  const int ju = ch.j_first - STEPS + lane;
   auto column = [&](int j) {
     if (L.y_periodic) {
       if (j < 1) j += L.ny;
@@ -73,15 +71,18 @@ __device__ __forceinline__ void run_strip(
     }
     return min(max(j, 0), L.ny + 1);
   };
-  auto place = [&](int j) {
+  auto place = [&](int j) {   // in a row of the lattice
     const unsigned jj = (unsigned)(j + B - 1);
     return ((jj / B) * (9u * B) + jj % B) * (unsigned)sizeof(R);
   };
-  const int ju = ch.j_first - K + lane, j = column(ju);
-  const bool out = lane >= K && lane < K + ch.cols;
+  const int j = column(ju);
+  const bool out = lane >= STEPS && lane < STEPS + ch.cols;
   const bool wall_lo = lo != 0 && ju == 1, wall_hi = hi != 0 && ju == L.ny;
   const bool zg = (wall_lo && lo == 1) || (wall_hi && hi == 1);
-  const bool bb = (wall_lo && lo == 2) || (wall_hi && hi == 2);
+  // the lane beside a bounce-back wall's cell loads that cell's own outward
+  // populations for it: the diagonals of row i itself, where the other lanes'
+  // come from rows i -+ 1
+  const bool helper = (lo == 2 && ju == 0) || (hi == 2 && ju == L.ny + 1);
   const unsigned p0 = place(j);
   // zero-gradient: the unknown directions are what the inner neighbour pulls,
   // from the wall cell's own column
@@ -89,11 +90,7 @@ __device__ __forceinline__ void run_strip(
   const unsigned pp = place(zg && wall_hi ? j : column(ju + 1));
   auto wrap = [&](int i) { return L.x_periodic ? (i < 1 ? i + L.nx : i > L.nx ? i - L.nx : i) : i; };
   auto row_at = [&](int i) {
-    return (uint64_t)((unsigned)wrap(i) * (unsigned)L.nbj) * (9u * B * (unsigned)sizeof(R));
-  };
-  auto load = [&](int i, int k, unsigned at) {
-    return *reinterpret_cast<const R*>(reinterpret_cast<const char*>(fsrc + k * B) + row_at(i) +
-                                       at);
+    return (unsigned)wrap(i) * (unsigned)L.nbj * (9u * B * (unsigned)sizeof(R));
   };
   // step `st` computes rows i_first - (K - st) .. i_first + rows - 1 + (K - st)
   const int begin = 3 * (st - 1), count = ch.rows + 2 * (K - st);
@@ -101,131 +98,132 @@ __device__ __forceinline__ void run_strip(
   int i = ch.i_first - (K - st);
   T* const to = reinterpret_cast<T*>(smem) + (st - 1) * RING * PITCH + 1 + lane;
   const T* const from = to - RING * PITCH;
-  // the first step's row, a row ahead; the wall's own opposite populations
-  R raw[9], back[3];
-  auto fetch = [&](int row) {
+  // The first step's rows, AHEAD of them in registers: with one, the memory
+  // system is mostly idle (FP64 8192x2048: 349 us per step against 165; four or
+  // six are no faster).
+  R raw[AHEAD][9];
+  auto fetch = [&](R (&r)[9], int row) {
+    const unsigned r0 = row_at(row), rp = row_at(row + 1), rm = row_at(row - 1);
+    const unsigned dp = helper ? r0 : rp, dm = helper ? r0 : rm;
 #pragma unroll
-    for (int k = 0; k < 9; ++k)
-      raw[k] = load(row - CX[k], k, CY[k] == 0 ? p0 : CY[k] > 0 ? pm : pp);
-    if (lo == 2 || hi == 2) {
-      if (wall_lo) {
-        back[0] = load(row, 4, p0);
-        back[1] = load(row, 7, p0);
-        back[2] = load(row, 8, p0);
-      }
-      if (wall_hi) {
-        back[0] = load(row, 2, p0);
-        back[1] = load(row, 5, p0);
-        back[2] = load(row, 6, p0);
-      }
+    for (int k = 0; k < 9; ++k) {
+      const unsigned at = CX[k] == 0 ? r0 : CX[k] < 0 ? (k > 4 ? dp : rp) : (k > 4 ? dm : rm);
+      r[k] = *reinterpret_cast<const R*>(reinterpret_cast<const char*>(fsrc + k * B) +
+                                         (at + (CY[k] == 0 ? p0 : CY[k] > 0 ? pm : pp)));
     }
   };
-  if (st == 1) fetch(i);
+  if (st == 1) {
+#pragma unroll
+    for (int q = 0; q < AHEAD; ++q)
+      if (q < count) fetch(raw[q], i + q);
+  }
   int a3 = 0, a4 = 0;   // ring slots this row is written to (row number mod 3 and 4)
 #pragma unroll 1
-  for (int t = 0; t < total; ++t) {
-    if (st <= K && t >= begin && t < begin + count) {
-      T g[9];
-      if (st == 1) {
+  for (int t0 = 0; t0 < total; t0 += AHEAD) {
 #pragma unroll
-        for (int k = 0; k < 9; ++k) g[k] = C::dec(raw[k], k, Kc);
-        if (lo == 2 || hi == 2) {
-          if (bb) {
-            // directions 2, 5, 6 from 4, 7, 8 (low wall), 4, 7, 8 from 2, 5, 6
+    for (int u = 0; u < AHEAD; ++u) {
+      const int t = t0 + u;
+      if (t >= total) break;   // the whole workgroup
+      if (st <= K && t >= begin && t < begin + count) {
+        T g[9];
+        if (st == 1) {
+#pragma unroll
+          for (int k = 0; k < 9; ++k) g[k] = C::dec(raw[u][k], k, Kc);
+          if (lo == 2) {
+            const T b4 = wave_from_prev(g[4]), b7 = wave_from_prev(g[7]),
+                    b8 = wave_from_prev(g[8]);
             if (wall_lo) {
-              g[2] = C::dec(back[0], 4, Kc);
-              g[5] = C::dec(back[1], 7, Kc);
-              g[6] = C::dec(back[2], 8, Kc);
-            } else {
-              g[4] = C::dec(back[0], 2, Kc);
-              g[7] = C::dec(back[1], 5, Kc);
-              g[8] = C::dec(back[2], 6, Kc);
+              g[2] = b4;
+              g[5] = b7;
+              g[6] = b8;
+            }
+          }
+          if (hi == 2) {
+            const T b2 = wave_from_next(g[2]), b5 = wave_from_next(g[5]),
+                    b6 = wave_from_next(g[6]);
+            if (wall_hi) {
+              g[4] = b2;
+              g[7] = b5;
+              g[8] = b6;
+            }
+          }
+          if (t + AHEAD < count) fetch(raw[u], i + AHEAD);
+        } else {
+          // rows i (number n + 1 of the step before), i + 1 (n + 2), i - 1 (n)
+          const int same = (a3 == 2 ? 0 : a3 + 1) * 3;
+          const int next = RING_B + (a3 == 0 ? 2 : a3 - 1) * 3;
+          const T* const r0 = from + same * PITCH;
+          const T* const rb = from + next * PITCH;
+          const T* const rc = from + (RING_C + a4 * 3) * PITCH;
+#pragma unroll
+          for (int k = 0; k < 9; ++k)
+            g[k] = (CX[k] == 0 ? r0 : CX[k] < 0 ? rb : rc)[SLOT[k] * PITCH - CY[k]];
+          if ((lo | hi) && (wall_lo || wall_hi)) {
+            const T* const own_b = from + (RING_B + same) * PITCH;
+            const T* const own_c = from + (RING_C + ((a4 + 1) & 3) * 3) * PITCH;
+#pragma unroll
+            for (int k = 1; k < 9; ++k) {
+              if (CY[k] == 0 || (CY[k] == 1 ? !wall_lo : !wall_hi)) continue;
+              const int o = INV[k];
+              g[k] = zg ? (CX[k] == 0 ? r0 : CX[k] < 0 ? rb : rc)[SLOT[k] * PITCH]
+                        : (CX[o] == 0 ? r0 : CX[o] < 0 ? own_b : own_c)[SLOT[o] * PITCH];
             }
           }
         }
-        if (t + 1 < begin + count) fetch(i + 1);
-      } else {
-        // rows i (number n + 1 of the step before), i + 1 (n + 2), i - 1 (n)
-        const int same = (a3 + 1 >= 3 ? a3 - 2 : a3 + 1) * 3;
-        const int next = RING_B + (a3 + 2 >= 3 ? a3 - 1 : a3 + 2) * 3;
-        const int prev = RING_C + a4 * 3;
-        const T* const r0 = from + same * PITCH;
-        const T* const rb = from + next * PITCH;
-        const T* const rc = from + prev * PITCH;
+        const int cell = L.origin + wrap(i) * L.pitch + j;
+        T ffx = (T)0, ffy = (T)0;
+        if (FORCING != D2Q9_FORCING_NONE && L.force_source == D2Q9_FSRC_FIELD) {
+          const T* ff = static_cast<const T*>(L.force_field);
+          ffx = ff[cell];
+          ffy = ff[L.plane + cell];
+        }
+        T drho, rho, ux, uy, fx, fy, px, py;
+        moments<T, FORCING, C::dev>(g, L, Kc, ffx, ffy, drho, rho, ux, uy, fx, fy, px, py);
+        collide<T, MODEL, FORCING, C::dev>(g, Kc, drho, rho, ux, uy, fx, fy, px, py);
+        const uint32_t key = sizeof(R) == 2 ? cell_key((uint32_t)cell) : 0u;
+        if (st < K) {
+          T* const w0 = to + a3 * 3 * PITCH;
+          T* const wc = to + (RING_C + a4 * 3) * PITCH;
+          if (sizeof(R) == 2 && !round_last) {
 #pragma unroll
-        for (int k = 0; k < 9; ++k)
-          g[k] = (CX[k] == 0 ? r0 : CX[k] < 0 ? rb : rc)[SLOT[k] * PITCH - CY[k]];
-        if (lo | hi) {
-          if (zg) {
+            for (int k = 0; k < 9; ++k) g[k] = tiled::through_storage<S>(g[k], k, key, Kc);
+          }
 #pragma unroll
-            for (int k = 1; k < 9; ++k)
-              if (CY[k] == 1 ? wall_lo : CY[k] == -1 ? wall_hi : false)
-                g[k] = (CX[k] == 0 ? r0 : CX[k] < 0 ? rb : rc)[SLOT[k] * PITCH];
-          } else if (bb) {
-            const T* const own_b = from + (RING_B + same) * PITCH;
-            const T* const own_c = from + (RING_C + (a4 + 1 & 3) * 3) * PITCH;
+          for (int k = 0; k < 9; ++k)
+            (CX[k] == 0 ? w0 : CX[k] < 0 ? w0 + RING_B * PITCH : wc)[SLOT[k] * PITCH] = g[k];
+        } else if (out) {
+          // plain stores: a strip's segments end inside cache lines that the
+          // next strip completes (non-temporal: FP32 8192x2048 91 us against 83)
+          const unsigned at = row_at(i) + p0;
 #pragma unroll
-            for (int k = 1; k < 9; ++k)
-              if (CY[k] == 1 ? wall_lo : CY[k] == -1 ? wall_hi : false)
-                g[k] = (CX[INV[k]] == 0 ? r0 : CX[INV[k]] < 0 ? own_b
-                                                              : own_c)[SLOT[INV[k]] * PITCH];
+          for (int k = 0; k < 9; ++k)
+            *reinterpret_cast<R*>(reinterpret_cast<char*>(fdst + k * B) + at) =
+                C::encs(g[k], k, key, Kc);
+          if (write_mom) {
+            mdst[cell] = rho;
+            mdst[L.plane + cell] = ux;
+            mdst[2 * L.plane + cell] = uy;
           }
         }
+        ++i;
+        a3 = a3 == 2 ? 0 : a3 + 1;
+        a4 = (a4 + 1) & 3;
       }
-      const int iw = wrap(i);
-      const int cell = L.origin + iw * L.pitch + j;
-      T ffx = (T)0, ffy = (T)0;
-      if (FORCING != D2Q9_FORCING_NONE && L.force_source == D2Q9_FSRC_FIELD) {
-        const T* ff = static_cast<const T*>(L.force_field);
-        ffx = ff[cell];
-        ffy = ff[L.plane + cell];
-      }
-      T drho, rho, ux, uy, fx, fy, px, py;
-      moments<T, FORCING, C::dev>(g, L, Kc, ffx, ffy, drho, rho, ux, uy, fx, fy, px, py);
-      collide<T, MODEL, FORCING, C::dev>(g, Kc, drho, rho, ux, uy, fx, fy, px, py);
-      const uint32_t key = sizeof(R) == 2 ? cell_key((uint32_t)cell) : 0u;
-      if (st < K) {
-        T* const w0 = to + a3 * 3 * PITCH;
-        T* const wc = to + (RING_C + a4 * 3) * PITCH;
-        if (sizeof(R) == 2 && !round_last) {
-#pragma unroll
-          for (int k = 0; k < 9; ++k) g[k] = tiled::through_storage<S>(g[k], k, key, Kc);
-        }
-#pragma unroll
-        for (int k = 0; k < 9; ++k)
-          (CX[k] == 0 ? w0 : CX[k] < 0 ? w0 + RING_B * PITCH : wc)[SLOT[k] * PITCH] = g[k];
-      } else if (out) {
-        char* const d = reinterpret_cast<char*>(fdst) + row_at(i);
-#pragma unroll
-        for (int k = 0; k < 9; ++k) {
-          using W = typename Word<sizeof(R)>::type;
-          const R v = C::encs(g[k], k, key, Kc);
-          W w;
-          __builtin_memcpy(&w, &v, sizeof(W));
-          store_nt(w, reinterpret_cast<W*>(d + (size_t)(k * B) * sizeof(R) + p0));
-        }
-        if (write_mom) {
-          mdst[cell] = rho;
-          mdst[L.plane + cell] = ux;
-          mdst[2 * L.plane + cell] = uy;
-        }
-      }
-      ++i;
-      a3 = a3 == 2 ? 0 : a3 + 1;
-      a4 = (a4 + 1) & 3;
+      __syncthreads();
     }
-    __syncthreads();
   }
 }
 
-template <int S, int FORCING>
+// Waves per SIMD the registers must allow: the rings of three FP64 chunks
+// (47.5 KB each) or six float ones fill a CU's LDS.
+template <int S>
 constexpr int waves_per_simd() {
   return S == D2Q9_STORE_F64 ? 4 : 6;
 }
 
 // Workgroups [0, n_tiles): tiles of TILE x TILE cells; the others: chunks.
 template <int S, int MODEL, int FORCING>
-__global__ __launch_bounds__(THREADS, (waves_per_simd<S, FORCING>())) void k_strip(
+__global__ __launch_bounds__(THREADS, waves_per_simd<S>()) void k_strip(
     const d2q9_lattice L, const d2q9_tiled_desc D, const d2q9_strip_desc P, int K,
     const typename Codec<S>::raw* __restrict__ fsrc, typename Codec<S>::raw* __restrict__ fdst,
     const typename Codec<S>::T* __restrict__ msrc, typename Codec<S>::T* __restrict__ mdst,

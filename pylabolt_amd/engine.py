@@ -403,8 +403,8 @@ class CaseTables:
     def strip_split(self, steps, cols, tile, chunk_rows):
         """Chunks and tiles of the strip sweep (d2q9_strip_steps).
 
-        Strips of ``cols`` columns (the last one moved to end at the last
-        column) are cut along x into chunks of about ``chunk_rows`` rows
+        Strips of ``cols`` columns (the last one of what is left, or the last
+        two sharing it) are cut along x into chunks of about ``chunk_rows`` rows
         whose cells, and the cells within ``steps`` of them, are all plain
         fluid -- or the straight zero-gradient or bounce-back wall of the
         first or last column, of one kind along those rows.  Periodic sides
@@ -424,11 +424,13 @@ class CaseTables:
                            np.where(inl[:, 0] & (side[:, 0] == 2), 2, -1))
         hi_kind = np.where(inl[:, -1] & (side[:, -1] == 1), 1,
                            np.where(inl[:, -1] & (side[:, -1] == 3), 2, -1))
-        starts = list(range(0, ny - cols, cols)) + [ny - cols]
+        starts = list(range(0, ny, cols))
+        if ny - starts[-1] < 2 * steps:
+            starts[-1] -= 2 * steps      # a wall in no strip's margin
         chunks = []
         covered = np.zeros((nx, ny), dtype=bool)
-        for js in starts:
-            c0, c1 = js - steps, js + cols + steps   # region columns
+        for js, je in zip(starts, starts[1:] + [ny]):
+            c0, c1 = js - steps, je + steps   # region columns
             if self.y_periodic:
                 bad = np.take(rough, np.arange(c0, c1) % ny,
                               axis=1).any(axis=1)
@@ -461,9 +463,9 @@ class CaseTables:
                     continue
                 n = max(1, int(round((b - a) / chunk_rows)))
                 cut = [a + (b - a) * q // n for q in range(n + 1)]
-                chunks += [(cut[q] + 1, cut[q + 1] - cut[q], js + 1, cols,
+                chunks += [(cut[q] + 1, cut[q + 1] - cut[q], js + 1, je - js,
                             int(ext[s])) for q in range(n)]
-                covered[a:b, js:js + cols] = True
+                covered[a:b, js:je] = True
         # neighbouring strips of the same rows next to each other
         chunks.sort(key=lambda c: (c[0], c[2]))
         left = ~covered & ((inner & nt.CELL_FLUID) != 0)
@@ -698,6 +700,30 @@ def tiled_shape(sizes, double, forced):
     return best[1:]
 
 
+# cells above which one fused sweep is faster than a tiled launch of one step
+# (us per step: FP32 1024x256 6.6 against 7.4, BF16 4096x1024 34 against 53,
+# FP64 2048x1024 52 against 75; FP64 1001x413 22 against 15, its two kernels
+# and their join)
+_SINGLE_FUSED_CELLS = {8: 1 << 20, 4: 1 << 18}
+# chunks of the strip sweep the GPU holds at once
+_STRIP_SLOTS = {8: 768, 4: 1536}
+# the strip sweep's tiles recompute most of their cells: a lattice with more
+# than this share of its cells in them takes the tiled sweep
+_STRIP_TILE_SHARE = 0.12
+
+
+def strip_rows(nx, strips, double):
+    """Rows of a strip-sweep chunk, or None where the sweep does not pay.
+
+    With r rows for each chunk the GPU holds at once, chunks of r / 2 rows (24
+    to 128) leave little of a last round idle and of a chunk's first rows
+    wasted.  Below r = 20 the tiled sweep wins: us per step FP32 1024x1024 (r
+    = 12) 9.9 tiled, 14.5 strips; 1500x1300 (r = 23) 14.1 and 11.3; FP64
+    1100x1100 (r = 29) 17.9 and 17.2, 8192x2048 215 and 168."""
+    r = nx * strips / _STRIP_SLOTS[8 if double else 4]
+    return None if r < 20 else int(min(128, max(24, r / 2)))
+
+
 def force_tables(nx, ny, groups):
     """Device-ready node and group records for d2q9_momentum_exchange.
 
@@ -761,10 +787,11 @@ class D2Q9Engine:
     ``TWO_STEP_MIN_BYTES`` and it is the faster sweep (``_two_step_wins``;
     the results are bitwise those of single steps), for 16-bit storage only
     when asked (its intermediate step stays in FP32, which changes the
-    rounding).  Otherwise steps go through the tiled sweep
-    (d2q9_tiled_steps, several steps per launch, bitwise single steps in
-    every storage form), or single sweeps where the case cannot be
-    expressed in its tables or a solid moves.
+    rounding).  Otherwise steps go through the strip sweep on large
+    lattices (d2q9_strip_steps) and the tiled sweep on others
+    (d2q9_tiled_steps), several steps per launch and bitwise single steps in
+    every storage form, or through single sweeps where the case cannot be
+    expressed in their tables or a solid moves.
     """
 
     def __init__(self, nx, ny, solid_pad, density, velocity, elements,
@@ -908,6 +935,9 @@ class D2Q9Engine:
         self._init_density = np.asarray(density, dtype=np.float64)
         self._init_velocity = np.asarray(velocity, dtype=np.float64)
         self._setup_tiled()
+        self._setup_strips()
+        self._single_fused = (self.nx * self.ny > _SINGLE_FUSED_CELLS[
+            8 if self.storage == nt.STORE_F64 else 4])
         self.time_step = 0
         self.initialize()
 
@@ -1048,6 +1078,46 @@ class D2Q9Engine:
         self.tiled = D
         self._tiled_p = ctypes.byref(D)
 
+    def _setup_strips(self, rows=None):
+        """Chunks and tiles of the strip sweep, where a lattice with tables
+        for the tiled sweep is large enough (``rows``: of a chunk, whatever
+        the size)."""
+        self.strips = None
+        if self.tiled is None:
+            return
+        shape = [ctypes.c_int32() for _ in range(3)]
+        nt.check(self.lib.d2q9_strip_shape(*[ctypes.byref(v) for v in shape]),
+                 "d2q9_strip_shape")
+        steps, cols, tile = (v.value for v in shape)
+        want = rows or strip_rows(self.nx, -(-self.ny // cols),
+                                  self.storage == nt.STORE_F64)
+        split = (self.tables.strip_split(steps, cols, tile, want)
+                 if want else None)
+        if split is None or (not rows and split[2] > _STRIP_TILE_SHARE):
+            return
+        with torch.cuda.stream(self.stream):
+            self._strip_lists = [torch.from_numpy(a).to(self.device)
+                                 for a in split[:2]]
+        P = nt.StripDesc()
+        P.n_chunks, P.n_tiles = len(split[0]), len(split[1])
+        P.chunks, P.tiles = (t.data_ptr() for t in self._strip_lists)
+        self.strips = P
+        self._strip_p = ctypes.byref(P)
+        self._strip_steps = steps
+
+    def _advance_strips(self, n, write_moments):
+        """``n`` steps through the strip sweep."""
+        a, m = self.i_pop, self.i_mom
+        nt.check(self.lib.d2q9_strip_steps(
+            self._Lp, self._tiled_p, self._strip_p, nt.ptr(self.f[a]),
+            nt.ptr(self.f[1 - a]), nt.ptr(self.mom[m]),
+            nt.ptr(self.mom[1 - m]), n, int(write_moments), 0,
+            self._stream_ptr), "d2q9_strip_steps")
+        flip = -(-n // self._strip_steps) & 1
+        self.i_pop, self.i_mom = a ^ flip, m ^ flip
+        self.mom_full = bool(write_moments)
+        self.time_step += n
+
     def _advance_tiled(self, n, write_moments):
         """``n`` steps through the tiled sweep; the first one collides
         ``pop_new`` where that is in memory."""
@@ -1113,8 +1183,8 @@ class D2Q9Engine:
         """pop = pop_new = feq(rho0, u0) (equilibrium_kernels.py:38-78)."""
         if self.tiled is not None and np.any(
                 self._init_velocity.reshape(-1, 2)[self._tiled_solid]):
-            # the tiled sweep is for solids at rest
-            self.tiled = None
+            # the tiled and strip sweeps are for solids at rest
+            self.tiled = self.strips = None
         with torch.cuda.stream(self.stream):
             m = self._mom_from_host(self._init_density, self._init_velocity)
             self.mom[0].copy_(m)
@@ -1185,7 +1255,7 @@ class D2Q9Engine:
 
     def step(self, write_moments=False):
         """Advance one reference time step."""
-        if self.tiled is not None:
+        if self.tiled is not None and not self._single_fused:
             self._advance_tiled(1, write_moments)
             return
         if self.i_pop_new is not None:
@@ -1210,7 +1280,15 @@ class D2Q9Engine:
         if n <= 0:
             return
         if self.tiled is not None:
-            self._advance_tiled(n, write_moments)
+            if self.strips is not None and self.i_pop_new is not None:
+                self.step(write_moments and n == 1)
+                n -= 1
+            if n == 1:
+                self.step(write_moments)
+            elif n > 1 and self.strips is not None:
+                self._advance_strips(n, write_moments)
+            elif n > 1:
+                self._advance_tiled(n, write_moments)
             return
         if self.i_pop_new is not None:
             self.step(write_moments and n == 1)

@@ -8,7 +8,8 @@ from oracle import d2q9_oracle as O
 from pylabolt_amd import _native as nt
 from pylabolt_amd import cases
 from pylabolt_amd.engine import (CX, CY, INV, CaseTables,
-                                 elements_from_boundary, tiled_shape)
+                                 elements_from_boundary, strip_rows,
+                                 tiled_shape)
 from pylabolt_amd.base.state import State
 from tests.helpers import oracle_case
 
@@ -145,3 +146,59 @@ def test_tiled_shape_fits_a_workgroup(nx, ny, double, forced):
     rows, width, steps = tiled_shape(((nx, ny),), double, forced)
     assert width in (16, 32, 64) and rows * width <= 1024
     assert steps >= 1 and rows > 2 * steps and width > 2 * steps
+
+
+STRIP_CASES = {
+    "channel": lambda: cases.poiseuille_channel(60, 64),
+    "channel_wide": lambda: cases.poiseuille_channel(40, 233),
+    "cylinder": lambda: cases.cylinder(150, 200, diameter=20),
+    "cavity": lambda: cases.lid_driven_cavity(70, 121),
+    "box": lambda: _box(45, 119),
+    "box_edge": lambda: _box(60, 130, (0.0, 0.0)),
+}
+
+
+@pytest.mark.parametrize("rows", [8, 24, 1000])
+@pytest.mark.parametrize("name", STRIP_CASES)
+def test_strip_split_covers_with_plain_chunks(name, rows):
+    """Every fluid cell is in a chunk or a tile; every cell within 4 of a
+    chunk is plain fluid or the stated wall."""
+    sim = STRIP_CASES[name]()
+    st = State(sim)
+    nx, ny = int(st.domain.Nx_rank), int(st.domain.Ny_rank)
+    t = CaseTables(nx, ny, st.fields.solid, elements_from_boundary(st.boundary),
+                   st.boundary.x_periodic, st.boundary.y_periodic, 64, 4)
+    chunks, tiles, share = t.strip_split(4, 56, 8, rows)
+    assert share == tiles.shape[0] * 64 / (nx * ny)
+    inner = t.flags_pad[1:-1, 1:-1]
+    side = t.wall_side_pad[1:-1, 1:-1]
+    seen = np.zeros((nx, ny), dtype=bool)
+    for i, n, j, cols, walls in chunks:
+        assert 1 <= i and i + n - 1 <= nx and 1 <= j and j + cols - 1 <= ny
+        assert 8 <= cols <= 56 and n >= 1
+        lo, hi = walls & 3, walls >> 2
+        seen[i - 1:i - 1 + n, j - 1:j - 1 + cols] = True
+        for r in range(i - 5, i + n + 3):
+            if not t.x_periodic:
+                assert 0 <= r < nx
+            for c in range(j - 5, j + cols + 3):
+                if not t.y_periodic and not 0 <= c < ny:
+                    assert (lo and j == 1) if c < 0 else (
+                        hi and j + cols - 1 == ny)
+                    continue
+                f = inner[r % nx, c % ny]
+                if f == nt.CELL_FLUID:
+                    continue
+                assert f == nt.CELL_FLUID | nt.CELL_BC
+                s = side[r % nx, c]
+                assert (c == 0 and s == {1: 0, 2: 2}[lo]) or (
+                    c == ny - 1 and s == {1: 1, 2: 3}[hi])
+    for i, j in tiles:
+        seen[i - 1:i + 7, j - 1:j + 7] = True
+    assert seen[t.fluid_pad[1:-1, 1:-1]].all()
+
+
+def test_strip_rows_rule():
+    assert strip_rows(1024, 19, False) is None
+    assert strip_rows(8192, 37, True) == 128
+    assert strip_rows(1500, 24, False) == 24

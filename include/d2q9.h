@@ -275,7 +275,9 @@ int d2q9_deep_rows(void);
  * population), of boundary element bits 16..23, or of element bits 24..31
  * when bit 7 + d is set too; has_vel and has_pres: some such element is of
  * type D2Q9_RULE_VEL, D2Q9_RULE_PRES.  n_elems (at most 32) boundary
- * elements are in bc_elems.  The solids must be at rest.
+ * elements are in bc_elems.  The solids must be at rest.  round_last: 16-bit
+ * storage rounds only the last step of a launch and keeps the others in FP32
+ * (not bitwise single steps any more: fewer roundings).
  *
  * The steps go f_a -> f_b -> f_a ... once per launch, ceil(n / steps)
  * launches (the last one's target holds the result), the moments alike.
@@ -287,6 +289,7 @@ int d2q9_deep_rows(void);
 typedef struct d2q9_tiled_desc {
   int32_t rows, width, steps;
   int32_t n_elems, has_vel, has_pres;
+  int32_t round_last;
   const uint32_t* cells;
   const uint32_t* codes;
 } d2q9_tiled_desc;
@@ -415,10 +418,9 @@ int d2q9_batched_step(const d2q9_batch_entry* entries,
 
 /*
  * Strip sweep: n fused steps, up to 4 per launch, as d2q9_tiled_steps (bitwise
- * single steps; with round_last, 16-bit storage rounds only the last step of
- * a launch, which keeps the others in FP32).  d2q9_strip_shape gives the most
- * steps of a launch, a strip's output columns and a tile's output rows and
- * columns.
+ * single steps unless D asks for round_last).  d2q9_strip_shape gives the
+ * most steps of a launch, a strip's output columns and a tile's output rows
+ * and columns.
  *
  * chunks: `cols` (at most a strip's) columns from j_first on by `rows` rows
  * from i_first on.  Every cell of a chunk and within `steps` cells of it is
@@ -448,8 +450,7 @@ typedef struct d2q9_strip_desc {
 int d2q9_strip_shape(int32_t* steps, int32_t* cols, int32_t* tile);
 int d2q9_strip_steps(const d2q9_lattice* L, const d2q9_tiled_desc* D,
                      const d2q9_strip_desc* P, void* f_a, void* f_b, void* mom_a,
-                     void* mom_b, int32_t n, int write_moments, int round_last,
-                     void* stream);
+                     void* mom_b, int32_t n, int write_moments, void* stream);
 
 /*
  * Batched tiled sweep: n fused steps of many lattices of one storage type

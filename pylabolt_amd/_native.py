@@ -102,6 +102,7 @@ class TiledDesc(ctypes.Structure):
     _fields_ = [("rows", ctypes.c_int32), ("width", ctypes.c_int32),
                 ("steps", ctypes.c_int32), ("n_elems", ctypes.c_int32),
                 ("has_vel", ctypes.c_int32), ("has_pres", ctypes.c_int32),
+                ("round_last", ctypes.c_int32),
                 ("cells", ctypes.c_void_p), ("codes", ctypes.c_void_p)]
 
 
@@ -120,7 +121,7 @@ class StripDesc(ctypes.Structure):
 # boundary elements a launch of the tiled sweep holds (d2q9_tiled_desc)
 TILED_MAX_ELEMS = 32
 
-assert ctypes.sizeof(TiledDesc) == 40
+assert ctypes.sizeof(TiledDesc) == 48
 assert ctypes.sizeof(BcElem) == 40 and ctypes.sizeof(BcNode) == 20
 
 _P = ctypes.c_void_p
@@ -164,7 +165,7 @@ SIGNATURES = {
     "d2q9_strip_steps": (ctypes.c_int, [_LP, ctypes.POINTER(TiledDesc),
                                         ctypes.POINTER(StripDesc), _P, _P, _P,
                                         _P, ctypes.c_int32, ctypes.c_int,
-                                        ctypes.c_int, _P]),
+                                        _P]),
     "d2q9_tiled_batch": (ctypes.c_int, [_P, _P] + [ctypes.c_int] * 10 + [_P]),
     "d2q9_momentum_exchange": (ctypes.c_int, [_LP, _P, _P, _P, _P,
                                               ctypes.c_int64, _P, ctypes.c_int,

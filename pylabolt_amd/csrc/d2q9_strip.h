@@ -52,7 +52,7 @@ template <int S, int MODEL, int FORCING>
 __device__ __forceinline__ void run_strip(
     const d2q9_lattice& L, char* __restrict__ smem, const d2q9_strip_chunk ch, int K,
     const typename Codec<S>::raw* __restrict__ fsrc, typename Codec<S>::raw* __restrict__ fdst,
-    typename Codec<S>::T* __restrict__ mdst, int write_mom, int round_last) {
+    typename Codec<S>::T* __restrict__ mdst, int write_mom, bool round_last) {
   using C = Codec<S>;
   using T = typename C::T;
   using R = typename C::raw;
@@ -227,7 +227,7 @@ __global__ __launch_bounds__(THREADS, waves_per_simd<S>()) void k_strip(
     const d2q9_lattice L, const d2q9_tiled_desc D, const d2q9_strip_desc P, int K,
     const typename Codec<S>::raw* __restrict__ fsrc, typename Codec<S>::raw* __restrict__ fdst,
     const typename Codec<S>::T* __restrict__ msrc, typename Codec<S>::T* __restrict__ mdst,
-    int write_mom, int round_last) {
+    int write_mom) {
   extern __shared__ __align__(16) char smem[];
   const int b = (int)blockIdx.x;
   if (b < P.n_tiles) {
@@ -238,11 +238,11 @@ __global__ __launch_bounds__(THREADS, waves_per_simd<S>()) void k_strip(
     return;
   }
   run_strip<S, MODEL, FORCING>(L, smem, P.chunks[xcd_remap(b - P.n_tiles, P.n_chunks)], K, fsrc,
-                               fdst, mdst, write_mom, round_last);
+                               fdst, mdst, write_mom, D.round_last != 0);
 }
 
 struct Launch {
-  int K, write_mom, round_last;
+  int K, write_mom;
   const void* fsrc;
   void* fdst;
   const void* msrc;
@@ -268,7 +268,7 @@ hipError_t launch_one(const d2q9_lattice* L, const d2q9_tiled_desc* D, const d2q
                      A.stream, *L, *D, *P, A.K, static_cast<const typename C::raw*>(A.fsrc),
                      static_cast<typename C::raw*>(A.fdst),
                      static_cast<const typename C::T*>(A.msrc),
-                     static_cast<typename C::T*>(A.mdst), A.write_mom, A.round_last);
+                     static_cast<typename C::T*>(A.mdst), A.write_mom);
   return hipGetLastError();
 }
 

@@ -25,7 +25,7 @@ extern "C" int d2q9_strip_shape(int32_t* steps, int32_t* cols, int32_t* tile) {
 
 extern "C" int d2q9_strip_steps(const d2q9_lattice* L, const d2q9_tiled_desc* D,
                                 const d2q9_strip_desc* P, void* f_a, void* f_b, void* mom_a,
-                                void* mom_b, int32_t n, int write_moments, int round_last,
+                                void* mom_b, int32_t n, int write_moments,
                                 void* stream) {
   if (int r = validate_lattice(L)) return r;
   if (!D || !P || !f_a || !f_b || !mom_a || !mom_b)
@@ -43,7 +43,6 @@ extern "C" int d2q9_strip_steps(const d2q9_lattice* L, const d2q9_tiled_desc* D,
   void* m[2] = {mom_a, mom_b};
   strip::Launch A;
   A.stream = static_cast<hipStream_t>(stream);
-  A.round_last = round_last;
   for (int a = 0; a < launches; ++a) {
     A.K = base + (a < longer ? 1 : 0);
     A.write_mom = a == launches - 1 && write_moments;

@@ -16,8 +16,9 @@
 // special cell), and only moving walls and fixed-pressure nodes add
 // arithmetic of their own, in the order of apply_bc.  Periodic sides are
 // images in the grown region.  The arithmetic per cell is that of the
-// single step and 16-bit storage rounds every step, so the result is bitwise
-// that of K single steps in every storage form.
+// single step and 16-bit storage rounds every step (the last of a launch
+// only, when asked), so the result is bitwise that of K single steps in every
+// storage form.
 //
 // What bounds it: for small lattices the latency of a launch (about 4 us
 // of load, collide, store and hand-over) which the K steps share; for larger
@@ -165,6 +166,7 @@ __device__ __forceinline__ void run_tile(
   uint32_t from[4] = {};    // special cells: LDS elements to read, two a word
   uint32_t arith = 0;       // special cells: directions with arithmetic
   T ffx = (T)0, ffy = (T)0;
+  const bool each = sizeof(R) == 2 && !D.round_last;   // every step is rounded
   {
     const int r = e / W, c = e % W;
     int i = i0 + r, j = j0 + c;
@@ -263,7 +265,7 @@ __device__ __forceinline__ void run_tile(
     const uint32_t key = sizeof(R) == 2 ? cell_key((uint32_t)cell) : 0u;
     if (st < K) {
 #pragma unroll
-      for (int k = 0; k < 9; ++k) s[e * 9 + k] = through_storage<S>(g[k], k, key, Kc);
+      for (int k = 0; k < 9; ++k) s[e * 9 + k] = each ? through_storage<S>(g[k], k, key, Kc) : g[k];
       if (keep) {
         if (D.has_vel) srho[e] = rho;
         if (D.has_pres) {

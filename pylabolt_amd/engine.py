@@ -786,8 +786,9 @@ class D2Q9Engine:
     and FP32 storage when the two population buffers exceed
     ``TWO_STEP_MIN_BYTES`` and it is the faster sweep (``_two_step_wins``;
     the results are bitwise those of single steps), for 16-bit storage only
-    when asked (its intermediate step stays in FP32, which changes the
-    rounding).  Otherwise steps go through the strip sweep on large
+    when asked (it then rounds the stored step of a launch only, which
+    changes the numerics; where the two-step sweep would need a rim, the
+    strip or tiled sweep runs that way instead).  Otherwise steps go through the strip sweep on large
     lattices (d2q9_strip_steps) and the tiled sweep on others
     (d2q9_tiled_steps), several steps per launch and bitwise single steps in
     every storage form, or through single sweeps where the case cannot be
@@ -930,6 +931,14 @@ class D2Q9Engine:
                         2 * self.f[0].numel() * self.f[0].element_size()
                         > TWO_STEP_MIN_BYTES and self._two_step_wins())
         self._two_step_req = bool(two_step)
+        # 16-bit storage asked to round fewer steps, where a rim would slow
+        # the two-step sweep: us per step two-step against strips or tiles
+        # that round the last step of a launch, FP16 8192x2048 90 / 66, BF16
+        # 3790x1973 48 / 33, 900x700 14.3 / 6.8 (without a rim BF16
+        # 2048x1024 13.8 / 16.5)
+        self._round_last = (self._two_step_req and
+                            self.raw_dtype.itemsize == 2 and
+                            self._codes is not None and not self._rimless())
         self.two_step = False
         self._setup_two_step()
         self._init_density = np.asarray(density, dtype=np.float64)
@@ -978,6 +987,11 @@ class D2Q9Engine:
         d = self.tables.deep_split(int(self.lib.d2q9_deep_rows()))
         if d.n_deep == 0:
             return
+        self.n_deep = d.n_deep
+        self.deep_fraction = float(d.covered.mean())
+        if self._round_last:
+            self.two_step = True
+            return
         dev = self.device
         with torch.cuda.stream(self.stream):
             self._deep = {
@@ -1020,20 +1034,26 @@ class D2Q9Engine:
         self._rim_a, self._rim_b = rims
         self._rim_ap = ctypes.byref(self._rim_a)
         self._rim_bp = ctypes.byref(self._rim_b)
-        self.n_deep = d.n_deep
-        self.deep_fraction = float(d.covered.mean())
         self.two_step = True
         # a graph replays an even number of two-step sweeps, so the buffers
         # return to their roles
         self.graph_steps = max(4, self.graph_steps // 4 * 4)
 
+    def _rimless(self):
+        """Whether deep tiles of the two-step sweep cover the lattice: a
+        channel periodic in x with straight walls at y, whole blocks and
+        tile heights."""
+        t = self.tables
+        plain = not (t.flags_pad & nt.CELL_NEAR_SOLID).any()
+        return bool(plain and t.x_periodic and not t.y_periodic and
+                    self.nx % self.tile_i == 0 and self.ny % self.B == 0 and
+                    t.wall_inline_wrap[:, [0, -1]].all())
+
     def _two_step_wins(self):
         """Whether the two-step sweep is the faster one for a lattice of
         more than TWO_STEP_MIN_BYTES.
 
-        It is where it has no rim (a channel periodic in x with straight
-        walls at y, whole blocks and tile heights: us per step against the
-        tiled sweep's, FP32 2048x1024 16.3 / 18.2, FP64 1024x1024 19.6 /
+        It is where it has no rim (us per step against the tiled sweep's, FP32 2048x1024 16.3 / 18.2, FP64 1024x1024 19.6 /
         23.8, 4096x1024 67 / 80) and for forced FP64 at large sizes, whose
         tiled kernel is short of registers.  Elsewhere the rim's kernels and
         its fork and join cost more than the tiled sweep's repeated cells:
@@ -1044,11 +1064,7 @@ class D2Q9Engine:
         if (self.storage == nt.STORE_F64 and self.forcing is not None and
                 self.nx * self.ny > 1 << 20):
             return True
-        t = self.tables
-        plain = not (t.flags_pad & nt.CELL_NEAR_SOLID).any()
-        return bool(plain and t.x_periodic and not t.y_periodic and
-                    self.nx % self.tile_i == 0 and self.ny % self.B == 0 and
-                    t.wall_inline_wrap[:, [0, -1]].all())
+        return self._rimless()
 
     def _setup_tiled(self):
         """Tables of the tiled sweep on the device, where the lattice takes
@@ -1057,7 +1073,7 @@ class D2Q9Engine:
         self._tiled_arrays = None
         t, tables = self.tables, self._codes
         self._codes = None
-        if self.two_step or tables is None:
+        if tables is None or (self.two_step and not self._round_last):
             return
         cells, codes, has_vel, has_pres = tables
         rows, width, steps = tiled_shape(
@@ -1071,6 +1087,7 @@ class D2Q9Engine:
         D.rows, D.width, D.steps = rows, width, steps
         D.n_elems = len(t.elems)
         D.has_vel, D.has_pres = int(has_vel), int(has_pres)
+        D.round_last = int(self.two_step)
         D.cells, D.codes = dev["cells"].data_ptr(), dev["codes"].data_ptr()
         self._tiled_arrays = dev
         self._tiled_solid = np.flatnonzero(
@@ -1111,7 +1128,7 @@ class D2Q9Engine:
         nt.check(self.lib.d2q9_strip_steps(
             self._Lp, self._tiled_p, self._strip_p, nt.ptr(self.f[a]),
             nt.ptr(self.f[1 - a]), nt.ptr(self.mom[m]),
-            nt.ptr(self.mom[1 - m]), n, int(write_moments), 0,
+            nt.ptr(self.mom[1 - m]), n, int(write_moments),
             self._stream_ptr), "d2q9_strip_steps")
         flip = -(-n // self._strip_steps) & 1
         self.i_pop, self.i_mom = a ^ flip, m ^ flip
@@ -1148,6 +1165,8 @@ class D2Q9Engine:
         self._upload_tiles()
         if self.two_step:
             self._setup_two_step()
+        if self.tiled is not None:
+            self.tiled.round_last = int(self.two_step)
 
     # ---- layout helpers -------------------------------------------------
     def _upload_plane(self, pad, dtype, count=1):
@@ -1185,6 +1204,9 @@ class D2Q9Engine:
                 self._init_velocity.reshape(-1, 2)[self._tiled_solid]):
             # the tiled and strip sweeps are for solids at rest
             self.tiled = self.strips = None
+            if self._round_last:
+                self._round_last = False
+                self._setup_two_step()
         with torch.cuda.stream(self.stream):
             m = self._mom_from_host(self._init_density, self._init_velocity)
             self.mom[0].copy_(m)
@@ -1241,6 +1263,9 @@ class D2Q9Engine:
 
     def step2(self, write_moments=False):
         """Advance two reference time steps with the two-step sweep."""
+        if self.tiled is not None:
+            self.advance(2, write_moments)
+            return
         if self.i_pop_new is not None:
             self.step()
             self.step(write_moments)

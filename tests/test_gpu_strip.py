@@ -2,8 +2,10 @@
 edges of strips, chunks and launches."""
 import numpy as np
 import pytest
+import torch
 
 from pylabolt_amd import cases
+from pylabolt_amd.engine import pop_aos
 from pylabolt_amd.solvers.fluidLB import Solver
 from tests.test_host_tiled import STRIP_CASES, _box
 
@@ -92,3 +94,72 @@ def test_large_lattices_take_the_strips():
         s.advance(n)
         ref.advance(n)
         assert np.array_equal(s.engine.pop(), ref.engine.pop())
+
+
+@pytest.mark.parametrize("storage", ["f16dev", "bf16dev"])
+@pytest.mark.parametrize("strips", [False, True])
+@pytest.mark.parametrize("name", list(STRIP_CASES))
+def test_round_last_is_the_float_sweep(name, strips, storage):
+    """A launch that rounds only its last step gives the moments of FP32
+    storage from the same state bit for bit, and its populations to one unit
+    of the 16-bit form's last place (FP16: 2^-10 of the deviation, BF16:
+    2^-7, and FP16's smallest number)."""
+    one = []
+    for st in (storage, "f32"):
+        e = _pair(STRIP_CASES[name], st, 24)[0]
+        if not strips:
+            e.strips = None
+        e.advance(1)
+        one.append(e)
+    a, b = one
+    a.tiled.round_last = 1
+    fluid = a.tables.fluid_pad.ravel()
+    w = np.asarray(a.weights)
+    # the whole state, cells outside the fluid too: a cell may pull from them
+    scale = np.array([a.L.dev_scale[k] for k in range(9)])
+    a.stream.synchronize()
+    with torch.cuda.stream(b.stream):
+        buf, nx, ny, B, nbj = b.f[b.i_pop], b.nx, b.ny, b.B, b.nbj
+        aos = pop_aos(a.f[a.i_pop], nx, ny, B, nbj).float() / torch.tensor(
+            scale, dtype=torch.float32, device=b.device)
+        rows = buf.reshape(nx + 2, nbj, 9, B).permute(0, 2, 1, 3).reshape(
+            nx + 2, 9, nbj * B).clone()
+        rows[:, :, B - 1:B - 1 + ny + 2] = aos.reshape(
+            nx + 2, ny + 2, 9).permute(0, 2, 1)
+        buf.copy_(rows.reshape(nx + 2, 9, nbj, B).permute(0, 2, 1, 3).reshape(
+            -1))
+        b.mom[b.i_mom].copy_(a.mom[a.i_mom])
+    b.stream.synchronize()
+    n = 4 if strips else a.tiled.steps
+    a.advance(n)
+    b.advance(n)
+    for x, y in zip(a.moments_host(), b.moments_host()):
+        assert np.array_equal(x[fluid], y[fluid])
+    x, y = a.pop()[fluid], b.pop()[fluid]
+    bits, least = (10, 2.0 ** -24) if storage == "f16dev" else (7, 2.0 ** -120)
+    lim = np.abs(y - w) * 2.0 ** -bits + least / scale + 1e-16
+    assert (np.abs(x - y) <= lim).all()
+
+
+def test_two_step_request_in_16_bits():
+    """A 16-bit lattice asked for the two-step sweep rounds the last step of
+    a launch: by strips or tiles where that sweep has a rim, and through it
+    where it has none; other storage forms keep it."""
+    def engine(sim, storage):
+        s = Solver(simulation=sim, storage=storage, verbose=False,
+                   two_step=True)
+        s.set_backend()
+        assert s.engine.two_step
+        return s.engine
+    e = engine(cases.cylinder(400, 300, diameter=30), "bf16dev")
+    assert e.tiled.round_last == 1 and e.strips is None
+    e.step2(True)
+    assert e.time_step == 2 and e.moments_host()[0].size
+    e.set_tile_rows(2)
+    assert e.tiled.round_last == int(e.two_step)
+    assert engine(cases.lid_driven_cavity(1500, 1300),
+                  "f16dev").strips is not None
+    for sim, storage in ((cases.poiseuille_channel(512, 256), "f16dev"),
+                         (cases.cylinder(400, 300, diameter=30), "f32")):
+        e = engine(sim, storage)
+        assert e.tiled is None and e._deep is not None

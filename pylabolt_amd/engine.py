@@ -405,7 +405,8 @@ class CaseTables:
 
         Strips of ``cols`` columns (the last one of what is left, or the last
         two sharing it) are cut along x into chunks of about ``chunk_rows`` rows
-        whose cells, and the cells within ``steps`` of them, are all plain
+        (or what that function of the lengths of all runs of rows gives; None:
+        no split) whose cells, and the cells within ``steps`` of them, are all plain
         fluid -- or the straight zero-gradient or bounce-back wall of the
         first or last column, of one kind along those rows.  Periodic sides
         count as their images.  Every fluid cell in no chunk lies in a tile of
@@ -427,7 +428,7 @@ class CaseTables:
         starts = list(range(0, ny, cols))
         if ny - starts[-1] < 2 * steps:
             starts[-1] -= 2 * steps      # a wall in no strip's margin
-        chunks = []
+        runs = []
         covered = np.zeros((nx, ny), dtype=bool)
         for js, je in zip(starts, starts[1:] + [ny]):
             c0, c1 = js - steps, je + steps   # region columns
@@ -461,11 +462,18 @@ class CaseTables:
                 b = min(e - steps - off, nx)
                 if b - a < 2 * tile:
                     continue
-                n = max(1, int(round((b - a) / chunk_rows)))
-                cut = [a + (b - a) * q // n for q in range(n + 1)]
-                chunks += [(cut[q] + 1, cut[q + 1] - cut[q], js + 1, je - js,
-                            int(ext[s])) for q in range(n)]
+                runs.append((a, b, js, je, int(ext[s])))
                 covered[a:b, js:je] = True
+        if callable(chunk_rows):
+            chunk_rows = chunk_rows(np.array([b - a for a, b, *_ in runs]))
+            if chunk_rows is None:
+                return None
+        chunks = []
+        for a, b, js, je, walls in runs:
+            n = max(1, int(round((b - a) / chunk_rows)))
+            cut = [a + (b - a) * q // n for q in range(n + 1)]
+            chunks += [(cut[q] + 1, cut[q + 1] - cut[q], js + 1, je - js,
+                        walls) for q in range(n)]
         # neighbouring strips of the same rows next to each other
         chunks.sort(key=lambda c: (c[0], c[2]))
         left = ~covered & ((inner & nt.CELL_FLUID) != 0)
@@ -712,16 +720,34 @@ _STRIP_SLOTS = {8: 768, 4: 1536}
 _STRIP_TILE_SHARE = 0.12
 
 
-def strip_rows(nx, strips, double):
-    """Rows of a strip-sweep chunk, or None where the sweep does not pay.
+def strip_rows(lengths, double, rounds=False):
+    """Rows of a strip-sweep chunk for runs of ``lengths`` rows, or None where
+    the sweep does not pay.
 
-    With r rows for each chunk the GPU holds at once, chunks of r / 2 rows (24
-    to 128) leave little of a last round idle and of a chunk's first rows
-    wasted.  Below r = 20 the tiled sweep wins: us per step FP32 1024x1024 (r
-    = 12) 9.9 tiled, 14.5 strips; 1500x1300 (r = 23) 14.1 and 11.3; FP64
-    1100x1100 (r = 29) 17.9 and 17.2, 8192x2048 215 and 168."""
-    r = nx * strips / _STRIP_SLOTS[8 if double else 4]
-    return None if r < 20 else int(min(128, max(24, r / 2)))
+    A chunk takes its rows and about 8 to fill and drain its waves.  A round
+    of chunks that only partly fills the GPU takes as long as its latency,
+    0.45 of a full round, and 0.75 of that where the rounds before it overlap
+    it.  Over 15 lattices of 0.5 to 17 M cells and chunks of 12 to 160 rows
+    this picks within 1 % of the best on average, 6 % on one (FP32 2048x1024
+    forced: 26 rows 14.3 us per step, 24 rows, just over a round, 17.3).
+
+    Below 9 rows (FP64 12) for each chunk the GPU holds at once the tiled
+    sweep is as fast (us per step strips / tiled: FP32 900x900 7.0 / 7.7, FP64
+    700x700 9.6 / 9.7, 1024x1024 14.4 / 16.7), below 20 with ``rounds``, 16-bit storage
+    that rounds every step (BF16 1100x1100 11.5 / 11.1, 1300x1300 13.5 /
+    14.8)."""
+    if lengths.size == 0:
+        return None
+    slots = _STRIP_SLOTS[8 if double else 4]
+    if lengths.sum() < slots * (20 if rounds else 12 if double else 9):
+        return None
+    rows = np.arange(8, 161)
+    n = np.maximum(1, np.rint(lengths[:, None] / rows))
+    longest = np.ceil(lengths[:, None] / n).max(axis=0)
+    full, last = np.divmod(n.sum(axis=0), slots)
+    part = np.where(full > 0, 0.75, 1.0) * (0.45 + 0.55 * last / slots)
+    cost = (longest + 8) * (full + np.where(last > 0, part, 0.0))
+    return int(rows[np.argmin(cost)])
 
 
 def force_tables(nx, ny, groups):
@@ -784,11 +810,11 @@ class D2Q9Engine:
     ``two_step`` advances pairs of steps with one sweep over the deep
     interior (d2q9_fused_step2) when deep tiles fit; by default for FP64
     and FP32 storage when the two population buffers exceed
-    ``TWO_STEP_MIN_BYTES`` and it is the faster sweep (``_two_step_wins``;
-    the results are bitwise those of single steps), for 16-bit storage only
-    when asked (it then rounds the stored step of a launch only, which
-    changes the numerics; where the two-step sweep would need a rim, the
-    strip or tiled sweep runs that way instead).  Otherwise steps go through the strip sweep on large
+    ``TWO_STEP_MIN_BYTES`` and they cover the lattice (the results are
+    bitwise those of single steps), for 16-bit storage only when asked (it
+    then rounds the stored step of a launch only, which changes the
+    numerics).  Where the strip or tiled sweep is the faster one it runs
+    instead, to the same rounding (``_choose_sweep``).  Otherwise steps go through the strip sweep on large
     lattices (d2q9_strip_steps) and the tiled sweep on others
     (d2q9_tiled_steps), several steps per launch and bitwise single steps in
     every storage form, or through single sweeps where the case cannot be
@@ -929,16 +955,10 @@ class D2Q9Engine:
             # may do
             two_step = (self.storage in (nt.STORE_F64, nt.STORE_F32) and
                         2 * self.f[0].numel() * self.f[0].element_size()
-                        > TWO_STEP_MIN_BYTES and self._two_step_wins())
+                        > TWO_STEP_MIN_BYTES and
+                        (self._codes is None or self._rimless()))
         self._two_step_req = bool(two_step)
-        # 16-bit storage asked to round fewer steps, where a rim would slow
-        # the two-step sweep: us per step two-step against strips or tiles
-        # that round the last step of a launch, FP16 8192x2048 90 / 66, BF16
-        # 3790x1973 48 / 33, 900x700 14.3 / 6.8 (without a rim BF16
-        # 2048x1024 13.8 / 16.5)
-        self._round_last = (self._two_step_req and
-                            self.raw_dtype.itemsize == 2 and
-                            self._codes is not None and not self._rimless())
+        self._choose_sweep()
         self.two_step = False
         self._setup_two_step()
         self._init_density = np.asarray(density, dtype=np.float64)
@@ -989,7 +1009,7 @@ class D2Q9Engine:
             return
         self.n_deep = d.n_deep
         self.deep_fraction = float(d.covered.mean())
-        if self._round_last:
+        if self._several:
             self.two_step = True
             return
         dev = self.device
@@ -1049,22 +1069,41 @@ class D2Q9Engine:
                     self.nx % self.tile_i == 0 and self.ny % self.B == 0 and
                     t.wall_inline_wrap[:, [0, -1]].all())
 
-    def _two_step_wins(self):
-        """Whether the two-step sweep is the faster one for a lattice of
-        more than TWO_STEP_MIN_BYTES.
+    def _choose_sweep(self):
+        """``_split``: the strip sweep's chunks and tiles, where it pays;
+        ``_several``: the strip or tiled sweep runs even where two steps per
+        sweep were asked for; ``_round_last``: it then rounds 16-bit values
+        at the last step of a launch only.
 
-        It is where it has no rim (us per step against the tiled sweep's, FP32 2048x1024 16.3 / 18.2, FP64 1024x1024 19.6 /
-        23.8, 4096x1024 67 / 80) and for forced FP64 at large sizes, whose
-        tiled kernel is short of registers.  Elsewhere the rim's kernels and
-        its fork and join cost more than the tiled sweep's repeated cells:
-        FP64 cylinder 1001x413 7.4 us tiled, 25 two-step, 8192x2048 220 /
-        235; FP32 cylinder 2999x1111 22.6 / 34, 8192x2048 112 / 122."""
-        if self._codes is None:
-            return True
-        if (self.storage == nt.STORE_F64 and self.forcing is not None and
-                self.nx * self.ny > 1 << 20):
-            return True
-        return self._rimless()
+        The two-step sweep keeps small lattices that ask for it (by
+        default none) and, of those without a rim, 16-bit ones and MRT in
+        FP64 below 8 M cells: us per step against the strips', FP16
+        4096x1024 27.6 / 29.8, BF16 2048x1024 13.4 / 14.1, FP64 MRT 2048x1024
+        34 / 39, 4096x1024 63 / 69, 8192x2048 240 / 223, but BGK 4096x1024 65
+        / 63 and FP32 4096x1024 36 / 30.  With a rim its kernels, fork and
+        join cost more: FP64 1371x1362 forced 36 / 28, 3001x1333 75 / 66,
+        FP16 8192x2048 90 / 73, BF16 900x700 14.3 / 6.1 (tiled)."""
+        self._split = None
+        if self._codes is not None:
+            shape = [ctypes.c_int32() for _ in range(3)]
+            nt.check(self.lib.d2q9_strip_shape(
+                *[ctypes.byref(v) for v in shape]), "d2q9_strip_shape")
+            self._strip_shape = tuple(v.value for v in shape)
+            bits = 8 * self.raw_dtype.itemsize
+            split = self.tables.strip_split(
+                *self._strip_shape, functools.partial(
+                    strip_rows, double=bits == 64,
+                    rounds=bits == 16 and not self._two_step_req))
+            if split is not None and split[2] <= _STRIP_TILE_SHARE:
+                self._split = split
+        half = self.raw_dtype.itemsize == 2
+        rimless = self._rimless()
+        keep = rimless and self.nx * self.ny < 1 << 23 and (
+            half or (self.storage == nt.STORE_F64 and self.model == "MRT"))
+        self._several = not self._two_step_req or (
+            self._codes is not None and not keep and
+            (self._split is not None or (half and not rimless)))
+        self._round_last = half and self._two_step_req and self._several
 
     def _setup_tiled(self):
         """Tables of the tiled sweep on the device, where the lattice takes
@@ -1073,7 +1112,7 @@ class D2Q9Engine:
         self._tiled_arrays = None
         t, tables = self.tables, self._codes
         self._codes = None
-        if tables is None or (self.two_step and not self._round_last):
+        if tables is None or (self.two_step and not self._several):
             return
         cells, codes, has_vel, has_pres = tables
         rows, width, steps = tiled_shape(
@@ -1087,7 +1126,7 @@ class D2Q9Engine:
         D.rows, D.width, D.steps = rows, width, steps
         D.n_elems = len(t.elems)
         D.has_vel, D.has_pres = int(has_vel), int(has_pres)
-        D.round_last = int(self.two_step)
+        D.round_last = int(self._round_last and self.two_step)
         D.cells, D.codes = dev["cells"].data_ptr(), dev["codes"].data_ptr()
         self._tiled_arrays = dev
         self._tiled_solid = np.flatnonzero(
@@ -1096,21 +1135,14 @@ class D2Q9Engine:
         self._tiled_p = ctypes.byref(D)
 
     def _setup_strips(self, rows=None):
-        """Chunks and tiles of the strip sweep, where a lattice with tables
-        for the tiled sweep is large enough (``rows``: of a chunk, whatever
+        """Lists of the strip sweep on the device, where a lattice with
+        tables for the tiled sweep takes it (``rows``: of a chunk, whatever
         the size)."""
         self.strips = None
-        if self.tiled is None:
-            return
-        shape = [ctypes.c_int32() for _ in range(3)]
-        nt.check(self.lib.d2q9_strip_shape(*[ctypes.byref(v) for v in shape]),
-                 "d2q9_strip_shape")
-        steps, cols, tile = (v.value for v in shape)
-        want = rows or strip_rows(self.nx, -(-self.ny // cols),
-                                  self.storage == nt.STORE_F64)
-        split = (self.tables.strip_split(steps, cols, tile, want)
-                 if want else None)
-        if split is None or (not rows and split[2] > _STRIP_TILE_SHARE):
+        split = self._split
+        if rows is not None:
+            split = self.tables.strip_split(*self._strip_shape, rows)
+        if self.tiled is None or split is None:
             return
         with torch.cuda.stream(self.stream):
             self._strip_lists = [torch.from_numpy(a).to(self.device)
@@ -1120,10 +1152,29 @@ class D2Q9Engine:
         P.chunks, P.tiles = (t.data_ptr() for t in self._strip_lists)
         self.strips = P
         self._strip_p = ctypes.byref(P)
-        self._strip_steps = steps
+        self._strip_steps = self._strip_shape[0]
 
     def _advance_strips(self, n, write_moments):
-        """``n`` steps through the strip sweep."""
+        """``n`` steps through the strip sweep.
+
+        A launch of 2 or 3 steps costs nearly as much as one of 4 (FP32
+        8192x2048: 380, 390 and 405 us), so one step left over goes through
+        step() (220 us).  Where 16-bit storage rounds every step the sweep is
+        bound by its arithmetic and the single sweep is relatively cheap:
+        two left over are single steps too (BF16 8192x2048: 110 us each, 240
+        to 370 a launch of 2), with a force three (112 each, 390)."""
+        tail = n % self._strip_steps
+        most = 1
+        if self.raw_dtype.itemsize == 2 and not self.tiled.round_last:
+            most = 2 if self.forcing is None else 3
+        if tail > most:
+            tail = 0
+        if n > tail:
+            self._strip_launches(n - tail, write_moments and not tail)
+        for q in range(tail):
+            self.step(write_moments and q == tail - 1)
+
+    def _strip_launches(self, n, write_moments):
         a, m = self.i_pop, self.i_mom
         nt.check(self.lib.d2q9_strip_steps(
             self._Lp, self._tiled_p, self._strip_p, nt.ptr(self.f[a]),
@@ -1166,7 +1217,7 @@ class D2Q9Engine:
         if self.two_step:
             self._setup_two_step()
         if self.tiled is not None:
-            self.tiled.round_last = int(self.two_step)
+            self.tiled.round_last = int(self._round_last and self.two_step)
 
     # ---- layout helpers -------------------------------------------------
     def _upload_plane(self, pad, dtype, count=1):
@@ -1204,8 +1255,8 @@ class D2Q9Engine:
                 self._init_velocity.reshape(-1, 2)[self._tiled_solid]):
             # the tiled and strip sweeps are for solids at rest
             self.tiled = self.strips = None
-            if self._round_last:
-                self._round_last = False
+            if self._several and self.two_step:
+                self._several = self._round_last = False
                 self._setup_two_step()
         with torch.cuda.stream(self.stream):
             m = self._mom_from_host(self._init_density, self._init_velocity)

@@ -199,6 +199,17 @@ def test_strip_split_covers_with_plain_chunks(name, rows):
 
 
 def test_strip_rows_rule():
-    assert strip_rows(1024, 19, False) is None
-    assert strip_rows(8192, 37, True) == 128
-    assert strip_rows(1500, 24, False) == 24
+    """One row count per case: chunks just fill whole rounds of what the GPU
+    holds at once (1536, in FP64 768), or None for small lattices."""
+    def rows(nx, strips, double, **kw):
+        return strip_rows(np.full(strips, nx), double, **kw)
+    assert rows(800, 14, False) is None
+    assert rows(1024, 19, False, rounds=True) is None
+    assert strip_rows(np.zeros(0, dtype=int), True) is None
+    for nx, strips, double in ((2048, 19, False), (1500, 24, False),
+                               (1100, 20, True), (900, 17, False)):
+        r = rows(nx, strips, double)
+        n = strips * max(1, round(nx / r))
+        slots = 768 if double else 1536
+        assert 0.85 * slots < n <= slots
+    assert 40 <= rows(8192, 37, True) <= 160

@@ -302,7 +302,8 @@ int d2q9_tiled_steps(const d2q9_lattice* L, const d2q9_tiled_desc* D, void* f_a,
 int d2q9_moments(const d2q9_lattice* L, const void* f, void* mom,
                  void* stream);
 
-/* FP64 sum of all populations over fluid cells into *out (device double).
+/* FP64 sum of all populations over fluid cells into *out.  The results of
+ * this and of the other reductions are device or pinned host memory.
  * work: device doubles, at least d2q9_reduce_work_len(L) of them. */
 int64_t d2q9_reduce_work_len(const d2q9_lattice* L);
 int d2q9_mass_fp64(const d2q9_lattice* L, const void* f, double* work,

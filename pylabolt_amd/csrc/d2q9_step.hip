@@ -18,6 +18,7 @@
 // overlapped kernels; the float forms run a fused step as one kernel.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstddef>
 #include <initializer_list>
 #include <map>
@@ -460,31 +461,73 @@ __global__ __launch_bounds__(256) void k_moments(const d2q9_lattice L,
   mom[2 * P + c] = uy;
 }
 
+// Workgroups of a residue reduction: a wave takes 64 cells of a row at a
+// time, one such piece while 2048 workgroups last.
+int residue_blocks(const d2q9_lattice* L) {
+  const int64_t pieces = (int64_t)L->nx * ((L->ny + 63) / 64), waves = RED_THREADS / 64;
+  return (int)std::min<int64_t>((pieces + waves - 1) / waves, RED_MAX_BLOCKS);
+}
+
+// Sums of a residue's six terms per workgroup.  Bound by latency on small
+// lattices, by memory on large ones; a wave's row and column come from one
+// scalar division.  (With 8 cells per thread from 64-bit divisions of a flat
+// index, 128x128 FP64 took 14 us in 8 workgroups.)
 template <typename T>
 __global__ __launch_bounds__(RED_THREADS) void k_residue_partial(
-    const d2q9_lattice L, const T* mom, T* mom_old, double* partial) {
-  __shared__ double sh[RED_THREADS / 64];
-  const int64_t n = (int64_t)L.nx * L.ny;
+    const d2q9_lattice L, const T* __restrict__ mom, T* __restrict__ mom_old,
+    double* __restrict__ partial) {
+  constexpr int WAVES = RED_THREADS / 64;
+  __shared__ double sh[6][WAVES];
+  const int lane = (int)threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const unsigned across = (unsigned)(L.ny + 63) / 64u;
+  const unsigned pieces = (unsigned)L.nx * across, step = gridDim.x * (unsigned)WAVES;
   double acc[6] = {0, 0, 0, 0, 0, 0};
-  for (int64_t e = (int64_t)blockIdx.x * RED_THREADS + threadIdx.x; e < n;
-       e += (int64_t)gridDim.x * RED_THREADS) {
-    const int i = 1 + (int)(e / L.ny), j = 1 + (int)(e % L.ny);
+  for (unsigned p = blockIdx.x * (unsigned)WAVES + (unsigned)wave; p < pieces; p += step) {
+    const int i = 1 + (int)(p / across), j = 1 + (int)(p % across) * 64 + lane;
+    if (j > L.ny) continue;
     const int64_t c = cell_index(L, i, j);
+    // all loads before the flag is looked at
+    T v[3], o[3];
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+      v[q] = mom[q * L.plane + c];
+      o[q] = mom_old[q * L.plane + c];
+    }
     if (!(L.flags[c] & D2Q9_CELL_FLUID)) continue;
 #pragma unroll
     for (int q = 0; q < 3; ++q) {
-      double v = (double)mom[q * L.plane + c];
-      double o = (double)mom_old[q * L.plane + c];
-      double d = v - o;
+      const double d = (double)v[q] - (double)o[q];
       acc[2 * q] += d * d;
-      acc[2 * q + 1] += o * o;
-      mom_old[q * L.plane + c] = mom[q * L.plane + c];
+      acc[2 * q + 1] += (double)o[q] * (double)o[q];
+      mom_old[q * L.plane + c] = v[q];
     }
   }
+#pragma unroll
   for (int q = 0; q < 6; ++q) {
-    double r = block_sum(acc[q], sh);
-    if (threadIdx.x == 0) partial[q * RED_MAX_BLOCKS + blockIdx.x] = r;
+    double r = acc[q];
+    for (int off = 32; off > 0; off >>= 1) r += __shfl_down(r, off, 64);
+    if (lane == 0) sh[q][wave] = r;
   }
+  __syncthreads();
+  if (threadIdx.x < 6) {
+    double r = 0.0;
+    for (int w = 0; w < WAVES; ++w) r += sh[threadIdx.x][w];
+    partial[threadIdx.x * RED_MAX_BLOCKS + blockIdx.x] = r;
+  }
+}
+
+// out[q] = the sum of the workgroups' partial sums q in a fixed order, one
+// wave each.
+__global__ __launch_bounds__(6 * 64) void k_residue_finish(const double* __restrict__ partial,
+                                                           int nblocks,
+                                                           double* __restrict__ out) {
+  const int q = (int)threadIdx.x >> 6, lane = (int)threadIdx.x & 63;
+  double r = 0.0;
+#pragma unroll 4
+  for (int b = lane; b < nblocks; b += 64) r += partial[q * RED_MAX_BLOCKS + b];
+  for (int off = 32; off > 0; off >>= 1) r += __shfl_down(r, off, 64);
+  if (lane == 0) out[q] = r;
 }
 
 __global__ __launch_bounds__(256) void k_copy16(const uint4* __restrict__ src,
@@ -898,7 +941,7 @@ int d2q9_residues(const d2q9_lattice* L, const void* mom, void* mom_old,
   if (int r = validate(L)) return r;
   if (!mom || !mom_old || !work || !out) return fail(D2Q9_E_ARG, "null buffer");
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const int nb = red_blocks(L);
+  const int nb = residue_blocks(L);
   if (L->storage == D2Q9_STORE_F64) {
     hipLaunchKernelGGL((k_residue_partial<double>), dim3(nb), dim3(RED_THREADS), 0, s,
                        *L, static_cast<const double*>(mom), static_cast<double*>(mom_old), work);
@@ -906,7 +949,7 @@ int d2q9_residues(const d2q9_lattice* L, const void* mom, void* mom_old,
     hipLaunchKernelGGL((k_residue_partial<float>), dim3(nb), dim3(RED_THREADS), 0, s,
                        *L, static_cast<const float*>(mom), static_cast<float*>(mom_old), work);
   }
-  hipLaunchKernelGGL((k_finish<6>), dim3(1), dim3(RED_THREADS), 0, s, work, nb, out);
+  hipLaunchKernelGGL(k_residue_finish, dim3(1), dim3(6 * 64), 0, s, work, nb, out);
   return check_hip(hipGetLastError(), "k_residue launch");
 }
 

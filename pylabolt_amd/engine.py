@@ -882,7 +882,6 @@ class D2Q9Engine:
             if force_field is not None:
                 self.force_field = self._pitched_vector(force_field)
             self.work = torch.zeros(6 * 2048, dtype=torch.float64, device=dev)
-            self.red_out = torch.zeros(8, dtype=torch.float64, device=dev)
         L = nt.Lattice()
         L.nx, L.ny, L.pitch, L.origin, L.plane = (self.nx, self.ny, self.pitch,
                                                  ORIGIN, P)
@@ -942,6 +941,7 @@ class D2Q9Engine:
         self._upload_tiles()
         self.graph_steps = max(2, int(graph_steps) // 2 * 2)
         self._graphs = {}
+        self._red_out = None
         # several steps per launch: the tiled sweep's tables, where the case
         # can be expressed in them
         self._codes = (self.tables.special_codes()
@@ -1465,14 +1465,24 @@ class D2Q9Engine:
         self.stream.synchronize()
 
     # ---- reductions -----------------------------------------------------
+    # Results go to pinned host memory, which kernels write: one wait for the
+    # engine's stream and no copy (a copy is another launch and wait of about
+    # 15 us, on the caller's stream).
+    def _reduced(self):
+        """Pinned host memory for the results of a reduction."""
+        if self._red_out is None:
+            self._red_out = torch.zeros(8, dtype=torch.float64,
+                                        pin_memory=True)
+        return self._red_out
+
     def mass(self, which="pop"):
         """FP64 sum of the populations over fluid cells."""
         idx = self.i_pop if which == "pop" else self.materialize()
         nt.check(self.lib.d2q9_mass_fp64(
             self._Lp, nt.ptr(self.f[idx]), nt.ptr(self.work),
-            nt.ptr(self.red_out), self._stream_ptr), "d2q9_mass_fp64")
+            nt.ptr(self._reduced()), self._stream_ptr), "d2q9_mass_fp64")
         self.synchronize()
-        return float(self.red_out[0].item())
+        return float(self._red_out[0])
 
     def set_force_groups(self, groups):
         """Upload the momentum-exchange node and group tables (see
@@ -1489,7 +1499,7 @@ class D2Q9Engine:
                 "work": torch.zeros(3 * nblocks, dtype=torch.float64,
                                     device=self.device),
                 "out": torch.zeros(3 * max(1, grecs.size),
-                                   dtype=torch.float64, device=self.device),
+                                   dtype=torch.float64, pin_memory=True),
             }
         return h
 
@@ -1508,8 +1518,8 @@ class D2Q9Engine:
             nt.ptr(handle["work"]), nt.ptr(handle["out"]), self._stream_ptr),
             "d2q9_momentum_exchange")
         self.synchronize()
-        return handle["out"][:3 * handle["n_groups"]].cpu().numpy().reshape(
-            -1, 3)
+        return handle["out"][:3 * handle["n_groups"]].numpy().reshape(
+            -1, 3).copy()
 
     def residue_sums(self, mom_old):
         """Six FP64 residue sums of the current moments against
@@ -1518,10 +1528,10 @@ class D2Q9Engine:
             raise RuntimeError("moments of this step were not stored")
         nt.check(self.lib.d2q9_residues(
             self._Lp, nt.ptr(self.mom[self.i_mom]), nt.ptr(mom_old),
-            nt.ptr(self.work), nt.ptr(self.red_out), self._stream_ptr),
+            nt.ptr(self.work), nt.ptr(self._reduced()), self._stream_ptr),
             "d2q9_residues")
         self.synchronize()
-        return self.red_out[:6].cpu().numpy().copy()
+        return self._red_out[:6].numpy().copy()
 
     # ---- host views (reference layouts) -----------------------------------
     def _decode_aos(self, idx):

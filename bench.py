@@ -6,17 +6,15 @@ bottom, FP64 populations -- the configuration the metric is quoted on.
 Synthetic initial state (rest, rho = 1), as in the reference's case files.
 
 One "step" is one reference time step (stream + boundaries + moments +
-collision) over the whole lattice: one fused kernel launch, replayed from a
-HIP graph.  MLUPS = Nx * Ny * steps / t / 1e6.  The kernel time comes from
+collision) over the whole lattice.  MLUPS = Nx * Ny * steps / t / 1e6.  The kernel time comes from
 HIP events recorded on the engine's own stream around the timed steps.
 
 Roofline: a single-step sweep reads and writes the 9 populations of every
 cell once per update: 144 B in FP64, 72 B in FP32, 36 B for 16-bit
-storage.  FP64 and FP32 advance pairs of steps with one launch
-(d2q9_fused_step2): the deep interior is read and written once per two
-updates (144 B per cell and launch in FP64), the rim twice (288 B);
-``achieved`` is those bytes over the launch's time (two steps),
-``single_step_equivalent_gbs`` what a single-step sweep would have to move
+storage.  The strip sweep (d2q9_strip_steps) reads and writes them once per
+launch of four steps, the two-step sweep (d2q9_fused_step2) once per two for
+the deep interior and twice for the rim; ``achieved`` is those bytes over
+the launch's time, ``single_step_equivalent_gbs`` what a single-step sweep would have to move
 at the measured update rate.  Peak is
 MI355X's 8 TB/s HBM3E.  ``traffic`` is the measured HBM bytes per launch
 from rocprofv3 FETCH_SIZE/WRITE_SIZE counters (profiles/), when present.
@@ -25,8 +23,8 @@ The CPU baseline is the C++/OpenMP restatement of the reference's
 multi-pass step (oracle/d2q9_ref.cpp) on the same workload for a bounded
 number of steps, on the host cores.
 
-The timed steps replay HIP graphs only: the graph chunk is chosen to
-divide ``--steps`` (a multiple of 4 up to 64; otherwise chunks of 32 and
+Where steps replay HIP graphs (the two-step and single sweeps), the timed
+ones replay nothing else: the graph chunk is chosen to divide ``--steps`` (a multiple of 4 up to 64; otherwise chunks of 32 and
 the remainder eager) and captured before the timer starts.
 
 Also reported: ``forms``, FP32 and 16-bit-storage runs of the same
@@ -37,8 +35,8 @@ the case's reference speed u_ref = 0.05); ``channel``, the gravity-driven
 MRT + Guo channel 4096 x 1024 at its full 20,000 steps in every storage
 form: MLUPS and roofline of each, velocity error against the FP64 run and
 of every form against the start-up series of plane Poiseuille flow;
-``batched``, 256 seeded lattices of uneven size advanced by one persistent
-launch per step; ``adjoint``, the forward + backward cost of the adjoint
+``batched``, 256 seeded lattices of uneven size advanced by one launch per
+several steps of them all; ``adjoint``, the forward + backward cost of the adjoint
 channel over its plain forward (one graph of all its steps), run in a
 child process (``ChildLeg``) so that a failure there cannot take the
 benchmark line with it; and a plain copy kernel's bandwidth on the same
@@ -229,8 +227,8 @@ def adjoint_cost(steps=2000, reps=3):
             best = dt if best is None else min(best, dt)
         return best
 
-    # plain forward: one graph of the same init + N sweeps, moments stored
-    # at the last step only, no checkpoints; its buffers are set up by a
+    # plain forward: one graph of the same init and the same sweeps, moments
+    # stored at the last step only, no checkpoints; its buffers are set up by a
     # rollout forward before the timer
     r0 = ro["sqrt"]
     r0.forward(Ft, ut)
@@ -240,12 +238,13 @@ def adjoint_cost(steps=2000, reps=3):
         nt.check(eng.lib.d2q9_init_eq(eng._Lp, nt.ptr(r0.work[0]),
                                       nt.ptr(r0.work[1]), nt.ptr(r0.mom0),
                                       eng._stream_ptr), "d2q9_init_eq")
-        prev = r0.work[0]
-        for n in range(1, steps + 1):
-            dst = r0.work[n % 2]
-            r0._sweep(prev, dst, r0.mscratch[(n - 1) % 2], r0.mscratch[n % 2],
-                      n == 1, n == steps)
-            prev = dst
+        prev, n = r0.work[0], 0
+        for m in r0._per_launch(steps):
+            dst = r0.work[1] if prev is r0.work[0] else r0.work[0]
+            r0._sweeps(prev, dst, r0.mom0,
+                       r0.mscratch[0] if n + m == steps else None, n == 0, m,
+                       False)
+            prev, n = dst, n + m
     g_plain = r0._capture(issue_plain)
 
     def plain():
@@ -255,8 +254,8 @@ def adjoint_cost(steps=2000, reps=3):
     t_plain = timed(plain)
     eng.lib.d2q9_graph_destroy(g_plain)
     out["plain_forward_ms"] = t_plain * 1e3
-    out["plain_forward"] = ("one HIP graph: d2q9_init_eq + collide + "
-                            f"{steps - 1} fused steps, no checkpoints")
+    out["plain_forward"] = (f"one HIP graph: d2q9_init_eq + {steps} steps, "
+                            "several per launch, no checkpoints")
     for m, r in ro.items():
         u = r.forward(Ft, ut)
         g = torch.zeros_like(u)
@@ -274,9 +273,9 @@ def batched_form(steps=5000, warmup=50, per_lattice_steps=100, n=256,
                  seed=0):
     """Batched workload: ``n`` seeded lattices (sizes uniform over the
     multiples of 32 in 64..1024 x 64..512, Re in [50, 400], even ids cavity
-    BGK, odd ids Guo-forced channel MRT), FP32, one persistent launch per
-    step replayed from HIP graphs, launch configuration from the
-    autotuner.  Aggregate MLUPS = sum of cells * steps / t.  The same
+    BGK, odd ids Guo-forced channel MRT), FP32, several steps of all of them
+    per launch (``config``, the autotuner's choice, is for the persistent
+    kernel that takes batches the tiled sweep cannot).  Aggregate MLUPS = sum of cells * steps / t.  The same
     lattices advanced one launch per lattice per step are timed beside it
     over ``per_lattice_steps`` steps."""
     import torch
@@ -303,7 +302,9 @@ def batched_form(steps=5000, warmup=50, per_lattice_steps=100, n=256,
     t = timed(lambda: batch.advance(steps, write_moments=True))
     cells = batch.cells
     mlups = cells * steps / t / 1e6
-    achieved = mlups * 1e6 * BYTES_PER_CELL["f32"] / 1e9
+    # a launch reads and writes every cell once for all its steps
+    achieved = (mlups * 1e6 * BYTES_PER_CELL["f32"] / 1e9 /
+                batch.steps_per_launch)
     finite = all(bool(np.isfinite(e.moments_host()[1]).all())
                  for e in batch.engines[:8])
     mlups_pl = None
@@ -316,6 +317,7 @@ def batched_form(steps=5000, warmup=50, per_lattice_steps=100, n=256,
         "lattices": n, "cells": cells, "steps": steps,
         "mlups": mlups, "us_per_step": t / steps * 1e6,
         "achieved_gbs": achieved, "frac": achieved / PEAK_GBS,
+        "steps_per_launch": batch.steps_per_launch,
         "config": batch.config.as_dict(), "items_per_step": batch.n_items,
         "tuner_candidates": len(tuner.trials),
         "setup_and_tune_s": t_setup,
@@ -338,10 +340,23 @@ def load_pmc(workload, storage):
 
 def sweep_rate(engine, bpc, ms_step, cells):
     """HBM rate of the measured sweep: (achieved GB/s, single-step
-    equivalent GB/s, two-step details or None).  A two-step launch moves
-    bpc per deep cell and 2 bpc per rim cell for two updates."""
+    equivalent GB/s, details of a launch of several steps or None).  The
+    strip sweep moves bpc per cell and launch, a two-step launch bpc per deep
+    cell and 2 bpc per rim cell."""
     single = bpc * cells / (ms_step * 1e-3) / 1e9
-    if not getattr(engine, "two_step", False):
+    n = None
+    if engine.strips is not None:
+        n, kind = engine.strip_steps, "d2q9_strip_steps (k_strip)"
+    elif engine.tiled is not None:
+        n, kind = engine.tiled.steps, "d2q9_tiled_steps (k_tiled)"
+    if n is not None:
+        return bpc * cells / (n * ms_step * 1e-3) / 1e9, single, {
+            "launch": f"{kind}, {n} steps per launch",
+            "kind": "strips" if engine.strips is not None else "tiled",
+            "steps_per_launch": n,
+            "algorithmic_bytes_per_launch": bpc * cells,
+            "launch_us": n * ms_step * 1e3}
+    if not engine.two_step:
         return single, single, None
     deep = int(round(engine.deep_fraction * cells))
     rim = cells - deep
@@ -350,6 +365,7 @@ def sweep_rate(engine, bpc, ms_step, cells):
     return achieved, single, {
         "launch": "d2q9_fused_step2 (k_deep2 + rim sweeps), two steps per "
                   "launch",
+        "kind": "two-step", "steps_per_launch": 2,
         "deep_cells": deep, "rim_cells": rim, "deep_fraction": deep / cells,
         "algorithmic_bytes_per_launch": launch_bytes,
         "launch_us": 2 * ms_step * 1e3}
@@ -357,8 +373,9 @@ def sweep_rate(engine, bpc, ms_step, cells):
 
 def run_form(sim, storage, steps, warmup, tile, use_graph=True):
     """Time ``steps`` steps of ``sim`` in one storage form after ``warmup``
-    steps.  Every form asks for the two-step sweep (FP64 and FP32 would
-    take it by size anyway; 16-bit storage only on request)."""
+    steps.  Every form asks for two steps per sweep, which in 16-bit storage
+    lets any sweep of several steps round the last one only (FP64 and FP32
+    give the same bits through every sweep)."""
     from pylabolt_amd.solvers.fluidLB import Solver
     solver = Solver(simulation=sim, storage=storage, tile=tile,
                     graph_steps=graph_steps_for(steps), verbose=False,
@@ -397,7 +414,7 @@ def startup_series(y, H, nu, g, t, terms=400):
 def channel_leg(storages, steps=None, warmup=100):
     """Gravity-driven channel 4096 x 1024, MRT + second-order Guo, Re = 100
     at u_max = 0.05, from rest, all its steps (20,000) in every storage
-    form, two-step sweeps from HIP graphs.  Per form: MLUPS and roofline of
+    form, two or more steps per launch.  Per form: MLUPS and roofline of
     the whole run, velocity error against the FP64 run (relative L2 over
     all cells) and the x-averaged profile against the start-up series."""
     import torch
@@ -431,7 +448,7 @@ def channel_leg(storages, steps=None, warmup=100):
                "us_per_step": ms_step * 1e3, "gbs": achieved,
                "frac": achieved / PEAK_GBS,
                "single_step_equivalent_gbs": single,
-               "two_step": two is not None,
+               "launch": two["kind"] if two else "single",
                "u_rel_l2_vs_startup_series": float(
                    np.linalg.norm(prof - series) / np.linalg.norm(series))}
         if ref is None:
@@ -591,7 +608,8 @@ def run_legs(args, adj_leg):
         a2, single2, two2 = sweep_rate(s2.engine, BYTES_PER_CELL[form], st2,
                                        cells)
         rec = {"mlups": m2, "us_per_step": st2 * 1e3, "gbs": a2,
-               "frac": a2 / PEAK_GBS, "two_step": two2 is not None,
+               "frac": a2 / PEAK_GBS,
+               "launch": two2["kind"] if two2 else "single",
                "single_step_equivalent_gbs": single2}
         if main is None:
             main = (ms2, wall2, st2, m2, a2, single2, two2)
@@ -658,7 +676,7 @@ def run_legs(args, adj_leg):
         log(f"copy kernel: {copy_gbs:.0f} GB/s")
     pmc = load_pmc(args.workload, args.storage)
     traffic = pmc["hbm_bytes_per_launch"] if pmc else None
-    if pmc and two is not None and pmc.get("launch") != "two-step":
+    if pmc and two is not None and pmc.get("launch") != two["kind"]:
         traffic = None     # counters of another launch shape
     traffic_source = (f"profiles/pmc_{args.workload}_{args.storage}.json: "
                       "rocprofv3 FETCH_SIZE and WRITE_SIZE of the same "
@@ -693,7 +711,8 @@ def run_legs(args, adj_leg):
                      "traffic": traffic,
                      "traffic_source": traffic_source,
                      "bytes_per_cell_update": (
-                         two["algorithmic_bytes_per_launch"] / (2 * cells)
+                         two["algorithmic_bytes_per_launch"] /
+                         (two["steps_per_launch"] * cells)
                          if two else bpc),
                      "single_step_bytes_per_cell_update": bpc,
                      "single_step_equivalent_gbs": single_equiv},

@@ -313,6 +313,7 @@ class BatchedLattices:
         the whole batch; off where some lattice has no tables for it."""
         self.tiled = all(e.tiled is not None for e in self.engines)
         self._tiled_key = None
+        self.steps_per_launch = 1
         if not self.tiled:
             return
         self._tiled_region = tiled_shape(
@@ -320,6 +321,7 @@ class BatchedLattices:
             self.storage == "f64",
             any(e.forcing is not None for e in self.engines))
         rows, width, steps = self._tiled_region
+        self.steps_per_launch = steps
         items = []
         for l, e in enumerate(self.engines):
             ti, tj = np.meshgrid(np.arange(-(-e.nx // (rows - 2 * steps))),

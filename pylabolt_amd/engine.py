@@ -1152,7 +1152,7 @@ class D2Q9Engine:
         P.chunks, P.tiles = (t.data_ptr() for t in self._strip_lists)
         self.strips = P
         self._strip_p = ctypes.byref(P)
-        self._strip_steps = self._strip_shape[0]
+        self.strip_steps = self._strip_shape[0]
 
     def _advance_strips(self, n, write_moments):
         """``n`` steps through the strip sweep.
@@ -1163,7 +1163,7 @@ class D2Q9Engine:
         bound by its arithmetic and the single sweep is relatively cheap:
         two left over are single steps too (BF16 8192x2048: 110 us each, 240
         to 370 a launch of 2), with a force three (112 each, 390)."""
-        tail = n % self._strip_steps
+        tail = n % self.strip_steps
         most = 1
         if self.raw_dtype.itemsize == 2 and not self.tiled.round_last:
             most = 2 if self.forcing is None else 3
@@ -1181,7 +1181,7 @@ class D2Q9Engine:
             nt.ptr(self.f[1 - a]), nt.ptr(self.mom[m]),
             nt.ptr(self.mom[1 - m]), n, int(write_moments),
             self._stream_ptr), "d2q9_strip_steps")
-        flip = -(-n // self._strip_steps) & 1
+        flip = -(-n // self.strip_steps) & 1
         self.i_pop, self.i_mom = a ^ flip, m ^ flip
         self.mom_full = bool(write_moments)
         self.time_step += n

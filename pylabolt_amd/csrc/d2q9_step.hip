@@ -626,7 +626,8 @@ int aux_for_stream(hipStream_t s, Aux** out) {
 }
 
 // fork == false: the general/fix-up kernel runs on `s` too, before the
-// bulk kernel (for callers that already run on the auxiliary stream).
+// bulk kernel (for callers that already run on the auxiliary stream, and
+// for the collide-only and stream-only sweeps).
 template <int S, int MODEL, int FORCING, int PHASE>
 int launch_sweep(const d2q9_lattice* L, const void* fsrc, void* fdst,
                  const void* msrc, void* mdst, int write_mom, hipStream_t s,
@@ -727,20 +728,25 @@ int dispatch(const d2q9_lattice* L, const void* fsrc, void* fdst, const void* ms
   if (PHASE != PHASE_STREAM && !mdst) return fail(D2Q9_E_ARG, "null mom_dst");
   if (fsrc == fdst) return fail(D2Q9_E_ARG, "f_src and f_dst must differ");
   hipStream_t s = static_cast<hipStream_t>(stream);
+  // the first and the last sweep of a run alone need not overlap their two
+  // kernels: the join costs what the overlap saves, and a lattice that is
+  // otherwise swept without a fork is spared the auxiliary stream, whose
+  // creation takes 0.25 ms
+  const bool fork = PHASE == PHASE_FUSED;
   if (PHASE == PHASE_STREAM) {
     // streaming never touches the collision model: one instantiation each
     switch (L->storage) {
-      case D2Q9_STORE_F64: return launch_sweep<D2Q9_STORE_F64, D2Q9_BGK, D2Q9_FORCING_NONE, PHASE>(L, fsrc, fdst, msrc, mdst, 0, s);
-      case D2Q9_STORE_F32: return launch_sweep<D2Q9_STORE_F32, D2Q9_BGK, D2Q9_FORCING_NONE, PHASE>(L, fsrc, fdst, msrc, mdst, 0, s);
-      case D2Q9_STORE_F16DEV: return launch_sweep<D2Q9_STORE_F16DEV, D2Q9_BGK, D2Q9_FORCING_NONE, PHASE>(L, fsrc, fdst, msrc, mdst, 0, s);
-      case D2Q9_STORE_BF16DEV: return launch_sweep<D2Q9_STORE_BF16DEV, D2Q9_BGK, D2Q9_FORCING_NONE, PHASE>(L, fsrc, fdst, msrc, mdst, 0, s);
+      case D2Q9_STORE_F64: return launch_sweep<D2Q9_STORE_F64, D2Q9_BGK, D2Q9_FORCING_NONE, PHASE>(L, fsrc, fdst, msrc, mdst, 0, s, fork);
+      case D2Q9_STORE_F32: return launch_sweep<D2Q9_STORE_F32, D2Q9_BGK, D2Q9_FORCING_NONE, PHASE>(L, fsrc, fdst, msrc, mdst, 0, s, fork);
+      case D2Q9_STORE_F16DEV: return launch_sweep<D2Q9_STORE_F16DEV, D2Q9_BGK, D2Q9_FORCING_NONE, PHASE>(L, fsrc, fdst, msrc, mdst, 0, s, fork);
+      case D2Q9_STORE_BF16DEV: return launch_sweep<D2Q9_STORE_BF16DEV, D2Q9_BGK, D2Q9_FORCING_NONE, PHASE>(L, fsrc, fdst, msrc, mdst, 0, s, fork);
     }
   } else {
     switch (L->storage) {
-      case D2Q9_STORE_F64: return dispatch_model<D2Q9_STORE_F64, PHASE>(L, fsrc, fdst, msrc, mdst, wm, s);
-      case D2Q9_STORE_F32: return dispatch_model<D2Q9_STORE_F32, PHASE>(L, fsrc, fdst, msrc, mdst, wm, s);
-      case D2Q9_STORE_F16DEV: return dispatch_model<D2Q9_STORE_F16DEV, PHASE>(L, fsrc, fdst, msrc, mdst, wm, s);
-      case D2Q9_STORE_BF16DEV: return dispatch_model<D2Q9_STORE_BF16DEV, PHASE>(L, fsrc, fdst, msrc, mdst, wm, s);
+      case D2Q9_STORE_F64: return dispatch_model<D2Q9_STORE_F64, PHASE>(L, fsrc, fdst, msrc, mdst, wm, s, fork);
+      case D2Q9_STORE_F32: return dispatch_model<D2Q9_STORE_F32, PHASE>(L, fsrc, fdst, msrc, mdst, wm, s, fork);
+      case D2Q9_STORE_F16DEV: return dispatch_model<D2Q9_STORE_F16DEV, PHASE>(L, fsrc, fdst, msrc, mdst, wm, s, fork);
+      case D2Q9_STORE_BF16DEV: return dispatch_model<D2Q9_STORE_BF16DEV, PHASE>(L, fsrc, fdst, msrc, mdst, wm, s, fork);
     }
   }
   return fail(D2Q9_E_ARG, "bad storage");

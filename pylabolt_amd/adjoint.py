@@ -10,11 +10,15 @@ dL/du_N and returns dL/dF and dL/du0.  ``LBMFlow`` wraps the pair as a
 Memory/compute schedule (``checkpoint``):
 
 * ``"sqrt"`` (default): the forward pass stores the post-collision
-  populations every K = ceil(sqrt(N)) steps -- the step that produces a
-  checkpoint writes straight into its slot, so checkpoints cost no extra
-  traffic; the backward pass walks the segments last to first, re-running
-  each segment's K forward steps to store their rho/u (24 B per cell per
-  step), then running the K adjoint steps.  Memory: ~2 sqrt(N) lattices.
+  populations every K steps -- the step that produces a checkpoint writes
+  straight into its slot, so checkpoints cost no extra traffic -- and the
+  rho/u of each of the last K steps (24 B per cell per step); the backward
+  pass walks the segments last to first, re-running the K forward steps of
+  each but the last to store their rho/u, then running the K adjoint steps.
+  K is about sqrt(N): memory of about 12 sqrt(N) planes of 8 B per cell.  (At
+  sqrt(3 N) it is least, 10.4, and fewer steps run again, but the moments of a
+  segment outgrow the last-level cache sooner: 1024x256 over 400 steps 8.55 ms
+  with K = 36, 8.50 with 20.)
 * ``"moments"``: the forward pass stores rho/u of every step (24 B per cell
   per step, 12.6 GB for 2000 steps of 1024 x 256) and the backward pass
   recomputes nothing.
@@ -88,12 +92,17 @@ class FlowRollout:
         dev = eng.device
         P, L = eng.plane, eng.pop_len
         N = self.steps
-        self.K = int(math.ceil(math.sqrt(N))) if self.mode == "sqrt" else N
+        # whole launches; the first segment takes what is left
+        most = eng.tiled.steps if eng.tiled is not None else 1
+        self.K = (min(N, -(-math.ceil(math.sqrt(N)) // most) * most)
+                  if self.mode == "sqrt" else N)
         self.nseg = int(math.ceil(N / self.K))
+        # segment s runs the steps ends[s] + 1 .. ends[s + 1]
+        self.ends = [0] + [N - q * self.K
+                           for q in range(self.nseg - 1, -1, -1)]
         z = dict(dtype=torch.float64, device=dev)
         with torch.cuda.stream(eng.stream):
-            nck = self.nseg if self.mode == "sqrt" else 1
-            self.ck = [torch.zeros(L, **z) for _ in range(nck)]
+            self.ck = [torch.zeros(L, **z) for _ in range(self.nseg)]
             self.work = [torch.zeros(L, **z) for _ in range(2)]
             # rho/u of the steps of a segment, one after another
             moments = torch.zeros(self.K, 3 * P, **z)
@@ -108,8 +117,11 @@ class FlowRollout:
         self._rho0 = torch.from_numpy(
             np.asarray(f.density).reshape(self.nx + 2, self.ny + 2)).to(dev)
         self._fwd_graph = None
-        self._bwd_graph = None
+        self._bwd_graphs = {}
         self._last_moments = None
+        # whether the ring holds the last segment's moments of the last
+        # forward pass (a backward pass of several segments replaces them)
+        self._ring_is_last = False
 
     # ---- checks --------------------------------------------------------
     def _check_permutation(self):
@@ -201,23 +213,20 @@ class FlowRollout:
         (src, dst, msrc, mdst, first, steps, every) as for ``_sweeps``.
         The supported rules read no moments of the step before, so every
         launch may name the same msrc."""
-        N, K = self.steps, self.K
         ops = []
         # g_0 = feq(rho0, u0) lives in ck[0]; work[1] also receives it
-        prev, n = self.ck[0], 0
-        every = self.mode == "moments"
-        while n < N:
-            seg = min(K, N - n)
-            for q, m in enumerate(self._per_launch(seg)):
-                end = n + m
-                ckpt = not every and end % K == 0 and end // K < self.nseg
-                dst = (self.ck[end // K] if ckpt else
+        prev = self.ck[0]
+        for s in range(self.nseg):
+            n, end = self.ends[s], self.ends[s + 1]
+            last = s == self.nseg - 1
+            for m in self._per_launch(end - n):
+                dst = (self.ck[s + 1] if n + m == end and not last else
                        self.work[1] if prev is self.work[0] else self.work[0])
-                mdst = (self.ring[n] if every else
-                        self.mscratch[0] if end == N else None)
-                ops.append((prev, dst, self.mom0, mdst, n == 0, m, every))
-                prev, n = dst, end
-        self._last_moments = self.ring[N - 1] if every else self.mscratch[0]
+                ops.append((prev, dst, self.mom0,
+                            self.ring[n - self.ends[s]] if last else None,
+                            n == 0, m, last))
+                prev, n = dst, n + m
+        self._last_moments = self.ring[self.ends[-1] - self.ends[-2] - 1]
         return ops
 
     def _capture(self, issue):
@@ -243,13 +252,13 @@ class FlowRollout:
         for op in self._forward_ops():
             self._sweeps(*op)
 
-    def _issue_backward(self):
+    def _issue_backward(self, ring_is_last):
         e = self.eng
-        N, K = self.steps, self.K
+        N = self.steps
         lam_cur, lam_nxt = self.lam[0], self.lam[1]
         for s in range(self.nseg - 1, -1, -1):
-            n0, n1 = s * K + 1, min((s + 1) * K, N)
-            if self.mode == "sqrt":
+            n0, n1 = self.ends[s] + 1, self.ends[s + 1]
+            if s < self.nseg - 1 or not ring_is_last:
                 # recompute the segment, storing rho/u of each step
                 if s == 0:
                     nt.check(e.lib.d2q9_init_eq(
@@ -266,7 +275,7 @@ class FlowRollout:
                     prev, n = dst, n + m
             n = n1
             for m in self._per_launch(n1 - n0 + 1):
-                slot = (n - n0) if self.mode == "sqrt" else n - 1
+                slot = n - n0
                 seed = self.seed if n == N else None
                 if e.tiled is None:
                     rc = e.lib.d2q9_adjoint_step(
@@ -306,6 +315,7 @@ class FlowRollout:
                  "graph launch")
         with torch.cuda.stream(e.stream):
             u = self._from_pitched(self._last_moments, 1, 2)
+        self._ring_is_last = True
         e.stream.synchronize()
         return u
 
@@ -320,10 +330,13 @@ class FlowRollout:
             self.grad_f.zero_()
             for t in self.lam:
                 t.zero_()
-        if self._bwd_graph is None:
-            self._bwd_graph = self._capture(self._issue_backward)
-        nt.check(e.lib.d2q9_graph_launch(self._bwd_graph, e._stream_ptr),
-                 "graph launch")
+        ready = self._ring_is_last
+        if ready not in self._bwd_graphs:
+            self._bwd_graphs[ready] = self._capture(
+                lambda: self._issue_backward(ready))
+        self._ring_is_last = ready and self.nseg == 1
+        nt.check(e.lib.d2q9_graph_launch(self._bwd_graphs[ready],
+                                         e._stream_ptr), "graph launch")
         with torch.cuda.stream(e.stream):
             gf = self._from_pitched(self.grad_f, 0, 2)
             gu = self._from_pitched(self.grad_init, 1, 2)
@@ -331,10 +344,11 @@ class FlowRollout:
         return gf, gu
 
     def close(self):
-        for g in (self._fwd_graph, self._bwd_graph):
+        for g in (self._fwd_graph, *self._bwd_graphs.values()):
             if g is not None:
                 self.eng.lib.d2q9_graph_destroy(g)
-        self._fwd_graph = self._bwd_graph = None
+        self._fwd_graph = None
+        self._bwd_graphs = {}
 
 
 class LBMFlow(torch.autograd.Function):

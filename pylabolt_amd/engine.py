@@ -1313,7 +1313,8 @@ class D2Q9Engine:
         self.i_mom = 1 - self.i_mom
 
     def step2(self, write_moments=False):
-        """Advance two reference time steps with the two-step sweep."""
+        """Advance two reference time steps, with the two-step sweep where
+        the lattice takes it."""
         if self.tiled is not None:
             self.advance(2, write_moments)
             return

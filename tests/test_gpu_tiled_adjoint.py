@@ -55,3 +55,27 @@ def test_rollout_equals_single_steps(case, forcing, size, steps, mode):
         r.close()
     for a, b in zip(*got):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("steps,mode", [(3, "sqrt"), (40, "sqrt"),
+                                        (41, "sqrt"), (9, "moments")])
+def test_backward_again_and_another_forward(steps, mode):
+    """A second reverse pass of the same forward pass gives the same, though
+    the first one has replaced the moments of the last segment; so does one
+    after another forward pass and back."""
+    rng = np.random.default_rng(2)
+    force, u0, seed = (torch.tensor(rng.normal(0, s, (30, 40, 2)),
+                                    device="cuda") for s in (1e-5, 0.01, 1))
+    r = FlowRollout(_channel(30, 40, "guo_linear"), steps, checkpoint=mode)
+    u = r.forward(force, u0)
+    first = r.backward(seed)
+    again = r.backward(seed)
+    r.forward(2 * force, u0)
+    other = r.backward(seed)
+    v = r.forward(force, u0)
+    last = r.backward(seed)
+    r.close()
+    assert torch.equal(u, v)
+    for a, b, c, d in zip(first, again, last, other):
+        assert torch.equal(a, b) and torch.equal(a, c)
+    assert not torch.equal(other[1], first[1])

@@ -200,9 +200,9 @@ int d2q9_collide(const d2q9_lattice* L, const void* f_src, void* f_dst,
 int d2q9_stream_bc(const d2q9_lattice* L, const void* f_src, void* f_dst,
                    const void* mom_src, void* stream);
 
-/* The sweeps (d2q9_collide, d2q9_stream_bc, d2q9_fused_step) launch the
- * bulk tiles on `stream` and the general tiles plus fix-up cells on an
- * auxiliary stream, forked from and joined back to `stream` with events
+/* d2q9_collide and d2q9_stream_bc run on `stream` alone.  d2q9_fused_step
+ * launches the bulk tiles on `stream` and the general tiles plus fix-up cells
+ * on an auxiliary stream, forked from and joined back to `stream` with events
  * (both passes write disjoint cells), so the two overlap; the library
  * creates one auxiliary stream and event pair per caller stream (and
  * device) on first use and keeps them for the process (at most 4096

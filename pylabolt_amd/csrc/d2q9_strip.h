@@ -7,8 +7,8 @@
 // pulls from are there.  Steps hand rows on through LDS rings that hold what
 // is still to be pulled: three rows of the directions pulled from the same or
 // the next row, four of those pulled from the row before.  The first wave
-// pulls from the lattice (rows ahead, in registers), the last stores to the
-// other one.  A lane holds one cell, so a row is 64 cells wide, STEPS of them on
+// pulls from the lattice (a row or two ahead, in registers), the last stores
+// to the other one.  A lane holds one cell, so a row is 64 cells wide, STEPS of them on
 // either side for the neighbouring strips' sake only.  (Two cells a lane for the
 // float forms halve the waves a CU holds: FP32 2999x1111 22 us per step against
 // 18, 8192x2048 97 against 91.)
@@ -35,7 +35,6 @@ constexpr int THREADS = 64 * STEPS;
 constexpr int COLS = 64 - 2 * STEPS;         // output columns of a strip
 constexpr int TILE_W = 16;                   // region width of the tiles
 constexpr int TILE = TILE_W - 2 * STEPS;     // their output rows and columns
-constexpr int AHEAD = 2;                     // rows the first wave loads ahead
 // Rows of a ring, three directions each: 3 of 0,2,4, 3 of 3,6,7, 4 of 1,5,8.
 constexpr int RING_B = 9, RING_C = 18, RING = 30;
 
@@ -46,6 +45,23 @@ constexpr int PITCH = 64 + 2;                // values of an LDS row
 template <int S>
 constexpr size_t ring_bytes(int steps) {
   return (size_t)(steps - 1) * RING * PITCH * sizeof(typename Codec<S>::T);
+}
+
+// Barrier of the workgroup that waves may reach at different places of the
+// code, with the LDS traffic before it done: s_barrier counts arrivals.
+__device__ __forceinline__ void workgroup_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+}
+
+// A row's values: the loaded ones themselves, or room for them decoded.
+template <typename R, typename T>
+__device__ __forceinline__ T (&values_of(R (&raw)[9], T (&apart)[9]))[9] {
+  if constexpr (std::is_same<R, T>::value)
+    return raw;
+  else
+    return apart;
 }
 
 template <int S, int MODEL, int FORCING>
@@ -98,10 +114,6 @@ __device__ __forceinline__ void run_strip(
   int i = ch.i_first - (K - st);
   T* const to = reinterpret_cast<T*>(smem) + (st - 1) * RING * PITCH + 1 + lane;
   const T* const from = to - RING * PITCH;
-  // The first step's rows, AHEAD of them in registers: with one, the memory
-  // system is mostly idle (FP64 8192x2048: 349 us per step against 165; four or
-  // six are no faster).
-  R raw[AHEAD][9];
   auto fetch = [&](R (&r)[9], int row) {
     const unsigned r0 = row_at(row), rp = row_at(row + 1), rm = row_at(row - 1);
     const unsigned dp = helper ? r0 : rp, dm = helper ? r0 : rm;
@@ -112,106 +124,149 @@ __device__ __forceinline__ void run_strip(
                                          (at + (CY[k] == 0 ? p0 : CY[k] > 0 ? pm : pp)));
     }
   };
-  if (st == 1) {
-#pragma unroll
-    for (int q = 0; q < AHEAD; ++q)
-      if (q < count) fetch(raw[q], i + q);
-  }
   int a3 = 0, a4 = 0;   // ring slots this row is written to (row number mod 3 and 4)
-#pragma unroll 1
-  for (int t0 = 0; t0 < total; t0 += AHEAD) {
-#pragma unroll
-    for (int u = 0; u < AHEAD; ++u) {
-      const int t = t0 + u;
-      if (t >= total) break;   // the whole workgroup
-      if (st <= K && t >= begin && t < begin + count) {
-        T g[9];
-        if (st == 1) {
-#pragma unroll
-          for (int k = 0; k < 9; ++k) g[k] = C::dec(raw[u][k], k, Kc);
-          if (lo == 2) {
-            const T b4 = wave_from_prev(g[4]), b7 = wave_from_prev(g[7]),
-                    b8 = wave_from_prev(g[8]);
-            if (wall_lo) {
-              g[2] = b4;
-              g[5] = b7;
-              g[6] = b8;
-            }
-          }
-          if (hi == 2) {
-            const T b2 = wave_from_next(g[2]), b5 = wave_from_next(g[5]),
-                    b6 = wave_from_next(g[6]);
-            if (wall_hi) {
-              g[4] = b2;
-              g[7] = b5;
-              g[8] = b6;
-            }
-          }
-          if (t + AHEAD < count) fetch(raw[u], i + AHEAD);
-        } else {
-          // rows i (number n + 1 of the step before), i + 1 (n + 2), i - 1 (n)
-          const int same = (a3 == 2 ? 0 : a3 + 1) * 3;
-          const int next = RING_B + (a3 == 0 ? 2 : a3 - 1) * 3;
-          const T* const r0 = from + same * PITCH;
-          const T* const rb = from + next * PITCH;
-          const T* const rc = from + (RING_C + a4 * 3) * PITCH;
-#pragma unroll
-          for (int k = 0; k < 9; ++k)
-            g[k] = (CX[k] == 0 ? r0 : CX[k] < 0 ? rb : rc)[SLOT[k] * PITCH - CY[k]];
-          if ((lo | hi) && (wall_lo || wall_hi)) {
-            const T* const own_b = from + (RING_B + same) * PITCH;
-            const T* const own_c = from + (RING_C + ((a4 + 1) & 3) * 3) * PITCH;
-#pragma unroll
-            for (int k = 1; k < 9; ++k) {
-              if (CY[k] == 0 || (CY[k] == 1 ? !wall_lo : !wall_hi)) continue;
-              const int o = INV[k];
-              g[k] = zg ? (CX[k] == 0 ? r0 : CX[k] < 0 ? rb : rc)[SLOT[k] * PITCH]
-                        : (CX[o] == 0 ? r0 : CX[o] < 0 ? own_b : own_c)[SLOT[o] * PITCH];
-            }
-          }
-        }
-        const int cell = L.origin + wrap(i) * L.pitch + j;
-        T ffx = (T)0, ffy = (T)0;
-        if (FORCING != D2Q9_FORCING_NONE && L.force_source == D2Q9_FSRC_FIELD) {
-          const T* ff = static_cast<const T*>(L.force_field);
-          ffx = ff[cell];
-          ffy = ff[L.plane + cell];
-        }
-        T drho, rho, ux, uy, fx, fy, px, py;
-        moments<T, FORCING, C::dev>(g, L, Kc, ffx, ffy, drho, rho, ux, uy, fx, fy, px, py);
-        collide<T, MODEL, FORCING, C::dev>(g, Kc, drho, rho, ux, uy, fx, fy, px, py);
-        const uint32_t key = sizeof(R) == 2 ? cell_key((uint32_t)cell) : 0u;
-        if (st < K) {
-          T* const w0 = to + a3 * 3 * PITCH;
-          T* const wc = to + (RING_C + a4 * 3) * PITCH;
-          if (sizeof(R) == 2 && !round_last) {
-#pragma unroll
-            for (int k = 0; k < 9; ++k) g[k] = tiled::through_storage<S>(g[k], k, key, Kc);
-          }
-#pragma unroll
-          for (int k = 0; k < 9; ++k)
-            (CX[k] == 0 ? w0 : CX[k] < 0 ? w0 + RING_B * PITCH : wc)[SLOT[k] * PITCH] = g[k];
-        } else if (out) {
-          // plain stores: a strip's segments end inside cache lines that the
-          // next strip completes (non-temporal: FP32 8192x2048 91 us against 83)
-          const unsigned at = row_at(i) + p0;
-#pragma unroll
-          for (int k = 0; k < 9; ++k)
-            *reinterpret_cast<R*>(reinterpret_cast<char*>(fdst + k * B) + at) =
-                C::encs(g[k], k, key, Kc);
-          if (write_mom) {
-            mdst[cell] = rho;
-            mdst[L.plane + cell] = ux;
-            mdst[2 * L.plane + cell] = uy;
-          }
-        }
-        ++i;
-        a3 = a3 == 2 ? 0 : a3 + 1;
-        a4 = (a4 + 1) & 3;
-      }
-      __syncthreads();
+  // One row of step `st`, from its pulled populations on: moments, collision,
+  // and the row's way on.
+  auto finish = [&](T (&g)[9], auto stores) {
+    const int cell = L.origin + wrap(i) * L.pitch + j;
+    T ffx = (T)0, ffy = (T)0;
+    if (FORCING != D2Q9_FORCING_NONE && L.force_source == D2Q9_FSRC_FIELD) {
+      const T* ff = static_cast<const T*>(L.force_field);
+      ffx = ff[cell];
+      ffy = ff[L.plane + cell];
     }
-  }
+    T drho, rho, ux, uy, fx, fy, px, py;
+    moments<T, FORCING, C::dev>(g, L, Kc, ffx, ffy, drho, rho, ux, uy, fx, fy, px, py);
+    collide<T, MODEL, FORCING, C::dev>(g, Kc, drho, rho, ux, uy, fx, fy, px, py);
+    const uint32_t key = sizeof(R) == 2 ? cell_key((uint32_t)cell) : 0u;
+    if (!decltype(stores)::value || st < K) {
+      T* const w0 = to + a3 * 3 * PITCH;
+      T* const wc = to + (RING_C + a4 * 3) * PITCH;
+      if (sizeof(R) == 2 && !round_last) {
+#pragma unroll
+        for (int k = 0; k < 9; ++k) g[k] = tiled::through_storage<S>(g[k], k, key, Kc);
+      }
+#pragma unroll
+      for (int k = 0; k < 9; ++k)
+        (CX[k] == 0 ? w0 : CX[k] < 0 ? w0 + RING_B * PITCH : wc)[SLOT[k] * PITCH] = g[k];
+    } else if (out) {
+      // plain stores: a strip's segments end inside cache lines that the
+      // next strip completes (non-temporal: FP32 8192x2048 91 us against 83)
+      const unsigned at = row_at(i) + p0;
+#pragma unroll
+      for (int k = 0; k < 9; ++k)
+        *reinterpret_cast<R*>(reinterpret_cast<char*>(fdst + k * B) + at) =
+            C::encs(g[k], k, key, Kc);
+      if (write_mom) {
+        mdst[cell] = rho;
+        mdst[L.plane + cell] = ux;
+        mdst[2 * L.plane + cell] = uy;
+      }
+    }
+    ++i;
+    a3 = a3 == 2 ? 0 : a3 + 1;
+    a4 = (a4 + 1) & 3;
+  };
+  auto barriers = [&](int n) {
+#pragma unroll 1
+    for (int q = 0; q < n; ++q) workgroup_barrier();
+  };
+  // The first step: rows from the lattice, in two sets of registers.  Where
+  // storage and compute type agree a row is computed in its set while the next
+  // row's loads fill the other; 16-bit rows are decoded first and their set
+  // takes the row after the next.  (More rows in flight: no faster.)  Every
+  // row fetches, the last ones the last row again, and nothing here stores to
+  // memory, so that the compiler can wait for one row and leave the later one
+  // in flight: in a loop that all steps shared it waited for all loads, and
+  // copied each row (us per step before / after: FP64 8192x2048 149 / 142,
+  // 4096x1024 MRT + Guo 62.5 / 57, FP32 4096x1024 MRT + Guo 28.6 / 24.4,
+  // 2999x1111 17.2 / 16.5; FP32 8192x2048 72 / 74).
+  auto first = [&](auto stores) {
+    constexpr bool SAME = std::is_same<R, T>::value;
+    constexpr int AHEAD = SAME ? 1 : 2;
+    R raw[2][9];
+    const int last = i + count - 1;
+#pragma unroll
+    for (int q = 0; q < AHEAD; ++q) fetch(raw[q], min(i + q, last));
+    auto row = [&](auto set) {
+      constexpr int u = decltype(set)::value;
+      T apart[9];
+      T (&g)[9] = values_of(raw[u], apart);
+      if constexpr (!SAME) {
+#pragma unroll
+        for (int k = 0; k < 9; ++k) g[k] = C::dec(raw[u][k], k, Kc);
+      }
+      fetch(raw[SAME ? 1 - u : u], min(i + AHEAD, last));
+      if (lo == 2) {
+        const T b4 = wave_from_prev(g[4]), b7 = wave_from_prev(g[7]), b8 = wave_from_prev(g[8]);
+        if (wall_lo) {
+          g[2] = b4;
+          g[5] = b7;
+          g[6] = b8;
+        }
+      }
+      if (hi == 2) {
+        const T b2 = wave_from_next(g[2]), b5 = wave_from_next(g[5]), b6 = wave_from_next(g[6]);
+        if (wall_hi) {
+          g[4] = b2;
+          g[7] = b5;
+          g[8] = b6;
+        }
+      }
+      finish(g, stores);
+      workgroup_barrier();
+    };
+    // no way out between the rows of a turn: with one the compiler moves the
+    // sets at the loop's end, and waits for them
+    int left = count;
+#pragma unroll 1
+    for (; left > 1; left -= 2) {
+      row(std::integral_constant<int, 0>{});
+      row(std::integral_constant<int, 1>{});
+    }
+    if (left > 0) row(std::integral_constant<int, 0>{});
+    barriers(total - count);
+  };
+  // The steps after it.
+  auto later = [&]() {
+    barriers(begin);
+#pragma unroll 1
+    for (int t = 0; t < count; ++t) {
+      T g[9];
+      // rows i (number n + 1 of the step before), i + 1 (n + 2), i - 1 (n)
+      const int same = (a3 == 2 ? 0 : a3 + 1) * 3;
+      const int next = RING_B + (a3 == 0 ? 2 : a3 - 1) * 3;
+      const T* const r0 = from + same * PITCH;
+      const T* const rb = from + next * PITCH;
+      const T* const rc = from + (RING_C + a4 * 3) * PITCH;
+#pragma unroll
+      for (int k = 0; k < 9; ++k)
+        g[k] = (CX[k] == 0 ? r0 : CX[k] < 0 ? rb : rc)[SLOT[k] * PITCH - CY[k]];
+      if ((lo | hi) && (wall_lo || wall_hi)) {
+        const T* const own_b = from + (RING_B + same) * PITCH;
+        const T* const own_c = from + (RING_C + ((a4 + 1) & 3) * 3) * PITCH;
+#pragma unroll
+        for (int k = 1; k < 9; ++k) {
+          if (CY[k] == 0 || (CY[k] == 1 ? !wall_lo : !wall_hi)) continue;
+          const int o = INV[k];
+          g[k] = zg ? (CX[k] == 0 ? r0 : CX[k] < 0 ? rb : rc)[SLOT[k] * PITCH]
+                    : (CX[o] == 0 ? r0 : CX[o] < 0 ? own_b : own_c)[SLOT[o] * PITCH];
+        }
+      }
+      finish(g, std::true_type{});
+      workgroup_barrier();
+    }
+    barriers(total - begin - count);
+  };
+  // every wave passes `total` barriers, in whichever loop
+  if (st > K)
+    barriers(total);
+  else if (st > 1)
+    later();
+  else if (K > 1)
+    first(std::false_type{});
+  else
+    first(std::true_type{});
 }
 
 // Waves per SIMD the registers must allow: the rings of three FP64 chunks

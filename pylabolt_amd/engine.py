@@ -720,7 +720,7 @@ _STRIP_SLOTS = {8: 768, 4: 1536}
 _STRIP_TILE_SHARE = 0.12
 
 
-def strip_rows(lengths, double, rounds=False):
+def strip_rows(lengths, double, rounds=False, most=160):
     """Rows of a strip-sweep chunk for runs of ``lengths`` rows, or None where
     the sweep does not pay.
 
@@ -735,13 +735,19 @@ def strip_rows(lengths, double, rounds=False):
     sweep is as fast (us per step strips / tiled: FP32 900x900 7.0 / 7.7, FP64
     700x700 9.6 / 9.7, 1024x1024 14.4 / 16.7), below 20 with ``rounds``, 16-bit storage
     that rounds every step (BF16 1100x1100 11.5 / 11.1, 1300x1300 13.5 /
-    14.8)."""
+    14.8).
+
+    ``most``: FP32 without a force is light enough in arithmetic to be bound by
+    memory, and neighbouring strips that drift apart in long chunks no longer
+    share cache lines (8192x2048: 74.6 us per step with 24 rows, 84 with 96,
+    4413x1904 42.8 and 45.5), while FP64 and forced FP32 gain from few chunk
+    ends (FP64 8192x2048 156 and 142, forced FP32 97 and 88)."""
     if lengths.size == 0:
         return None
     slots = _STRIP_SLOTS[8 if double else 4]
     if lengths.sum() < slots * (20 if rounds else 12 if double else 9):
         return None
-    rows = np.arange(8, 161)
+    rows = np.arange(8, most + 1)
     n = np.maximum(1, np.rint(lengths[:, None] / rows))
     longest = np.ceil(lengths[:, None] / n).max(axis=0)
     full, last = np.divmod(n.sum(axis=0), slots)
@@ -1075,14 +1081,13 @@ class D2Q9Engine:
         sweep were asked for; ``_round_last``: it then rounds 16-bit values
         at the last step of a launch only.
 
-        The two-step sweep keeps small lattices that ask for it (by
-        default none) and, of those without a rim, 16-bit ones and MRT in
-        FP64 below 8 M cells: us per step against the strips', FP16
-        4096x1024 27.6 / 29.8, BF16 2048x1024 13.4 / 14.1, FP64 MRT 2048x1024
-        34 / 39, 4096x1024 63 / 69, 8192x2048 240 / 223, but BGK 4096x1024 65
-        / 63 and FP32 4096x1024 36 / 30.  With a rim its kernels, fork and
-        join cost more: FP64 1371x1362 forced 36 / 28, 3001x1333 75 / 66,
-        FP16 8192x2048 90 / 73, BF16 900x700 14.3 / 6.1 (tiled)."""
+        The two-step sweep keeps FP64 and FP32 lattices that ask for it and
+        are too small for strips, and those without tables.  us per step
+        two-step / strips, without a rim: FP64 MRT 2048x1024 34 / 35,
+        4096x1024 62 / 58, 8192x2048 240 / 203, FP32 4096x1024 36 / 26, FP16
+        4096x1024 28.9 / 27.5, BF16 2048x1024 13.2 / 12.6; with one (two more
+        kernels, a fork and a join): FP64 3001x1333 75 / 61, 1371x1362 36 /
+        24, FP16 8192x2048 90 / 73, BF16 900x700 14.3 / 6.1 (tiled)."""
         self._split = None
         if self._codes is not None:
             shape = [ctypes.c_int32() for _ in range(3)]
@@ -1093,16 +1098,13 @@ class D2Q9Engine:
             split = self.tables.strip_split(
                 *self._strip_shape, functools.partial(
                     strip_rows, double=bits == 64,
-                    rounds=bits == 16 and not self._two_step_req))
+                    rounds=bits == 16 and not self._two_step_req,
+                    most=32 if bits == 32 and self.forcing is None else 160))
             if split is not None and split[2] <= _STRIP_TILE_SHARE:
                 self._split = split
         half = self.raw_dtype.itemsize == 2
-        rimless = self._rimless()
-        keep = rimless and self.nx * self.ny < 1 << 23 and (
-            half or (self.storage == nt.STORE_F64 and self.model == "MRT"))
         self._several = not self._two_step_req or (
-            self._codes is not None and not keep and
-            (self._split is not None or (half and not rimless)))
+            self._codes is not None and (self._split is not None or half))
         self._round_last = half and self._two_step_req and self._several
 
     def _setup_tiled(self):

@@ -213,3 +213,4 @@ def test_strip_rows_rule():
         slots = 768 if double else 1536
         assert 0.85 * slots < n <= slots
     assert 40 <= rows(8192, 37, True) <= 160
+    assert rows(8192, 37, False, most=32) <= 32

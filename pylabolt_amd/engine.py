@@ -720,6 +720,13 @@ _STRIP_SLOTS = {8: 768, 4: 1536}
 _STRIP_TILE_SHARE = 0.12
 
 
+def strip_least(double, rounds=False):
+    """Rows in all strips below which the strip sweep does not pay (see
+    ``strip_rows``)."""
+    return _STRIP_SLOTS[8 if double else 4] * (20 if rounds else
+                                               12 if double else 9)
+
+
 def strip_rows(lengths, double, rounds=False, most=160):
     """Rows of a strip-sweep chunk for runs of ``lengths`` rows, or None where
     the sweep does not pay.
@@ -742,10 +749,8 @@ def strip_rows(lengths, double, rounds=False, most=160):
     share cache lines (8192x2048: 74.6 us per step with 24 rows, 84 with 96,
     4413x1904 42.8 and 45.5), while FP64 and forced FP32 gain from few chunk
     ends (FP64 8192x2048 156 and 142, forced FP32 97 and 88)."""
-    if lengths.size == 0:
-        return None
     slots = _STRIP_SLOTS[8 if double else 4]
-    if lengths.sum() < slots * (20 if rounds else 12 if double else 9):
+    if lengths.sum() < strip_least(double, rounds):
         return None
     rows = np.arange(8, most + 1)
     n = np.maximum(1, np.rint(lengths[:, None] / rows))
@@ -1095,11 +1100,15 @@ class D2Q9Engine:
                 *[ctypes.byref(v) for v in shape]), "d2q9_strip_shape")
             self._strip_shape = tuple(v.value for v in shape)
             bits = 8 * self.raw_dtype.itemsize
-            split = self.tables.strip_split(
-                *self._strip_shape, functools.partial(
-                    strip_rows, double=bits == 64,
-                    rounds=bits == 16 and not self._two_step_req,
-                    most=32 if bits == 32 and self.forcing is None else 160))
+            rounds = bits == 16 and not self._two_step_req
+            split = None
+            if self.nx * -(-self.ny // self._strip_shape[1]) >= strip_least(
+                    bits == 64, rounds):
+                split = self.tables.strip_split(
+                    *self._strip_shape, functools.partial(
+                        strip_rows, double=bits == 64, rounds=rounds,
+                        most=32 if bits == 32 and self.forcing is None
+                        else 160))
             if split is not None and split[2] <= _STRIP_TILE_SHARE:
                 self._split = split
         half = self.raw_dtype.itemsize == 2

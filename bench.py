@@ -344,19 +344,20 @@ def sweep_rate(engine, bpc, ms_step, cells):
     strip sweep moves bpc per cell and launch, a two-step launch bpc per deep
     cell and 2 bpc per rim cell."""
     single = bpc * cells / (ms_step * 1e-3) / 1e9
+    sweep = engine.sweep
     n = None
-    if engine.strips is not None:
+    if sweep == "strips":
         n, kind = engine.strip_steps, "d2q9_strip_steps (k_strip)"
-    elif engine.tiled is not None:
+    elif sweep == "tiled":
         n, kind = engine.tiled.steps, "d2q9_tiled_steps (k_tiled)"
     if n is not None:
         return bpc * cells / (n * ms_step * 1e-3) / 1e9, single, {
             "launch": f"{kind}, {n} steps per launch",
-            "kind": "strips" if engine.strips is not None else "tiled",
+            "kind": sweep,
             "steps_per_launch": n,
             "algorithmic_bytes_per_launch": bpc * cells,
             "launch_us": n * ms_step * 1e3}
-    if not engine.two_step:
+    if sweep == "single":
         return single, single, None
     deep = int(round(engine.deep_fraction * cells))
     rim = cells - deep
@@ -374,8 +375,8 @@ def sweep_rate(engine, bpc, ms_step, cells):
 def run_form(sim, storage, steps, warmup, tile, use_graph=True):
     """Time ``steps`` steps of ``sim`` in one storage form after ``warmup``
     steps.  Every form asks for two steps per sweep, which in 16-bit storage
-    lets any sweep of several steps round the last one only (FP64 and FP32
-    give the same bits through every sweep)."""
+    keeps the first of a pair in FP32 (FP64 and FP32 give the same bits
+    through every sweep)."""
     from pylabolt_amd.solvers.fluidLB import Solver
     solver = Solver(simulation=sim, storage=storage, tile=tile,
                     graph_steps=graph_steps_for(steps), verbose=False,

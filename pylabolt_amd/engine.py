@@ -822,14 +822,15 @@ class D2Q9Engine:
     interior (d2q9_fused_step2) when deep tiles fit; by default for FP64
     and FP32 storage when the two population buffers exceed
     ``TWO_STEP_MIN_BYTES`` and they cover the lattice (the results are
-    bitwise those of single steps), for 16-bit storage only when asked (it
-    then rounds the stored step of a launch only, which changes the
-    numerics).  Where the strip or tiled sweep is the faster one it runs
-    instead, to the same rounding (``_choose_sweep``).  Otherwise steps go through the strip sweep on large
-    lattices (d2q9_strip_steps) and the tiled sweep on others
+    bitwise those of single steps), for 16-bit storage only when asked (its
+    intermediate step stays in FP32, which changes the rounding).  FP64 and
+    FP32 lattices large enough for the strip sweep take that instead, to the
+    same bits (``_choose_sweep``).  Otherwise steps go through the strip sweep
+    on large lattices (d2q9_strip_steps) and the tiled sweep on others
     (d2q9_tiled_steps), several steps per launch and bitwise single steps in
     every storage form, or through single sweeps where the case cannot be
-    expressed in their tables or a solid moves.
+    expressed in their tables or a solid moves.  ``sweep`` names the one that
+    runs.
     """
 
     def __init__(self, nx, ny, solid_pad, density, velocity, elements,
@@ -1083,16 +1084,16 @@ class D2Q9Engine:
     def _choose_sweep(self):
         """``_split``: the strip sweep's chunks and tiles, where it pays;
         ``_several``: the strip or tiled sweep runs even where two steps per
-        sweep were asked for; ``_round_last``: it then rounds 16-bit values
-        at the last step of a launch only.
+        sweep were asked for.
 
-        The two-step sweep keeps FP64 and FP32 lattices that ask for it and
-        are too small for strips, and those without tables.  us per step
-        two-step / strips, without a rim: FP64 MRT 2048x1024 34 / 35,
-        4096x1024 62 / 58, 8192x2048 240 / 203, FP32 4096x1024 36 / 26, FP16
-        4096x1024 28.9 / 27.5, BF16 2048x1024 13.2 / 12.6; with one (two more
-        kernels, a fork and a join): FP64 3001x1333 75 / 61, 1371x1362 36 /
-        24, FP16 8192x2048 90 / 73, BF16 900x700 14.3 / 6.1 (tiled)."""
+        The two-step sweep keeps lattices that ask for it and are in 16-bit
+        storage or too small for strips, and those without tables.  us per
+        step two-step / strips, without a rim: FP64 MRT 2048x1024 34 / 35,
+        4096x1024 62 / 58, 8192x2048 240 / 203, FP32 4096x1024 36 / 26; with
+        one (two more kernels, a fork and a join): FP64 3001x1333 75 / 61,
+        1371x1362 36 / 24.  In 16-bit storage the sweep decides what is
+        rounded: the two-step sweep every second step (in the rim every
+        step), which no other one gives."""
         self._split = None
         if self._codes is not None:
             shape = [ctypes.c_int32() for _ in range(3)]
@@ -1100,7 +1101,7 @@ class D2Q9Engine:
                 *[ctypes.byref(v) for v in shape]), "d2q9_strip_shape")
             self._strip_shape = tuple(v.value for v in shape)
             bits = 8 * self.raw_dtype.itemsize
-            rounds = bits == 16 and not self._two_step_req
+            rounds = bits == 16
             split = None
             if self.nx * -(-self.ny // self._strip_shape[1]) >= strip_least(
                     bits == 64, rounds):
@@ -1111,19 +1112,19 @@ class D2Q9Engine:
                         else 160))
             if split is not None and split[2] <= _STRIP_TILE_SHARE:
                 self._split = split
-        half = self.raw_dtype.itemsize == 2
         self._several = not self._two_step_req or (
-            self._codes is not None and (self._split is not None or half))
-        self._round_last = half and self._two_step_req and self._several
+            self._split is not None and self.raw_dtype.itemsize != 2)
 
     def _setup_tiled(self):
         """Tables of the tiled sweep on the device, where the lattice takes
-        it."""
+        it.  A 16-bit lattice that runs the two-step sweep has them too: for
+        its single steps, and for all steps where that sweep goes."""
         self.tiled = None
         self._tiled_arrays = None
         t, tables = self.tables, self._codes
         self._codes = None
-        if tables is None or (self.two_step and not self._several):
+        if tables is None or (self.two_step and not self._several and
+                              self.raw_dtype.itemsize != 2):
             return
         cells, codes, has_vel, has_pres = tables
         rows, width, steps = tiled_shape(
@@ -1137,13 +1138,18 @@ class D2Q9Engine:
         D.rows, D.width, D.steps = rows, width, steps
         D.n_elems = len(t.elems)
         D.has_vel, D.has_pres = int(has_vel), int(has_pres)
-        D.round_last = int(self._round_last and self.two_step)
+        D.round_last = self._round_last()
         D.cells, D.codes = dev["cells"].data_ptr(), dev["codes"].data_ptr()
         self._tiled_arrays = dev
         self._tiled_solid = np.flatnonzero(
             (t.flags_pad & nt.CELL_SOLID).ravel())
         self.tiled = D
         self._tiled_p = ctypes.byref(D)
+
+    def _round_last(self):
+        """D.round_last: 16-bit lattices asked for two steps per sweep round
+        the stored step of a launch only."""
+        return int(self.two_step and self.raw_dtype.itemsize == 2)
 
     def _setup_strips(self, rows=None):
         """Lists of the strip sweep on the device, where a lattice with
@@ -1228,7 +1234,7 @@ class D2Q9Engine:
         if self.two_step:
             self._setup_two_step()
         if self.tiled is not None:
-            self.tiled.round_last = int(self._round_last and self.two_step)
+            self.tiled.round_last = self._round_last()
 
     # ---- layout helpers -------------------------------------------------
     def _upload_plane(self, pad, dtype, count=1):
@@ -1267,7 +1273,7 @@ class D2Q9Engine:
             # the tiled and strip sweeps are for solids at rest
             self.tiled = self.strips = None
             if self._several and self.two_step:
-                self._several = self._round_last = False
+                self._several = False
                 self._setup_two_step()
         with torch.cuda.stream(self.stream):
             m = self._mom_from_host(self._init_density, self._init_velocity)
@@ -1296,6 +1302,16 @@ class D2Q9Engine:
             self.close()
         except Exception:
             pass
+
+    @property
+    def sweep(self):
+        """The sweep that ``advance`` takes: "strips", "tiled", "two-step" or
+        "single"."""
+        if self.two_step and not self._several:
+            return "two-step"
+        if self.tiled is None:
+            return "single"
+        return "strips" if self.strips is not None else "tiled"
 
     # ---- kernels --------------------------------------------------------
     def _collide(self, src, dst, write_mom):
@@ -1326,10 +1342,11 @@ class D2Q9Engine:
     def step2(self, write_moments=False):
         """Advance two reference time steps, with the two-step sweep where
         the lattice takes it."""
-        if self.tiled is not None:
+        sweep = self.sweep
+        if sweep in ("strips", "tiled"):
             self.advance(2, write_moments)
             return
-        if self.i_pop_new is not None:
+        if self.i_pop_new is not None or sweep == "single":
             self.step()
             self.step(write_moments)
             return
@@ -1367,13 +1384,14 @@ class D2Q9Engine:
         n = int(n)
         if n <= 0:
             return
-        if self.tiled is not None:
-            if self.strips is not None and self.i_pop_new is not None:
+        sweep = self.sweep
+        if sweep in ("strips", "tiled"):
+            if sweep == "strips" and self.i_pop_new is not None:
                 self.step(write_moments and n == 1)
                 n -= 1
             if n == 1:
                 self.step(write_moments)
-            elif n > 1 and self.strips is not None:
+            elif n > 1 and sweep == "strips":
                 self._advance_strips(n, write_moments)
             elif n > 1:
                 self._advance_tiled(n, write_moments)
@@ -1381,7 +1399,7 @@ class D2Q9Engine:
         if self.i_pop_new is not None:
             self.step(write_moments and n == 1)
             n -= 1
-        if self.two_step:
+        if sweep == "two-step":
             # pairs of steps: graphs of graph_steps steps, the last pair
             # eager when it has to store the moments
             keep = 2 if write_moments else 0
@@ -1413,7 +1431,7 @@ class D2Q9Engine:
         """Capture (once) the graph that ``advance`` replays from the
         current buffer roles, without running it; a timed region that
         follows then replays graphs only."""
-        if self.i_pop_new is None and self.tiled is None:
+        if self.i_pop_new is None and self.sweep in ("two-step", "single"):
             full = self.mom_full
             self._graph_for_state()
             self.mom_full = full
@@ -1435,9 +1453,9 @@ class D2Q9Engine:
         nt.check(self.lib.d2q9_graph_begin(self._stream_ptr), "graph begin")
         err = None
         src = start
-        for _ in range(self.graph_steps // 2 if self.two_step
-                       else self.graph_steps):
-            if self.two_step:
+        pairs = self.sweep == "two-step"
+        for _ in range(self.graph_steps // 2 if pairs else self.graph_steps):
+            if pairs:
                 rc = self.lib.d2q9_fused_step2(
                     self._Lp, self._rim_ap, self._rim_bp,
                     nt.ptr(self._deep["deep"]), nt.ptr(self._deep["walls"]),

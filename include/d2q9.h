@@ -246,7 +246,9 @@ int d2q9_fused_step(const d2q9_lattice* L, const void* f_src, void* f_dst,
  * auxiliary stream, forked and joined as for d2q9_fused_step; when both rim
  * descriptors list no tile and no fix-up cell, the deep tiles alone run on
  * `stream`, with no fork and join.  All three population buffers and all
- * three moment buffers must differ. */
+ * three moment buffers must differ.  mom_tmp must hold what mom_src holds on
+ * cells that are not fluid: the rim's second step takes the velocities of
+ * solids from it, and kernels write moments of fluid cells only. */
 int d2q9_fused_step2(const d2q9_lattice* L, const d2q9_lattice* L_rim_a,
                      const d2q9_lattice* L_rim_b, const int32_t* deep_tiles,
                      const uint8_t* deep_walls, int32_t n_deep, const void* f_src,

@@ -1283,8 +1283,11 @@ class D2Q9Engine:
                                        nt.ptr(self.f[1]), nt.ptr(self.mom[0]),
                                        self._stream_ptr), "d2q9_init_eq")
         if hasattr(self, "f_tmp"):
+            # the second step of a pair reads the velocities of solids from
+            # mom_tmp, where kernels write fluid cells only
             with torch.cuda.stream(self.stream):
                 self.f_tmp.copy_(self.f[0])
+                self.mom_tmp.copy_(self.mom[0])
         # both buffers hold pop_new[0] == pop[0]
         self.i_pop = 1
         self.i_pop_new = 0

@@ -960,15 +960,20 @@ class D2Q9Engine:
                        if min(self.nx, self.ny) >= 2 and
                        self.f[0].numel() * self.f[0].element_size() < 1 << 32
                        else None)
+        # the two-step sweep with solids that move, which the tiled and strip
+        # sweeps do not take
+        self._two_step_moving = two_step
         if two_step is None:
             # FP64 and FP32 give the same bits either way; in 16-bit
             # storage the two-step sweep keeps the intermediate step in FP32
             # and so changes the numerics, which only an explicit request
             # may do
-            two_step = (self.storage in (nt.STORE_F64, nt.STORE_F32) and
-                        2 * self.f[0].numel() * self.f[0].element_size()
-                        > TWO_STEP_MIN_BYTES and
-                        (self._codes is None or self._rimless()))
+            self._two_step_moving = (
+                self.storage in (nt.STORE_F64, nt.STORE_F32) and
+                2 * self.f[0].numel() * self.f[0].element_size()
+                > TWO_STEP_MIN_BYTES)
+            two_step = self._two_step_moving and (self._codes is None or
+                                                  self._rimless())
         self._two_step_req = bool(two_step)
         self._choose_sweep()
         self.two_step = False
@@ -1272,8 +1277,8 @@ class D2Q9Engine:
                 self._init_velocity.reshape(-1, 2)[self._tiled_solid]):
             # the tiled and strip sweeps are for solids at rest
             self.tiled = self.strips = None
-            if self._several and self.two_step:
-                self._several = False
+            if self._several and self._two_step_moving:
+                self._several, self._two_step_req = False, True
                 self._setup_two_step()
         with torch.cuda.stream(self.stream):
             m = self._mom_from_host(self._init_density, self._init_velocity)

@@ -89,3 +89,16 @@ def test_solids_set_moving_after_the_engine_was_made():
     one = _solver("f64", False)
     one.advance(11)
     _same(s.engine, one.engine)
+
+
+def test_large_lattices_take_the_two_step_sweep_by_default():
+    default = _solver("f64", None, 1600, 1100).engine
+    small = _solver("f64", None).engine
+    half = _solver("bf16dev", None, 1600, 1100).engine
+    assert default.sweep == "two-step"
+    assert small.sweep == half.sweep == "single"
+    one = _solver("f64", False, 1600, 1100).engine
+    for n in (1, 6):
+        default.advance(n)
+        one.advance(n)
+    _same(default, one)

@@ -381,10 +381,8 @@ int d2q9_adjoint_steps(const d2q9_lattice* L, const d2q9_tiled_desc* D, int32_t 
 #define D2Q9_ADJ_ONE(FO, WV)                                                                   \
   case WV: {                                                                                   \
     auto kern = k_adjoint_tiled<FO, WV>;                                                       \
-    static const hipError_t limit =                                                            \
-        hipFuncSetAttribute(reinterpret_cast<const void*>(kern),                               \
-                            hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);           \
-    if ((e = limit) != hipSuccess) break;                                                      \
+    static PerDevice limit;                                                                    \
+    if ((e = tiled::allow_lds(limit, kern)) != hipSuccess) break;                              \
     hipLaunchKernelGGL(kern, grid, block, lds, s, *L, *D, tiles, ntj, n, rows, last_streamed,  \
                        ls, ld, m, mom_stride, su, gf);                                         \
     e = hipGetLastError();                                                                     \

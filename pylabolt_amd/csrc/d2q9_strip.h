@@ -310,10 +310,8 @@ hipError_t launch_one(const d2q9_lattice* L, const d2q9_tiled_desc* D, const d2q
                       const Launch& A) {
   using C = Codec<S>;
   auto kern = k_strip<S, MODEL, FORCING>;
-  static const hipError_t limit =
-      hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
-                          hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-  if (limit != hipSuccess) return limit;
+  static PerDevice limit;
+  if (const hipError_t e = tiled::allow_lds(limit, kern)) return e;
   size_t lds = ring_bytes<S>(A.K);
   if (P->n_tiles > 0) {
     const size_t t = tiled::lds_bytes(*D, (TILE + 2 * A.K) * TILE_W, sizeof(typename C::T));

@@ -27,6 +27,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include "d2q9_per_device.h"
 #include "d2q9_sweep.h"
 
 namespace d2q9 {
@@ -318,6 +319,19 @@ __global__ __launch_bounds__(MAX_CELLS, (waves_per_simd<S, FORCING>())) void k_t
 // a D2Q9_E_* code with the error text set.
 int check_desc(const d2q9_lattice* L, const d2q9_tiled_desc* D);
 
+// Lets a kernel have all LDS of a CU on the current device, where more than
+// 64 KB has to be asked for.
+template <typename K>
+hipError_t allow_lds(PerDevice& done, K* kern) {
+  int device = 0;
+  if (const hipError_t e = hipGetDevice(&device)) return e;
+  return static_cast<hipError_t>(done.once(device, [kern] {
+    return static_cast<int>(hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
+                                                hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                160 * 1024));
+  }));
+}
+
 // Arguments of one launch.
 struct Launch {
   int K, collide_first, write_mom;
@@ -339,10 +353,8 @@ template <int S, int MODEL, int FORCING, int W>
 hipError_t launch_one(const d2q9_lattice* L, const d2q9_tiled_desc* D, const Launch& A) {
   using C = Codec<S>;
   auto kern = k_tiled<S, MODEL, FORCING, W>;
-  static const hipError_t limit =
-      hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
-                          hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-  if (limit != hipSuccess) return limit;
+  static PerDevice limit;
+  if (const hipError_t e = allow_lds(limit, kern)) return e;
   // the region loses the rows a shorter launch does not need
   const int rows = D->rows - 2 * (D->steps - A.K);
   const int tr = rows - 2 * A.K, tc = W - 2 * A.K;

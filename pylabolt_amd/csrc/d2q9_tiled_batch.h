@@ -50,10 +50,8 @@ __global__ __launch_bounds__(MAX_CELLS, S == D2Q9_STORE_F64 ? 4 : 8) void k_tile
 template <int S, int W>
 hipError_t launch_batch_one(const BatchLaunch& A) {
   auto kern = k_tiled_batch<S, W>;
-  static const hipError_t limit =
-      hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
-                          hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-  if (limit != hipSuccess) return limit;
+  static PerDevice limit;
+  if (const hipError_t e = allow_lds(limit, kern)) return e;
   const int area = A.rows * W;
   const size_t lds = (size_t)((area * A.planes + 3) & ~3) * sizeof(typename Codec<S>::T) +
                      MAX_ELEMS * sizeof(d2q9_bc_elem);

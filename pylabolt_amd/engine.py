@@ -830,7 +830,8 @@ class D2Q9Engine:
     (d2q9_tiled_steps), several steps per launch and bitwise single steps in
     every storage form, or through single sweeps where the case cannot be
     expressed in their tables or a solid moves.  ``sweep`` names the one that
-    runs.
+    runs; the attribute ``two_step`` says that the two-step sweep was chosen
+    and deep tiles fit, also where the strips then take its place.
     """
 
     def __init__(self, nx, ny, solid_pad, density, velocity, elements,

@@ -121,9 +121,11 @@ class Solver:
         self.backend.create_engine(self.state, self.collision_operator,
                                    self.force_operator)
         eng = self.backend.engine
-        print_log(f"{'Engine':<10}: storage {eng.storage_name}, two-step "
-                  f"sweep {'on' if eng.two_step else 'off'}",
-                  0, self.verbose if verbose is None else verbose)
+        names = {"strips": "strip sweep", "tiled": "tiled sweep",
+                 "two-step": "two-step sweep", "single": "single steps"}
+        print_log(f"{'Engine':<10}: storage {eng.storage_name}, "
+                  f"{names[eng.sweep]}", 0,
+                  self.verbose if verbose is None else verbose)
         for op in (self.mpi_operator, self.collision_operator,
                    self.force_operator, self.compute_fields_operator,
                    self.streaming_operator, self.boundary_operator,

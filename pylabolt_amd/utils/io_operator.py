@@ -50,8 +50,10 @@ class InputOutputOperator:
         eng = getattr(self, "engine", None)
         if eng is not None:
             # not read by the reference's tools: how the run was computed
+            # (the sweep that runs, not the one asked for: in 16-bit storage
+            # the two-step sweep rounds every second step)
             meta["engine"] = {"storage": eng.storage_name,
-                              "two_step": bool(eng.two_step)}
+                              "two_step": eng.sweep == "two-step"}
         os.makedirs(self.field_save_path, exist_ok=True)
         with open(os.path.join(self.root, "metadata.json"), "w") as f:
             json.dump(meta, f, indent=4)

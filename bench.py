@@ -274,17 +274,15 @@ def batched_form(steps=5000, warmup=50, per_lattice_steps=100, n=256,
     """Batched workload: ``n`` seeded lattices (sizes uniform over the
     multiples of 32 in 64..1024 x 64..512, Re in [50, 400], even ids cavity
     BGK, odd ids Guo-forced channel MRT), FP32, several steps of all of them
-    per launch (``config``, the autotuner's choice, is for the persistent
-    kernel that takes batches the tiled sweep cannot).  Aggregate MLUPS = sum of cells * steps / t.  The same
+    per launch.  Aggregate MLUPS = sum of cells * steps / t.  The same
     lattices advanced one launch per lattice per step are timed beside it
     over ``per_lattice_steps`` steps."""
     import torch
     from pylabolt_amd import cases
-    from pylabolt_amd.batch import BatchAutotuner, BatchedLattices
+    from pylabolt_amd.batch import BatchedLattices
     sims = cases.batch_cases(n=n, seed=seed, steps=steps)
     t0 = time.perf_counter()
-    tuner = BatchAutotuner(reps=5)
-    batch = BatchedLattices(sims, storage="f32", tuner=tuner, graph_steps=50)
+    batch = BatchedLattices(sims, storage="f32", graph_steps=50)
     t_setup = time.perf_counter() - t0
     batch.advance(warmup)
     batch.synchronize()
@@ -318,9 +316,7 @@ def batched_form(steps=5000, warmup=50, per_lattice_steps=100, n=256,
         "mlups": mlups, "us_per_step": t / steps * 1e6,
         "achieved_gbs": achieved, "frac": achieved / PEAK_GBS,
         "steps_per_launch": batch.steps_per_launch,
-        "config": batch.config.as_dict(), "items_per_step": batch.n_items,
-        "tuner_candidates": len(tuner.trials),
-        "setup_and_tune_s": t_setup,
+        "tiles_per_launch": batch._tiled_count, "setup_s": t_setup,
         "per_lattice_launches_mlups": mlups_pl,
         "speedup_vs_per_lattice_launches": (mlups / mlups_pl
                                             if mlups_pl else None),

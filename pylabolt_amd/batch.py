@@ -150,9 +150,9 @@ class BatchedLattices:
 
     ``simulations``: case namespaces (the reference's ``simulation.py``
     dicts), each built into its own engine on one shared stream; they must
-    share the storage form (FP64 or FP32).  ``config``: a BatchConfig, or
-    None for the autotuner's choice (``tuner``, default a
-    BatchAutotuner with its cache).
+    share the storage form (FP64 or FP32).  ``config``: a BatchConfig of the
+    persistent kernel, or None for the autotuner's choice (``tuner``, or a
+    BatchAutotuner of its own once that kernel runs).
     """
 
     def __init__(self, simulations, storage="f32", config=None, tuner=None,
@@ -190,9 +190,16 @@ class BatchedLattices:
         self.cells = sum(e.nx * e.ny for e in self.engines)
         self._setup_tiled()
         self.config = None
+        # the tiled sweep uses no launch configuration: without a tuner given,
+        # tuning waits until the persistent kernel runs
+        self._tune_first = False
         if config is None:
-            tuner = tuner if tuner is not None else BatchAutotuner()
-            config = tuner.config_for(self)
+            if tuner is None and self.tiled:
+                self._tune_first = True
+                config = BatchConfig()
+            else:
+                tuner = tuner if tuner is not None else BatchAutotuner()
+                config = tuner.config_for(self)
         self.set_config(config)
 
     # ---- configuration ----------------------------------------------------
@@ -402,6 +409,9 @@ class BatchedLattices:
                 e.tiled is not None for e in self.engines):
             self._advance_tiled(n, write_moments)
             return
+        if self._tune_first and any(e.tiled is None for e in self.engines):
+            self._tune_first = False
+            self.set_config(BatchAutotuner().config_for(self))
         if fresh:
             # first step after initialisation: collide-only, per lattice
             for e in self.engines:

@@ -173,19 +173,24 @@ class CaseTables:
         zg_sides = {((0, 1), (2, 5, 6)): 0, ((0, -1), (4, 7, 8)): 1}
         bb_sides = {((0, 1), (2, 5, 6)): 2, ((0, -1), (4, 7, 8)): 3,
                     ((1, 0), (1, 5, 8)): 4, ((-1, 0), (3, 6, 7)): 5}
-        for (i, j), r in rules.items():
+
+        def wall_side(r):
             dirs = tuple(k for k in range(9) if r[k] & 15 != nt.RULE_STREAM)
             kinds = {r[k] & 15 for k in dirs}
             normals = {tuple(int(v) for v in self.elems[r[k] >> 4][1]["normal"])
                        for k in dirs}
             if len(kinds) != 1 or len(normals) != 1:
-                continue
+                return -1
             key = (normals.pop(), dirs)
-            kind = kinds.pop()
-            if kind == nt.RULE_ZG and key in zg_sides:
-                self.wall_side_pad[i, j] = zg_sides[key]
-            elif kind == nt.RULE_BB and key in bb_sides:
-                self.wall_side_pad[i, j] = bb_sides[key]
+            return {nt.RULE_ZG: zg_sides, nt.RULE_BB: bb_sides}.get(
+                kinds.pop(), {}).get(key, -1)
+
+        sides = {}      # the nodes of a wall have the same rules
+        for (i, j), r in rules.items():
+            r = tuple(r)
+            if r not in sides:
+                sides[r] = wall_side(r)
+            self.wall_side_pad[i, j] = sides[r]
         self.set_tile(tile_j, tile_i, solid_tiles)
 
     def set_tile(self, tile_j, tile_i, solid_tiles="sweep"):
@@ -345,60 +350,60 @@ class CaseTables:
         if len(self.elems) > nt.TILED_MAX_ELEMS:
             return None
         solid = (self.flags_pad & nt.CELL_SOLID) != 0
-        fluid = self.fluid_pad
-        special = fluid & ((self.flags_pad & (nt.CELL_NEAR_SOLID |
-                                              nt.CELL_BC)) != 0)
-        ii, jj = np.nonzero(special)
-        n = ii.size
+        flat = self.flags_pad.ravel()
+        # every special cell, and its place in the padded grid
+        at = np.flatnonzero((flat & (nt.CELL_NEAR_SOLID | nt.CELL_BC)) != 0)
+        at = at[self.fluid_pad.ravel()[at]]
+        n = at.size
         if n >= 1 << 24:
             return None
         cells = self.flags_pad.astype(np.uint32)
-        cells[ii, jj] |= np.arange(n, dtype=np.uint32) << np.uint32(8)
+        cells.ravel()[at] |= np.arange(n, dtype=np.uint32) << np.uint32(8)
         codes = np.zeros((max(1, n), 4), dtype=np.uint32)
-
-        def source(dr, dc, k):
-            return (dr + 1) | (dc + 1) << 2 | k << 4
-
-        bc = (self.flags_pad[ii, jj] & nt.CELL_BC) != 0
-        node = self.bc_slot_pad[ii, jj]
-        normal = np.array([[int(v) for v in e["normal"]]
-                           for _, e in self.elems] or [[0, 0]])
-        has_vel = has_pres = False
-        first = np.full(n, -1)
-        second = np.full(n, -1)
-        arith = np.zeros(n, dtype=np.int64)
-        for d in range(1, 9):
-            back = source(0, 0, int(INV[d]))
-            code = np.where(solid[ii - CX[d], jj - CY[d]], back,
-                            source(-CX[d], -CY[d], d))
-            rule = np.where(bc, self.bc_nodes[node, d].astype(np.int64), 0)
-            kind, elem = rule & 15, rule >> 4
-            moving = (kind == nt.RULE_VEL) | (kind == nt.RULE_PRES)
-            has_vel |= bool((kind == nt.RULE_VEL).any())
-            has_pres |= bool((kind == nt.RULE_PRES).any())
-            code = np.where((kind == nt.RULE_BB) | moving, back, code)
-            first = np.where(moving & (first < 0), elem, first)
-            other = moving & (elem != first)
-            if np.any(other & (second >= 0) & (second != elem)):
+        if n == 0:
+            return cells, codes, False, False
+        # one row per direction 1..8 from here on
+        cx, cy, inv = (v[1:, None] for v in (CX, CY, INV))
+        pull = cx * (self.ny + 2) + cy
+        back = 5 | inv << 4             # the cell itself, (0, 0)
+        solid = solid.ravel()
+        code = np.where(solid[at - pull], back,
+                        (1 - cx) | (1 - cy) << 2 | np.arange(1, 9)[:, None]
+                        << 4)
+        rule = self.bc_nodes[self.bc_slot_pad.ravel()[at], 1:9].T.astype(
+            np.int32)
+        rule[:, (flat[at] & nt.CELL_BC) == 0] = 0
+        kind, elem = rule & 15, rule >> 4
+        vel, pres = kind == nt.RULE_VEL, kind == nt.RULE_PRES
+        moving = vel | pres
+        code = np.where((kind == nt.RULE_BB) | moving, back, code)
+        each = np.arange(n)
+        first = elem[moving.argmax(axis=0), each]
+        other = moving & (elem != first)
+        second = elem[other.argmax(axis=0), each]
+        if np.any(other & (elem != second)):
+            return None
+        zd, zc = np.nonzero(kind == nt.RULE_ZG)
+        if zd.size:
+            normal = np.array([[int(v) for v in e["normal"]]
+                               for _, e in self.elems])
+            n0, n1 = normal[elem[zd, zc]].T
+            # the neighbour is interior, so its own are in range
+            nb = at[zc] + n0 * (self.ny + 2) + n1
+            if not self.fluid_pad.ravel()[nb].all():
                 return None
-            second = np.where(other, elem, second)
-            arith |= moving.astype(np.int64) << (d - 1)
-            arith |= other.astype(np.int64) << (d + 7)
-            zg = np.nonzero(kind == nt.RULE_ZG)[0]
-            if zg.size:
-                n0, n1 = normal[elem[zg]].T
-                bi, bj = ii[zg] + n0, jj[zg] + n1
-                if not fluid[bi, bj].all():
-                    return None
-                # the neighbour is interior, so its own are in range
-                code[zg] = np.where(solid[bi - CX[d], bj - CY[d]],
-                                    source(n0, n1, int(INV[d])),
-                                    source(n0 - CX[d], n1 - CY[d], d))
-            codes[:n, (d - 1) >> 2] |= code.astype(np.uint32) << np.uint32(
-                8 * ((d - 1) & 3))
-        arith |= np.maximum(first, 0) << 16 | np.maximum(second, 0) << 24
-        codes[:n, 2] = np.where(first >= 0, arith, 0)
-        return cells, codes, has_vel, has_pres
+            code[zd, zc] = np.where(
+                solid[nb - pull[zd, 0]],
+                (n0 + 1) | (n1 + 1) << 2 | inv[zd, 0] << 4,
+                (n0 - cx[zd, 0] + 1) | (n1 - cy[zd, 0] + 1) << 2 |
+                (zd + 1) << 4)
+        codes[:n, :2] = np.ascontiguousarray(code.T.astype(np.uint8)).view(
+            "<u4")
+        bit = np.arange(8)[:, None]
+        arith = ((moving << bit).sum(axis=0) | (other << (bit + 8)).sum(axis=0)
+                 | first << 16 | np.where(other.any(axis=0), second, 0) << 24)
+        codes[:n, 2] = np.where(moving.any(axis=0), arith, 0)
+        return cells, codes, bool(vel.any()), bool(pres.any())
 
     def strip_split(self, steps, cols, tile, chunk_rows):
         """Chunks and tiles of the strip sweep (d2q9_strip_steps).

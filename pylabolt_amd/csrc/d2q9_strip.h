@@ -16,7 +16,14 @@
 // Compared with a tile held in LDS, cells are computed twice only at the sides
 // of a strip (64 for 56 columns) and at the ends of a chunk, and loads,
 // arithmetic and stores of different rows overlap.  Per STEPS steps the lattice
-// is read about 1.15 times and written once.
+// is read 1.15 times in FP64 and about 1.45 in FP32 and 16 bits, and written 1.0
+// to 1.05 times (counters: FP64 8192x2048, FP32 2999x1111, BF16 4096x1024).
+//
+// What bounds it (same launches): FP64 without a force and FP32 HBM at 4.5 TB/s
+// and vector issue in 0.6 of the cycles at once; BF16 vector issue (0.77).
+// FP64 MRT + Guo, 4096x1024, is at neither limit, 2.6 TB/s and 0.51: 298
+// vector instructions per cell and step with the 12 waves per CU that the
+// rings leave room for.
 //
 // Chunks hold plain cells only, but for a straight zero-gradient or
 // bounce-back wall in the lattice's first or last column; every other cell

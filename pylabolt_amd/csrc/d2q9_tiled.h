@@ -116,16 +116,6 @@ __device__ __forceinline__ void apply_pres(const Consts<typename Codec<S>::T>& K
   }
 }
 
-// The two elements of a cell's arithmetic word: directions of each, and the
-// element's place.
-__device__ __forceinline__ uint32_t arith_mask(uint32_t a, int which) {
-  const uint32_t sel = (a >> 8) & 0xffu;
-  return (which ? sel : ~sel) & a & 0xffu;
-}
-__device__ __forceinline__ int arith_elem(uint32_t a, int which) {
-  return (int)((a >> (which ? 24 : 16)) & 0xffu);
-}
-
 // K steps of the output tile of (rows - 2 K) x tile_c cells from (i_first,
 // j_first) on, tile_c <= W - 2 K: region of `rows` x W cells, a wave holding 64 /
 // W rows, one cell per thread.  LDS element of direction k of region

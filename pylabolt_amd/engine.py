@@ -689,8 +689,8 @@ def tiled_shape(sizes, double, forced):
     several tiles compute; smaller regions spread a small lattice over more
     CUs.  The choice minimises a cost model (launch + steps + the waves of
     the busiest CU) over the regions of up to 1024 cells.  Against a sweep
-    of regions and steps on nine lattices from 128 x 128 to 4096 x 1024 it
-    picks the fastest region or one within 5 % of it, 14 % on one."""
+    of regions and steps on seven lattices from 128 x 128 to 1001 x 413 it
+    picks the fastest region or one within 4 % of it."""
     load, step, most = _TILED_COST[8 if double else 4, bool(forced)]
     best = None
     for width in (16, 32, 64):
@@ -1099,12 +1099,12 @@ class D2Q9Engine:
 
         The two-step sweep keeps lattices that ask for it and are in 16-bit
         storage or too small for strips, and those without tables.  us per
-        step two-step / strips, without a rim: FP64 MRT 2048x1024 34 / 35,
-        4096x1024 62 / 58, 8192x2048 240 / 203, FP32 4096x1024 36 / 26; with
-        one (two more kernels, a fork and a join): FP64 3001x1333 75 / 61,
-        1371x1362 36 / 24.  In 16-bit storage the sweep decides what is
-        rounded: the two-step sweep every second step (in the rim every
-        step), which no other one gives."""
+        step two-step / strips, without a rim: FP64 MRT 2048x1024 32.8 / 32.2,
+        4096x1024 59.5 / 55.5, 8192x2048 235 / 191, FP32 2048x1024 16.2 / 12.0,
+        4096x1024 34.6 / 25.4; with one (two more kernels, a fork and a join):
+        FP64 3001x1333 65 / 36, 1371x1362 36 / 20, FP32 22 / 9.  In 16-bit
+        storage the sweep decides what is rounded: the two-step sweep every
+        second step (in the rim every step), which no other one gives."""
         self._split = None
         if self._codes is not None:
             shape = [ctypes.c_int32() for _ in range(3)]

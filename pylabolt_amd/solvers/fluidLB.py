@@ -65,11 +65,11 @@ class Solver:
     graph chunk, the torch stream the engine runs on (a new one if None)
     how tiles holding solid cells are swept (``solid_tiles``: "sweep",
     "cells" or "auto"; None picks per storage form) and whether pairs of
-    steps run as one sweep over the deep interior (``two_step``; None and
-    False: not in 16-bit storage).  FP64 and FP32 lattices large enough for
-    the strip sweep take that whatever ``two_step`` says.  Every choice gives
-    bitwise the same results, but for ``two_step`` in 16-bit storage, whose
-    intermediate step stays in FP32.
+    steps run as one sweep over the deep interior (``two_step``; None: not in
+    16-bit storage).  FP64 and FP32 lattices large enough for the strip sweep
+    take that whatever ``two_step`` says, and smaller ones are faster without
+    it.  Every choice gives bitwise the same results, but for ``two_step`` in
+    16-bit storage, whose intermediate step stays in FP32.
     """
 
     def __init__(self, comm=None, backend="gpu", n_threads=None,

@@ -279,7 +279,13 @@ int d2q9_deep_rows(void);
  * type D2Q9_RULE_VEL, D2Q9_RULE_PRES.  n_elems (at most 32) boundary
  * elements are in bc_elems.  The solids must be at rest.  round_last: 16-bit
  * storage rounds only the last step of a launch and keeps the others in FP32
- * (not bitwise single steps any more: fewer roundings).
+ * (not bitwise single steps any more: fewer roundings).  pairs: 16-bit storage
+ * rounds as the two-step sweep does, in place of both.  1: every second step,
+ * counted from the first of the call, and the last.  2: so, but a cell with bit
+ * D2Q9_TILED_RIM in `cells` pulls values that were rounded after the first step
+ * of a pair too; every cell that such a cell pulls from, itself among them, has
+ * bit D2Q9_TILED_NEAR_RIM.  The steps of a launch are then even (but for the
+ * last), `steps` at least 2.
  *
  * The steps go f_a -> f_b -> f_a ... once per launch, ceil(n / steps)
  * launches (the last one's target holds the result), the moments alike.
@@ -288,10 +294,14 @@ int d2q9_deep_rows(void);
  * mom_steps + s * mom_stride elements, three planes each; mom_b is then not
  * written.  mom_a holds rho/u of the step before, as for d2q9_fused_step.
  */
+#define D2Q9_TILED_RIM 32u
+#define D2Q9_TILED_NEAR_RIM 64u
+
 typedef struct d2q9_tiled_desc {
   int32_t rows, width, steps;
   int32_t n_elems, has_vel, has_pres;
   int32_t round_last;
+  int32_t pairs;
   const uint32_t* cells;
   const uint32_t* codes;
 } d2q9_tiled_desc;
@@ -421,7 +431,7 @@ int d2q9_batched_step(const d2q9_batch_entry* entries,
 
 /*
  * Strip sweep: n fused steps, up to 4 per launch, as d2q9_tiled_steps (bitwise
- * single steps unless D asks for round_last).  d2q9_strip_shape gives the
+ * single steps unless D asks for round_last; pairs is refused).  d2q9_strip_shape gives the
  * most steps of a launch, a strip's output columns and a tile's output rows
  * and columns.
  *

@@ -102,7 +102,7 @@ class TiledDesc(ctypes.Structure):
     _fields_ = [("rows", ctypes.c_int32), ("width", ctypes.c_int32),
                 ("steps", ctypes.c_int32), ("n_elems", ctypes.c_int32),
                 ("has_vel", ctypes.c_int32), ("has_pres", ctypes.c_int32),
-                ("round_last", ctypes.c_int32),
+                ("round_last", ctypes.c_int32), ("pairs", ctypes.c_int32),
                 ("cells", ctypes.c_void_p), ("codes", ctypes.c_void_p)]
 
 
@@ -118,6 +118,8 @@ class StripDesc(ctypes.Structure):
                 ("chunks", ctypes.c_void_p), ("tiles", ctypes.c_void_p)]
 
 
+# bits of a cell in TiledDesc.cells beside its flags (TiledDesc.pairs == 2)
+TILED_RIM, TILED_NEAR_RIM = 32, 64
 # boundary elements a launch of the tiled sweep holds (d2q9_tiled_desc)
 TILED_MAX_ELEMS = 32
 

@@ -33,6 +33,7 @@ extern "C" int d2q9_strip_steps(const d2q9_lattice* L, const d2q9_tiled_desc* D,
   if (f_a == f_b || mom_a == mom_b)
     return sfail(D2Q9_E_ARG, "strip steps: the two buffers must differ");
   if (int r = tiled::check_desc(L, D)) return r;
+  if (D->pairs) return sfail(D2Q9_E_UNSUPPORTED, "strip steps: no rounding of pairs");
   if (n < 0 || P->n_tiles < 0 || P->n_chunks < 0 || (P->n_tiles > 0 && !P->tiles) ||
       (P->n_chunks > 0 && !P->chunks) || (int64_t)P->n_tiles + P->n_chunks > 0x7fffffff)
     return sfail(D2Q9_E_ARG, "strip steps: bad step count or lists");

@@ -17,13 +17,16 @@
 // arithmetic of their own, in the order of apply_bc.  Periodic sides are
 // images in the grown region.  The arithmetic per cell is that of the
 // single step and 16-bit storage rounds every step (the last of a launch
-// only, when asked), so the result is bitwise that of K single steps in every
-// storage form.
+// only, or as the two-step sweep, when asked), so the result is bitwise that of
+// K single steps in every storage form.
 //
 // What bounds it: for small lattices the latency of a launch (about 4 us
 // of load, collide, store and hand-over) which the K steps share; for larger
 // ones the work on the grown cells, (rows + 2K)(cols + 2K) / (rows cols) at
-// the first step.
+// the first step.  16-bit storage rounded in pairs (FP16 cylinder 900x700 7.4 us
+// per step; 14.5 by the two-step sweep): where there is a rim, a second copy of
+// the nine values in LDS, rounded after the first step of a pair in the cells
+// that a rim cell pulls from, leaves two workgroups of 1024 cells per CU.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -37,9 +40,10 @@ constexpr int MAX_ELEMS = 32;
 constexpr int MAX_CELLS = 1024;   // of a region, one per thread
 
 // Planes of LDS values besides the nine populations: rho where a cell is a
-// moving wall's, u where one is at fixed pressure.
+// moving wall's, u where one is at fixed pressure, and the rounded populations
+// for the rim's cells (pairs == 2).
 __host__ __device__ inline int lds_planes(const d2q9_tiled_desc& D) {
-  return 9 + (D.has_vel ? 1 : 0) + (D.has_pres ? 2 : 0);
+  return 9 + (D.has_vel ? 1 : 0) + (D.has_pres ? 2 : 0) + (D.pairs == 2 ? 9 : 0);
 }
 __host__ __device__ inline int lds_values(const d2q9_tiled_desc& D, int area) {
   return (area * lds_planes(D) + 3) & ~3;
@@ -140,6 +144,7 @@ __device__ __forceinline__ void run_tile(
   T* const s = reinterpret_cast<T*>(smem);
   T* const srho = s + 9 * area;
   T* const su = srho + (D.has_vel ? area : 0);
+  T* const srim = su + (D.has_pres ? 2 * area : 0);   // as s, 16-bit rims only
   d2q9_bc_elem* const elems = reinterpret_cast<d2q9_bc_elem*>(s + lds_values(D, area));
   const Consts<T> Kc = load_consts<T>(L);
   const int i0 = i_first - K, j0 = j_first - K;   // the region's first cell
@@ -157,7 +162,10 @@ __device__ __forceinline__ void run_tile(
   uint32_t from[4] = {};    // special cells: LDS elements to read, two a word
   uint32_t arith = 0;       // special cells: directions with arithmetic
   T ffx = (T)0, ffy = (T)0;
-  const bool each = sizeof(R) == 2 && !D.round_last;   // every step is rounded
+  // 16-bit storage: every step is rounded, or every second one
+  const bool each = sizeof(R) == 2 && !D.round_last && !D.pairs;
+  const bool pairs = sizeof(R) == 2 && D.pairs != 0;
+  bool rim = false, near_rim = false;
   {
     const int r = e / W, c = e % W;
     int i = i0 + r, j = j0 + c;
@@ -190,6 +198,10 @@ __device__ __forceinline__ void run_tile(
       if (info & D2Q9_CELL_FLUID) {
         depth = min(min(r, rows - 1 - r), min(c, W - 1 - c));
         keep = (info & D2Q9_CELL_STORE_MOM) != 0;
+        if (sizeof(R) == 2 && D.pairs == 2) {
+          rim = (info & D2Q9_TILED_RIM) != 0;
+          near_rim = (info & D2Q9_TILED_NEAR_RIM) != 0;
+        }
         if (FORCING != D2Q9_FORCING_NONE && L.force_source == D2Q9_FSRC_FIELD) {
           const T* ff = static_cast<const T*>(L.force_field);
           ffx = ff[cell];
@@ -209,6 +221,11 @@ __device__ __forceinline__ void run_tile(
       }
 #pragma unroll
       for (int k = 0; k < 9; ++k) s[e * 9 + k] = C::dec(raw[k], k, Kc);
+      if (sizeof(R) == 2 && D.pairs == 2) {
+        // cells that are not fluid keep these
+#pragma unroll
+        for (int k = 0; k < 9; ++k) srim[e * 9 + k] = C::dec(raw[k], k, Kc);
+      }
     }
     own = own && depth >= K;
   }
@@ -221,7 +238,8 @@ __device__ __forceinline__ void run_tile(
 #pragma unroll
         for (int k = 0; k < 9; ++k) g[k] = s[e * 9 + k];
       } else {
-        const T* const p = s + (e - W - 1) * 9;   // the cell's neighbourhood
+        // the cell's neighbourhood
+        const T* const p = (rim && !(st & 1) ? srim : s) + (e - W - 1) * 9;
         g[0] = p[(W + 1) * 9];
         if (from[0] == 0) {
 #pragma unroll
@@ -255,8 +273,14 @@ __device__ __forceinline__ void run_tile(
     collide<T, MODEL, FORCING, C::dev>(g, Kc, drho, rho, ux, uy, fx, fy, px, py);
     const uint32_t key = sizeof(R) == 2 ? cell_key((uint32_t)cell) : 0u;
     if (st < K) {
+      const bool round = each || (pairs && !(st & 1));
 #pragma unroll
-      for (int k = 0; k < 9; ++k) s[e * 9 + k] = each ? through_storage<S>(g[k], k, key, Kc) : g[k];
+      for (int k = 0; k < 9; ++k)
+        s[e * 9 + k] = round ? through_storage<S>(g[k], k, key, Kc) : g[k];
+      if (near_rim && (st & 1)) {
+#pragma unroll
+        for (int k = 0; k < 9; ++k) srim[e * 9 + k] = through_storage<S>(g[k], k, key, Kc);
+      }
       if (keep) {
         if (D.has_vel) srho[e] = rho;
         if (D.has_pres) {

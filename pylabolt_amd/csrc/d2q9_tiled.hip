@@ -19,6 +19,8 @@ int d2q9::tiled::check_desc(const d2q9_lattice* L, const d2q9_tiled_desc* D) {
   if (D->steps < 1 || (D->width != 16 && D->width != 32 && D->width != 64) ||
       2 * (int64_t)D->steps >= D->width || 2 * (int64_t)D->steps >= D->rows)
     return tfail(D2Q9_E_ARG, "tiled sweep: bad region or step count");
+  if (D->pairs < 0 || D->pairs > 2 || (D->pairs && D->steps < 2))
+    return tfail(D2Q9_E_ARG, "tiled sweep: bad pairs");
   if (D->n_elems < 0 || D->n_elems > tiled::MAX_ELEMS || (D->n_elems > 0 && !L->bc_elems) ||
       !D->cells || !D->codes)
     return tfail(D2Q9_E_ARG, "tiled sweep: bad special-cell tables");
@@ -44,10 +46,12 @@ extern "C" int d2q9_tiled_steps(const d2q9_lattice* L, const d2q9_tiled_desc* D,
   if (int r = tiled::check_desc(L, D)) return r;
   const size_t elem = L->storage == D2Q9_STORE_F64 ? 8 : 4;
   if (n == 0) return 0;
-  // launches of nearly equal length: the work on grown cells rises with the
-  // steps of a launch
-  const int launches = (n + D->steps - 1) / D->steps;
-  const int base = n / launches, longer = n % launches;
+  // launches of nearly equal length (the work on grown cells rises with their
+  // steps; whole pairs of them where pairs are rounded, a single step left over
+  // in the last launch, which has room for it)
+  const int unit = D->pairs ? 2 : 1, most = D->steps / unit * unit;
+  const int launches = n / most + (n % most != 0);
+  const int base = n / unit / launches, longer = n / unit % launches;
   void* f[2] = {f_a, f_b};
   void* m[2] = {mom_a, mom_b};
   char* const per_step = static_cast<char*>(mom_steps);
@@ -58,7 +62,7 @@ extern "C" int d2q9_tiled_steps(const d2q9_lattice* L, const d2q9_tiled_desc* D,
   A.mom_stride = mom_stride;
   int done = 0;
   for (int a = 0; a < launches; ++a) {
-    A.K = base + (a < longer ? 1 : 0);
+    A.K = unit * (base + (a < longer ? 1 : 0)) + (a == launches - 1 ? n % unit : 0);
     A.collide_first = a == 0 && collide_first;
     A.write_mom = a == launches - 1 && write_moments;
     A.fsrc = f[a & 1];

@@ -681,9 +681,9 @@ _TILED_CUS = 256
 
 
 @functools.lru_cache(maxsize=256)
-def tiled_shape(sizes, double, forced):
+def tiled_shape(sizes, double, forced, cells=1024):
     """(rows, width, steps) of the tiled sweep's region for the lattices of
-    ``sizes``, a tuple of (nx, ny), swept by one launch.
+    ``sizes``, a tuple of (nx, ny), swept by one launch, of at most ``cells``.
 
     More steps per launch share its latency but grow the work on cells that
     several tiles compute; smaller regions spread a small lattice over more
@@ -692,6 +692,7 @@ def tiled_shape(sizes, double, forced):
     of regions and steps on seven lattices from 128 x 128 to 1001 x 413 it
     picks the fastest region or one within 4 % of it."""
     load, step, most = _TILED_COST[8 if double else 4, bool(forced)]
+    most = min(most, cells)
     best = None
     for width in (16, 32, 64):
         for steps in (4, 6, 8):
@@ -718,6 +719,14 @@ def tiled_shape(sizes, double, forced):
 # FP64 2048x1024 52 against 75; FP64 1001x413 22 against 15, its two kernels
 # and their join)
 _SINGLE_FUSED_CELLS = {8: 1 << 20, 4: 1 << 18}
+# 16-bit lattices asked for two steps per sweep, without (True) and with a rim:
+# cells up to which tiles, with the same roundings, are faster.  us per step
+# tiles / two-step, FP16, calls of 80 steps: channel 512x256 2.9 / 4.2, 512x512
+# 4.1 / 4.5, 768x512 5.5 / 4.6; with a rim cylinder 400x300 2.7 / 13.9, 900x700
+# 7.4 / 14.5, 1500x1000 17.4 / 17.7, 2277x892 21.7 / 19.3.  Calls of 12 steps
+# replay no graph, which costs the two-step sweep's three kernels more:
+# 1500x1000 18.7 / 26.3, 2277x892 23.5 / 25.2, 2400x1200 31.3 / 28.2.
+_PAIRS_TILED_CELLS = {True: 5 << 16, False: 1 << 21}
 # chunks of the strip sweep the GPU holds at once
 _STRIP_SLOTS = {8: 768, 4: 1536}
 # the strip sweep's tiles recompute most of their cells: a lattice with more
@@ -829,8 +838,9 @@ class D2Q9Engine:
     ``TWO_STEP_MIN_BYTES`` and they cover the lattice (the results are
     bitwise those of single steps), for 16-bit storage only when asked (its
     intermediate step stays in FP32, which changes the rounding).  FP64 and
-    FP32 lattices large enough for the strip sweep take that instead, to the
-    same bits (``_choose_sweep``).  Otherwise steps go through the strip sweep
+    FP32 lattices large enough for the strip sweep take that instead, and small
+    16-bit ones the tiled sweep, to the same bits (``_choose_sweep``).
+    Otherwise steps go through the strip sweep
     on large lattices (d2q9_strip_steps) and the tiled sweep on others
     (d2q9_tiled_steps), several steps per launch and bitwise single steps in
     every storage form, or through single sweeps where the case cannot be
@@ -1032,6 +1042,7 @@ class D2Q9Engine:
             return
         self.n_deep = d.n_deep
         self.deep_fraction = float(d.covered.mean())
+        self._covered = d.covered
         if self._several:
             self.two_step = True
             return
@@ -1097,14 +1108,16 @@ class D2Q9Engine:
         ``_several``: the strip or tiled sweep runs even where two steps per
         sweep were asked for.
 
-        The two-step sweep keeps lattices that ask for it and are in 16-bit
-        storage or too small for strips, and those without tables.  us per
+        The two-step sweep keeps lattices that ask for it and are too small
+        for strips or, in 16-bit storage, too large for tiles, and those
+        without tables.  us per
         step two-step / strips, without a rim: FP64 MRT 2048x1024 32.8 / 32.2,
         4096x1024 59.5 / 55.5, 8192x2048 235 / 191, FP32 2048x1024 16.2 / 12.0,
         4096x1024 34.6 / 25.4; with one (two more kernels, a fork and a join):
         FP64 3001x1333 65 / 36, 1371x1362 36 / 20, FP32 22 / 9.  In 16-bit
         storage the sweep decides what is rounded: the two-step sweep every
-        second step (in the rim every step), which no other one gives."""
+        second step (in the rim every step), which the tiled one can do too
+        and the strips cannot."""
         self._split = None
         if self._codes is not None:
             shape = [ctypes.c_int32() for _ in range(3)]
@@ -1123,44 +1136,75 @@ class D2Q9Engine:
                         else 160))
             if split is not None and split[2] <= _STRIP_TILE_SHARE:
                 self._split = split
+        half = self.raw_dtype.itemsize == 2
         self._several = not self._two_step_req or (
-            self._split is not None and self.raw_dtype.itemsize != 2)
+            self._codes is not None and
+            self.nx * self.ny <= _PAIRS_TILED_CELLS[self._rimless()] if half
+            else self._split is not None)
 
     def _setup_tiled(self):
         """Tables of the tiled sweep on the device, where the lattice takes
         it.  A 16-bit lattice that runs the two-step sweep has them too: for
         its single steps, and for all steps where that sweep goes."""
         self.tiled = None
-        self._tiled_arrays = None
         t, tables = self.tables, self._codes
         self._codes = None
         if tables is None or (self.two_step and not self._several and
                               self.raw_dtype.itemsize != 2):
             return
         cells, codes, has_vel, has_pres = tables
+        # two workgroups per CU have room for the rim's rounded values and
+        # the planes of fixed pressures up to 960 cells
         rows, width, steps = tiled_shape(
             ((self.nx, self.ny),), self.storage == nt.STORE_F64,
-            self.forcing is not None)
+            self.forcing is not None,
+            960 if has_pres and self._pairs() else 1024)
         with torch.cuda.stream(self.stream):
-            dev = {"cells": self._upload_plane(cells, torch.int32),
-                   "codes": torch.from_numpy(codes.view(np.int32)).to(
-                       self.device)}
+            self._tiled_codes = torch.from_numpy(codes.view(np.int32)).to(
+                self.device)
         D = nt.TiledDesc()
         D.rows, D.width, D.steps = rows, width, steps
         D.n_elems = len(t.elems)
         D.has_vel, D.has_pres = int(has_vel), int(has_pres)
-        D.round_last = self._round_last()
-        D.cells, D.codes = dev["cells"].data_ptr(), dev["codes"].data_ptr()
-        self._tiled_arrays = dev
+        D.codes = self._tiled_codes.data_ptr()
+        self._set_rounding(D, cells)
         self._tiled_solid = np.flatnonzero(
             (t.flags_pad & nt.CELL_SOLID).ravel())
         self.tiled = D
         self._tiled_p = ctypes.byref(D)
 
-    def _round_last(self):
-        """D.round_last: 16-bit lattices asked for two steps per sweep round
-        the stored step of a launch only."""
-        return int(self.two_step and self.raw_dtype.itemsize == 2)
+    def _pairs(self):
+        """Whether a 16-bit lattice asked for two steps per sweep runs the
+        tiled sweep."""
+        return (self.two_step and self._several and
+                self.raw_dtype.itemsize == 2)
+
+    def _set_rounding(self, D, cells):
+        """What 16-bit lattices asked for two steps per sweep round in the
+        tiled sweep, and its plane of ``cells``: with ``pairs`` what the
+        two-step sweep does (TiledDesc), the cells outside its deep tiles
+        marked as the rim."""
+        D.round_last = int(self.two_step and self.raw_dtype.itemsize == 2)
+        D.pairs = 0
+        if self._pairs():
+            rim = self.tables.fluid_pad.copy()
+            rim[1:-1, 1:-1] &= ~self._covered
+            D.pairs = 2 if rim.any() else 1
+            near = rim.copy()
+            for axis, periodic in ((0, self.tables.x_periodic),
+                                   (1, self.tables.y_periodic)):
+                a = np.moveaxis(near, axis, 0)
+                if periodic:
+                    a[0], a[-1] = a[-2], a[1]
+                grown = a.copy()
+                grown[1:] |= a[:-1]
+                grown[:-1] |= a[1:]
+                a[:] = grown
+            bits = rim * nt.TILED_RIM + near * nt.TILED_NEAR_RIM
+            cells = cells | bits.astype(np.uint32)
+        with torch.cuda.stream(self.stream):
+            self._tiled_cells = self._upload_plane(cells, torch.int32)
+        D.cells = self._tiled_cells.data_ptr()
 
     def _setup_strips(self, rows=None):
         """Lists of the strip sweep on the device, where a lattice with
@@ -1225,7 +1269,10 @@ class D2Q9Engine:
             nt.ptr(self.mom[m]), nt.ptr(self.mom[1 - m]), n, int(first),
             int(write_moments), None, 0, self._stream_ptr),
             "d2q9_tiled_steps")
-        flip = -(-n // self.tiled.steps) & 1
+        most = self.tiled.steps
+        if self.tiled.pairs:
+            most -= most % 2
+        flip = -(-n // most) & 1
         self.i_pop, self.i_mom = a ^ flip, m ^ flip
         self.i_pop_new = None
         self.mom_full = bool(write_moments)
@@ -1244,8 +1291,8 @@ class D2Q9Engine:
         self._upload_tiles()
         if self.two_step:
             self._setup_two_step()
-        if self.tiled is not None:
-            self.tiled.round_last = self._round_last()
+        if self.tiled is not None and self.raw_dtype.itemsize == 2:
+            self._set_rounding(self.tiled, self.tables.special_codes()[0])
 
     # ---- layout helpers -------------------------------------------------
     def _upload_plane(self, pad, dtype, count=1):
@@ -1325,7 +1372,15 @@ class D2Q9Engine:
             return "two-step"
         if self.tiled is None:
             return "single"
-        return "strips" if self.strips is not None else "tiled"
+        return ("strips" if self.strips is not None and not self.tiled.pairs
+                else "tiled")
+
+    @property
+    def runs_pairs(self):
+        """Whether steps run in pairs: by the two-step sweep, or by tiles with
+        its roundings (16-bit storage)."""
+        return self.sweep == "two-step" or (self.tiled is not None and
+                                            self.tiled.pairs != 0)
 
     # ---- kernels --------------------------------------------------------
     def _collide(self, src, dst, write_mom):
@@ -1400,7 +1455,8 @@ class D2Q9Engine:
             return
         sweep = self.sweep
         if sweep in ("strips", "tiled"):
-            if sweep == "strips" and self.i_pop_new is not None:
+            if self.i_pop_new is not None and (sweep == "strips" or
+                                               self.tiled.pairs):
                 self.step(write_moments and n == 1)
                 n -= 1
             if n == 1:

@@ -124,7 +124,8 @@ class Solver:
         names = {"strips": "strip sweep", "tiled": "tiled sweep",
                  "two-step": "two-step sweep", "single": "single steps"}
         print_log(f"{'Engine':<10}: storage {eng.storage_name}, "
-                  f"{names[eng.sweep]}", 0,
+                  f"{names[eng.sweep]}"
+                  f"{', in pairs' if eng.runs_pairs else ''}", 0,
                   self.verbose if verbose is None else verbose)
         for op in (self.mpi_operator, self.collision_operator,
                    self.force_operator, self.compute_fields_operator,

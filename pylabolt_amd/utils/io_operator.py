@@ -50,10 +50,10 @@ class InputOutputOperator:
         eng = getattr(self, "engine", None)
         if eng is not None:
             # not read by the reference's tools: how the run was computed
-            # (the sweep that runs, not the one asked for: in 16-bit storage
-            # the two-step sweep rounds every second step)
+            # (what runs, not what was asked for: in 16-bit storage pairs of
+            # steps are rounded once)
             meta["engine"] = {"storage": eng.storage_name,
-                              "two_step": eng.sweep == "two-step"}
+                              "two_step": bool(eng.runs_pairs)}
         os.makedirs(self.field_save_path, exist_ok=True)
         with open(os.path.join(self.root, "metadata.json"), "w") as f:
             json.dump(meta, f, indent=4)

@@ -10,16 +10,16 @@ from pylabolt_amd.solvers.fluidLB import FluidLB, Solver
 from pylabolt_amd.utils.io_operator import InputOutputOperator
 
 
-@pytest.mark.parametrize("sweep", ["strips", "tiled", "two-step", "single"])
-def test_metadata(tmp_path, sweep):
+@pytest.mark.parametrize("pairs", [False, True])
+def test_metadata(tmp_path, pairs):
     st = State(cases.lid_driven_cavity(20, 16))
     io = InputOutputOperator(FluidLB(), st, root=str(tmp_path))
     # two_step as the engine has it where strips take the sweep's place
-    io.engine = SimpleNamespace(storage_name="f64", two_step=True, sweep=sweep)
+    io.engine = SimpleNamespace(storage_name="f64", two_step=True,
+                                runs_pairs=pairs)
     io.dump_metadata(st)
     meta = json.loads((tmp_path / "metadata.json").read_text())
-    assert meta["engine"] == {"storage": "f64",
-                              "two_step": sweep == "two-step"}
+    assert meta["engine"] == {"storage": "f64", "two_step": pairs}
 
 
 @pytest.mark.gpu
@@ -27,7 +27,11 @@ def test_metadata(tmp_path, sweep):
     (lambda: cases.poiseuille_channel(2048, 512), "f64", None, "strip sweep"),
     (lambda: cases.poiseuille_channel(120, 300), "f64", None, "tiled sweep"),
     (lambda: cases.poiseuille_channel(120, 512), "f16dev", True,
-     "two-step sweep")])
+     "tiled sweep, in pairs"),
+    (lambda: cases.poiseuille_channel(1024, 512), "f16dev", True,
+     "two-step sweep, in pairs"),
+    (lambda: cases.lid_driven_cavity(120, 512), "bf16dev", None,
+     "tiled sweep")])
 def test_log_line(capsys, sim, storage, two_step, want):
     s = Solver(simulation=sim(), storage=storage, two_step=two_step,
                verbose=False)
@@ -35,5 +39,4 @@ def test_log_line(capsys, sim, storage, two_step, want):
     line = [v for v in capsys.readouterr().out.splitlines()
             if v.startswith("Engine")]
     assert line and line[0].endswith(f"storage {storage}, {want}")
-    if want != "tiled sweep":
-        assert s.engine.two_step
+    assert s.engine.two_step == (want != "tiled sweep")

@@ -274,8 +274,9 @@ def batched_form(steps=5000, warmup=50, per_lattice_steps=100, n=256,
     """Batched workload: ``n`` seeded lattices (sizes uniform over the
     multiples of 32 in 64..1024 x 64..512, Re in [50, 400], even ids cavity
     BGK, odd ids Guo-forced channel MRT), FP32, several steps of all of them
-    per launch.  Aggregate MLUPS = sum of cells * steps / t.  The same
-    lattices advanced one launch per lattice per step are timed beside it
+    per launch (``config`` and ``items_per_step`` are those of the persistent
+    kernel that takes batches the tiled sweep cannot).  Aggregate MLUPS =
+    sum of cells * steps / t.  The same lattices advanced one launch per lattice per step are timed beside it
     over ``per_lattice_steps`` steps."""
     import torch
     from pylabolt_amd import cases
@@ -316,7 +317,8 @@ def batched_form(steps=5000, warmup=50, per_lattice_steps=100, n=256,
         "mlups": mlups, "us_per_step": t / steps * 1e6,
         "achieved_gbs": achieved, "frac": achieved / PEAK_GBS,
         "steps_per_launch": batch.steps_per_launch,
-        "tiles_per_launch": batch._tiled_count, "setup_s": t_setup,
+        "config": batch.config.as_dict(), "items_per_step": batch.n_items,
+        "setup_s": t_setup,
         "per_lattice_launches_mlups": mlups_pl,
         "speedup_vs_per_lattice_launches": (mlups / mlups_pl
                                             if mlups_pl else None),

@@ -294,9 +294,9 @@ __global__ __launch_bounds__(THREADS, waves_per_simd<S>()) void k_strip(
   const int b = (int)blockIdx.x;
   if (b < P.n_tiles) {
     const d2q9_strip_tile it = P.tiles[b];
-    tiled::run_tile<S, MODEL, FORCING, TILE_W>(L, D, smem, it.i_first, it.j_first, TILE, K,
-                                               TILE + 2 * K, 0, fsrc, fdst, msrc, mdst,
-                                               write_mom, nullptr, 0);
+    tiled::run_tile<S, MODEL, FORCING, TILE_W, false>(L, D, smem, it.i_first, it.j_first, TILE,
+                                                      K, TILE + 2 * K, 0, fsrc, fdst, msrc, mdst,
+                                                      write_mom, nullptr, 0);
     return;
   }
   run_strip<S, MODEL, FORCING>(L, smem, P.chunks[xcd_remap(b - P.n_tiles, P.n_chunks)], K, fsrc,
@@ -321,7 +321,7 @@ hipError_t launch_one(const d2q9_lattice* L, const d2q9_tiled_desc* D, const d2q
   if (const hipError_t e = tiled::allow_lds(limit, kern)) return e;
   size_t lds = ring_bytes<S>(A.K);
   if (P->n_tiles > 0) {
-    const size_t t = tiled::lds_bytes(*D, (TILE + 2 * A.K) * TILE_W, sizeof(typename C::T));
+    const size_t t = tiled::lds_bytes<false>(*D, (TILE + 2 * A.K) * TILE_W, sizeof(typename C::T));
     if (t > lds) lds = t;
   }
   hipLaunchKernelGGL(kern, dim3((unsigned)(P->n_tiles + P->n_chunks)), dim3(THREADS), lds,

@@ -41,17 +41,20 @@ constexpr int MAX_CELLS = 1024;   // of a region, one per thread
 
 // Planes of LDS values besides the nine populations: rho where a cell is a
 // moving wall's, u where one is at fixed pressure, and the rounded populations
-// for the rim's cells (pairs == 2).
+// for the rim's cells (pairs == 2).  PAIRS: of a kernel that rounds pairs.
+template <bool PAIRS>
 __host__ __device__ inline int lds_planes(const d2q9_tiled_desc& D) {
-  return 9 + (D.has_vel ? 1 : 0) + (D.has_pres ? 2 : 0) + (D.pairs == 2 ? 9 : 0);
+  return 9 + (D.has_vel ? 1 : 0) + (D.has_pres ? 2 : 0) + (PAIRS && D.pairs == 2 ? 9 : 0);
 }
+template <bool PAIRS>
 __host__ __device__ inline int lds_values(const d2q9_tiled_desc& D, int area) {
-  return (area * lds_planes(D) + 3) & ~3;
+  return (area * lds_planes<PAIRS>(D) + 3) & ~3;
 }
 // LDS of a launch: the planes of every cell of the region and the boundary
 // elements.
+template <bool PAIRS>
 __host__ __device__ inline size_t lds_bytes(const d2q9_tiled_desc& D, int area, size_t elem) {
-  return (size_t)lds_values(D, area) * elem + MAX_ELEMS * sizeof(d2q9_bc_elem);
+  return (size_t)lds_values<PAIRS>(D, area) * elem + MAX_ELEMS * sizeof(d2q9_bc_elem);
 }
 
 // Value as the storage form keeps it from one step to the next.
@@ -127,8 +130,10 @@ __device__ __forceinline__ void apply_pres(const Consts<typename Codec<S>::T>& K
 // a constant distance).  mom_steps, when not null, receives rho/u of every
 // owned cell after every step (step s at mom_steps + s * mom_stride), and
 // mdst is not written.  With collide_first the first step is moments and
-// collision of the loaded populations alone (no streaming).
-template <int S, int MODEL, int FORCING, int W>
+// collision of the loaded populations alone (no streaming).  PAIRS: D.pairs is
+// not 0 (a kernel of its own: in one with the other forms BF16 1024x256 took
+// 3.86 us per step with every step rounded, 3.72 without).
+template <int S, int MODEL, int FORCING, int W, bool PAIRS>
 __device__ __forceinline__ void run_tile(
     const d2q9_lattice& L, const d2q9_tiled_desc& D, char* __restrict__ smem, int i_first,
     int j_first, int tile_c, int K, int rows, int collide_first, const typename Codec<S>::raw* __restrict__ fsrc,
@@ -145,7 +150,7 @@ __device__ __forceinline__ void run_tile(
   T* const srho = s + 9 * area;
   T* const su = srho + (D.has_vel ? area : 0);
   T* const srim = su + (D.has_pres ? 2 * area : 0);   // as s, 16-bit rims only
-  d2q9_bc_elem* const elems = reinterpret_cast<d2q9_bc_elem*>(s + lds_values(D, area));
+  d2q9_bc_elem* const elems = reinterpret_cast<d2q9_bc_elem*>(s + lds_values<PAIRS>(D, area));
   const Consts<T> Kc = load_consts<T>(L);
   const int i0 = i_first - K, j0 = j_first - K;   // the region's first cell
   // the whole region lies in the lattice: nothing to wrap or to leave out
@@ -163,8 +168,7 @@ __device__ __forceinline__ void run_tile(
   uint32_t arith = 0;       // special cells: directions with arithmetic
   T ffx = (T)0, ffy = (T)0;
   // 16-bit storage: every step is rounded, or every second one
-  const bool each = sizeof(R) == 2 && !D.round_last && !D.pairs;
-  const bool pairs = sizeof(R) == 2 && D.pairs != 0;
+  const bool each = !PAIRS && sizeof(R) == 2 && !D.round_last;
   bool rim = false, near_rim = false;
   {
     const int r = e / W, c = e % W;
@@ -198,7 +202,7 @@ __device__ __forceinline__ void run_tile(
       if (info & D2Q9_CELL_FLUID) {
         depth = min(min(r, rows - 1 - r), min(c, W - 1 - c));
         keep = (info & D2Q9_CELL_STORE_MOM) != 0;
-        if (sizeof(R) == 2 && D.pairs == 2) {
+        if (PAIRS && D.pairs == 2) {
           rim = (info & D2Q9_TILED_RIM) != 0;
           near_rim = (info & D2Q9_TILED_NEAR_RIM) != 0;
         }
@@ -221,7 +225,7 @@ __device__ __forceinline__ void run_tile(
       }
 #pragma unroll
       for (int k = 0; k < 9; ++k) s[e * 9 + k] = C::dec(raw[k], k, Kc);
-      if (sizeof(R) == 2 && D.pairs == 2) {
+      if (PAIRS && D.pairs == 2) {
         // cells that are not fluid keep these
 #pragma unroll
         for (int k = 0; k < 9; ++k) srim[e * 9 + k] = C::dec(raw[k], k, Kc);
@@ -273,7 +277,7 @@ __device__ __forceinline__ void run_tile(
     collide<T, MODEL, FORCING, C::dev>(g, Kc, drho, rho, ux, uy, fx, fy, px, py);
     const uint32_t key = sizeof(R) == 2 ? cell_key((uint32_t)cell) : 0u;
     if (st < K) {
-      const bool round = each || (pairs && !(st & 1));
+      const bool round = PAIRS ? !(st & 1) : each;
 #pragma unroll
       for (int k = 0; k < 9; ++k)
         s[e * 9 + k] = round ? through_storage<S>(g[k], k, key, Kc) : g[k];
@@ -314,7 +318,7 @@ constexpr int waves_per_simd() {
   return S != D2Q9_STORE_F64 ? 8 : FORCING == D2Q9_FORCING_NONE ? 6 : 4;
 }
 
-template <int S, int MODEL, int FORCING, int W>
+template <int S, int MODEL, int FORCING, int W, bool PAIRS>
 __global__ __launch_bounds__(MAX_CELLS, (waves_per_simd<S, FORCING>())) void k_tiled(
     const d2q9_lattice L, const d2q9_tiled_desc D, int ntiles, int ntj, int K, int rows,
     int collide_first, const typename Codec<S>::raw* __restrict__ fsrc,
@@ -323,10 +327,9 @@ __global__ __launch_bounds__(MAX_CELLS, (waves_per_simd<S, FORCING>())) void k_t
     typename Codec<S>::T* __restrict__ mom_steps, int64_t mom_stride) {
   extern __shared__ __align__(16) char smem[];
   const int tile = xcd_remap((int)blockIdx.x, ntiles);
-  run_tile<S, MODEL, FORCING, W>(L, D, smem, 1 + (tile / ntj) * (rows - 2 * K),
-                                 1 + (tile % ntj) * (W - 2 * K), W - 2 * K, K, rows,
-                                 collide_first, fsrc, fdst, msrc, mdst, write_mom, mom_steps,
-                                 mom_stride);
+  run_tile<S, MODEL, FORCING, W, PAIRS>(
+      L, D, smem, 1 + (tile / ntj) * (rows - 2 * K), 1 + (tile % ntj) * (W - 2 * K), W - 2 * K, K,
+      rows, collide_first, fsrc, fdst, msrc, mdst, write_mom, mom_steps, mom_stride);
 }
 
 // The checks of a descriptor every entry point makes (d2q9_tiled.hip): 0, or
@@ -363,10 +366,10 @@ struct Launch {
 template <int S>
 hipError_t launch(const d2q9_lattice* L, const d2q9_tiled_desc* D, const Launch& A);
 
-template <int S, int MODEL, int FORCING, int W>
+template <int S, int MODEL, int FORCING, int W, bool PAIRS>
 hipError_t launch_one(const d2q9_lattice* L, const d2q9_tiled_desc* D, const Launch& A) {
   using C = Codec<S>;
-  auto kern = k_tiled<S, MODEL, FORCING, W>;
+  auto kern = k_tiled<S, MODEL, FORCING, W, PAIRS>;
   static PerDevice limit;
   if (const hipError_t e = allow_lds(limit, kern)) return e;
   // the region loses the rows a shorter launch does not need
@@ -374,7 +377,8 @@ hipError_t launch_one(const d2q9_lattice* L, const d2q9_tiled_desc* D, const Lau
   const int tr = rows - 2 * A.K, tc = W - 2 * A.K;
   const int ntj = (L->ny + tc - 1) / tc, tiles = (L->nx + tr - 1) / tr * ntj;
   hipLaunchKernelGGL(kern, dim3((unsigned)tiles), dim3((unsigned)((rows * W + 63) / 64 * 64)),
-                     lds_bytes(*D, rows * W, sizeof(typename C::T)), A.stream, *L, *D, tiles,
+                     lds_bytes<PAIRS>(*D, rows * W, sizeof(typename C::T)),
+                     A.stream, *L, *D, tiles,
                      ntj, A.K, rows, A.collide_first, static_cast<const typename C::raw*>(A.fsrc),
                      static_cast<typename C::raw*>(A.fdst),
                      static_cast<const typename C::T*>(A.msrc),
@@ -383,14 +387,22 @@ hipError_t launch_one(const d2q9_lattice* L, const d2q9_tiled_desc* D, const Lau
   return hipGetLastError();
 }
 
-template <int S, int MODEL, int FORCING>
-hipError_t launch_shape(const d2q9_lattice* L, const d2q9_tiled_desc* D, const Launch& A) {
+template <int S, int MODEL, int FORCING, bool PAIRS>
+hipError_t launch_width(const d2q9_lattice* L, const d2q9_tiled_desc* D, const Launch& A) {
   switch (D->width) {
-    case 16: return launch_one<S, MODEL, FORCING, 16>(L, D, A);
-    case 32: return launch_one<S, MODEL, FORCING, 32>(L, D, A);
-    case 64: return launch_one<S, MODEL, FORCING, 64>(L, D, A);
+    case 16: return launch_one<S, MODEL, FORCING, 16, PAIRS>(L, D, A);
+    case 32: return launch_one<S, MODEL, FORCING, 32, PAIRS>(L, D, A);
+    case 64: return launch_one<S, MODEL, FORCING, 64, PAIRS>(L, D, A);
   }
   return hipErrorInvalidValue;
+}
+
+template <int S, int MODEL, int FORCING>
+hipError_t launch_shape(const d2q9_lattice* L, const d2q9_tiled_desc* D, const Launch& A) {
+  if constexpr (sizeof(typename Codec<S>::raw) == 2) {
+    if (D->pairs) return launch_width<S, MODEL, FORCING, true>(L, D, A);
+  }
+  return launch_width<S, MODEL, FORCING, false>(L, D, A);
 }
 
 template <int S>

@@ -32,7 +32,7 @@ __global__ __launch_bounds__(MAX_CELLS, S == D2Q9_STORE_F64 ? 4 : 8) void k_tile
   auto md = static_cast<typename C::T*>(E.mom[1 - parity]);
 #define D2Q9_TILED_ITEM(KEY, M, F)                                                         \
   case KEY:                                                                                \
-    run_tile<S, M, F, W>(L, D, smem, 1 + it.ti * (rows - 2 * K), 1 + it.tj * tile_c,       \
+    run_tile<S, M, F, W, false>(L, D, smem, 1 + it.ti * (rows - 2 * K), 1 + it.tj * tile_c,       \
                          tile_c, K, rows, collide_first, fs, fd, ms, md, write_mom,        \
                          nullptr, 0);                                                      \
     break;

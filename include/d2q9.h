@@ -431,7 +431,7 @@ int d2q9_batched_step(const d2q9_batch_entry* entries,
 
 /*
  * Strip sweep: n fused steps, up to 4 per launch, as d2q9_tiled_steps (bitwise
- * single steps unless D asks for round_last; pairs is refused).  d2q9_strip_shape gives the
+ * single steps unless D asks for round_last or pairs).  d2q9_strip_shape gives the
  * most steps of a launch, a strip's output columns and a tile's output rows
  * and columns.
  *
@@ -444,7 +444,9 @@ int d2q9_batched_step(const d2q9_batch_entry* entries,
  * j_first) of tiles whose cells together with the chunks' cover every fluid
  * cell; a cell in several of them is written with the same bits.  D: the
  * tables of d2q9_tiled_steps (its region is not used), with their conditions.
- * The caller guarantees the lists; chunks are device memory, tiles too.
+ * D->pairs == 2: no cell of a chunk or within `steps` of it has bit
+ * D2Q9_TILED_RIM.  The caller guarantees the lists; chunks are device memory,
+ * tiles too.
  */
 typedef struct d2q9_strip_chunk {
   int32_t i_first, rows, j_first, cols, walls;

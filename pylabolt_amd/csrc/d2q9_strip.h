@@ -30,7 +30,8 @@
 // is in a tile of the tiled sweep, run by the same launch's first workgroups:
 // both read the source lattice alone and write different cells.  The
 // arithmetic per cell is the single step's; 16-bit storage rounds every step
-// (or, when asked, the last of a launch only).
+// (when asked, the last of a launch only, or as the two-step sweep: chunks then
+// hold cells of its deep tiles, rounded after every second step).
 #pragma once
 #include "d2q9_tiled.h"
 
@@ -42,6 +43,7 @@ constexpr int THREADS = 64 * STEPS;
 constexpr int COLS = 64 - 2 * STEPS;         // output columns of a strip
 constexpr int TILE_W = 16;                   // region width of the tiles
 constexpr int TILE = TILE_W - 2 * STEPS;     // their output rows and columns
+static_assert(STEPS % 2 == 0, "launches take whole pairs of steps");
 // Rows of a ring, three directions each: 3 of 0,2,4, 3 of 3,6,7, 4 of 1,5,8.
 constexpr int RING_B = 9, RING_C = 18, RING = 30;
 
@@ -71,7 +73,7 @@ __device__ __forceinline__ T (&values_of(R (&raw)[9], T (&apart)[9]))[9] {
     return apart;
 }
 
-template <int S, int MODEL, int FORCING>
+template <int S, int MODEL, int FORCING, bool PAIRS>
 __device__ __forceinline__ void run_strip(
     const d2q9_lattice& L, char* __restrict__ smem, const d2q9_strip_chunk ch, int K,
     const typename Codec<S>::raw* __restrict__ fsrc, typename Codec<S>::raw* __restrict__ fdst,
@@ -149,7 +151,7 @@ __device__ __forceinline__ void run_strip(
     if (!decltype(stores)::value || st < K) {
       T* const w0 = to + a3 * 3 * PITCH;
       T* const wc = to + (RING_C + a4 * 3) * PITCH;
-      if (sizeof(R) == 2 && !round_last) {
+      if (sizeof(R) == 2 && (PAIRS ? !(st & 1) : !round_last)) {
 #pragma unroll
         for (int k = 0; k < 9; ++k) g[k] = tiled::through_storage<S>(g[k], k, key, Kc);
       }
@@ -284,7 +286,7 @@ constexpr int waves_per_simd() {
 }
 
 // Workgroups [0, n_tiles): tiles of TILE x TILE cells; the others: chunks.
-template <int S, int MODEL, int FORCING>
+template <int S, int MODEL, int FORCING, bool PAIRS>
 __global__ __launch_bounds__(THREADS, waves_per_simd<S>()) void k_strip(
     const d2q9_lattice L, const d2q9_tiled_desc D, const d2q9_strip_desc P, int K,
     const typename Codec<S>::raw* __restrict__ fsrc, typename Codec<S>::raw* __restrict__ fdst,
@@ -294,13 +296,13 @@ __global__ __launch_bounds__(THREADS, waves_per_simd<S>()) void k_strip(
   const int b = (int)blockIdx.x;
   if (b < P.n_tiles) {
     const d2q9_strip_tile it = P.tiles[b];
-    tiled::run_tile<S, MODEL, FORCING, TILE_W, false>(L, D, smem, it.i_first, it.j_first, TILE,
+    tiled::run_tile<S, MODEL, FORCING, TILE_W, PAIRS>(L, D, smem, it.i_first, it.j_first, TILE,
                                                       K, TILE + 2 * K, 0, fsrc, fdst, msrc, mdst,
                                                       write_mom, nullptr, 0);
     return;
   }
-  run_strip<S, MODEL, FORCING>(L, smem, P.chunks[xcd_remap(b - P.n_tiles, P.n_chunks)], K, fsrc,
-                               fdst, mdst, write_mom, D.round_last != 0);
+  run_strip<S, MODEL, FORCING, PAIRS>(L, smem, P.chunks[xcd_remap(b - P.n_tiles, P.n_chunks)], K,
+                                      fsrc, fdst, mdst, write_mom, D.round_last != 0);
 }
 
 struct Launch {
@@ -312,16 +314,16 @@ struct Launch {
   hipStream_t stream;
 };
 
-template <int S, int MODEL, int FORCING>
+template <int S, int MODEL, int FORCING, bool PAIRS>
 hipError_t launch_one(const d2q9_lattice* L, const d2q9_tiled_desc* D, const d2q9_strip_desc* P,
                       const Launch& A) {
   using C = Codec<S>;
-  auto kern = k_strip<S, MODEL, FORCING>;
+  auto kern = k_strip<S, MODEL, FORCING, PAIRS>;
   static PerDevice limit;
   if (const hipError_t e = tiled::allow_lds(limit, kern)) return e;
   size_t lds = ring_bytes<S>(A.K);
   if (P->n_tiles > 0) {
-    const size_t t = tiled::lds_bytes<false>(*D, (TILE + 2 * A.K) * TILE_W, sizeof(typename C::T));
+    const size_t t = tiled::lds_bytes<PAIRS>(*D, (TILE + 2 * A.K) * TILE_W, sizeof(typename C::T));
     if (t > lds) lds = t;
   }
   hipLaunchKernelGGL(kern, dim3((unsigned)(P->n_tiles + P->n_chunks)), dim3(THREADS), lds,
@@ -336,18 +338,27 @@ template <int S>
 hipError_t launch(const d2q9_lattice* L, const d2q9_tiled_desc* D, const d2q9_strip_desc* P,
                   const Launch& A);
 
+template <int S, bool PAIRS>
+hipError_t launch_kind(const d2q9_lattice* L, const d2q9_tiled_desc* D, const d2q9_strip_desc* P,
+                       const Launch& A) {
+  switch (L->collision * 3 + L->forcing) {
+    case 0: return launch_one<S, D2Q9_BGK, D2Q9_FORCING_NONE, PAIRS>(L, D, P, A);
+    case 1: return launch_one<S, D2Q9_BGK, D2Q9_GUO_LINEAR, PAIRS>(L, D, P, A);
+    case 2: return launch_one<S, D2Q9_BGK, D2Q9_GUO_SECOND_ORDER, PAIRS>(L, D, P, A);
+    case 3: return launch_one<S, D2Q9_MRT, D2Q9_FORCING_NONE, PAIRS>(L, D, P, A);
+    case 4: return launch_one<S, D2Q9_MRT, D2Q9_GUO_LINEAR, PAIRS>(L, D, P, A);
+    case 5: return launch_one<S, D2Q9_MRT, D2Q9_GUO_SECOND_ORDER, PAIRS>(L, D, P, A);
+  }
+  return hipErrorInvalidValue;
+}
+
 template <int S>
 hipError_t launch_model(const d2q9_lattice* L, const d2q9_tiled_desc* D, const d2q9_strip_desc* P,
                         const Launch& A) {
-  switch (L->collision * 3 + L->forcing) {
-    case 0: return launch_one<S, D2Q9_BGK, D2Q9_FORCING_NONE>(L, D, P, A);
-    case 1: return launch_one<S, D2Q9_BGK, D2Q9_GUO_LINEAR>(L, D, P, A);
-    case 2: return launch_one<S, D2Q9_BGK, D2Q9_GUO_SECOND_ORDER>(L, D, P, A);
-    case 3: return launch_one<S, D2Q9_MRT, D2Q9_FORCING_NONE>(L, D, P, A);
-    case 4: return launch_one<S, D2Q9_MRT, D2Q9_GUO_LINEAR>(L, D, P, A);
-    case 5: return launch_one<S, D2Q9_MRT, D2Q9_GUO_SECOND_ORDER>(L, D, P, A);
+  if constexpr (sizeof(typename Codec<S>::raw) == 2) {
+    if (D->pairs) return launch_kind<S, true>(L, D, P, A);
   }
-  return hipErrorInvalidValue;
+  return launch_kind<S, false>(L, D, P, A);
 }
 
 #define D2Q9_STRIP_DECLARE(SV)                                                 \

@@ -33,19 +33,20 @@ extern "C" int d2q9_strip_steps(const d2q9_lattice* L, const d2q9_tiled_desc* D,
   if (f_a == f_b || mom_a == mom_b)
     return sfail(D2Q9_E_ARG, "strip steps: the two buffers must differ");
   if (int r = tiled::check_desc(L, D)) return r;
-  if (D->pairs) return sfail(D2Q9_E_UNSUPPORTED, "strip steps: no rounding of pairs");
   if (n < 0 || P->n_tiles < 0 || P->n_chunks < 0 || (P->n_tiles > 0 && !P->tiles) ||
       (P->n_chunks > 0 && !P->chunks) || (int64_t)P->n_tiles + P->n_chunks > 0x7fffffff)
     return sfail(D2Q9_E_ARG, "strip steps: bad step count or lists");
   if (n == 0 || P->n_tiles + P->n_chunks == 0) return 0;
+  // as d2q9_tiled_steps: whole pairs where pairs are rounded
+  const int unit = D->pairs ? 2 : 1;
   const int launches = (n + strip::STEPS - 1) / strip::STEPS;
-  const int base = n / launches, longer = n % launches;
+  const int base = n / unit / launches, longer = n / unit % launches;
   void* f[2] = {f_a, f_b};
   void* m[2] = {mom_a, mom_b};
   strip::Launch A;
   A.stream = static_cast<hipStream_t>(stream);
   for (int a = 0; a < launches; ++a) {
-    A.K = base + (a < longer ? 1 : 0);
+    A.K = unit * (base + (a < longer ? 1 : 0)) + (a == launches - 1 ? n % unit : 0);
     A.write_mom = a == launches - 1 && write_moments;
     A.fsrc = f[a & 1];
     A.fdst = f[1 - (a & 1)];

@@ -405,7 +405,7 @@ class CaseTables:
         codes[:n, 2] = np.where(moving.any(axis=0), arith, 0)
         return cells, codes, bool(vel.any()), bool(pres.any())
 
-    def strip_split(self, steps, cols, tile, chunk_rows):
+    def strip_split(self, steps, cols, tile, chunk_rows, deep=None):
         """Chunks and tiles of the strip sweep (d2q9_strip_steps).
 
         Strips of ``cols`` columns (the last one of what is left, or the last
@@ -418,18 +418,23 @@ class CaseTables:
         ``tile`` x ``tile`` cells.  Returns (chunks [n, 5] int32: first row,
         rows, first column, columns, walls; tiles [m, 2] int32; the share of
         the cells in tiles), rows and columns from 1, or None when a strip
-        does not fit."""
+        does not fit.  ``deep`` [nx, ny]: chunks and the cells within
+        ``steps`` of them keep to these cells."""
         nx, ny = self.nx, self.ny
         if ny < cols + 2 * steps or nx < 2 * steps + 1:
             return None
         inner = self.flags_pad[1:-1, 1:-1]
         rough = inner != nt.CELL_FLUID
+        if deep is not None:
+            rough = rough | ~deep
         side = self.wall_side_pad[1:-1, 1:-1]
         inl = self.wall_inline_wrap if self.x_periodic else self.wall_inline
         lo_kind = np.where(inl[:, 0] & (side[:, 0] == 0), 1,
                            np.where(inl[:, 0] & (side[:, 0] == 2), 2, -1))
         hi_kind = np.where(inl[:, -1] & (side[:, -1] == 1), 1,
                            np.where(inl[:, -1] & (side[:, -1] == 3), 2, -1))
+        if deep is not None:
+            lo_kind[~deep[:, 0]] = hi_kind[~deep[:, -1]] = -1
         starts = list(range(0, ny, cols))
         if ny - starts[-1] < 2 * steps:
             starts[-1] -= 2 * steps      # a wall in no strip's margin
@@ -722,11 +727,16 @@ _SINGLE_FUSED_CELLS = {8: 1 << 20, 4: 1 << 18}
 # 16-bit lattices asked for two steps per sweep, without (True) and with a rim:
 # cells up to which tiles, with the same roundings, are faster.  us per step
 # tiles / two-step, FP16, calls of 80 steps: channel 512x256 2.9 / 4.2, 512x512
-# 4.1 / 4.5, 768x512 5.5 / 4.6; with a rim cylinder 400x300 2.7 / 13.9, 900x700
-# 7.4 / 14.5, 1500x1000 17.4 / 17.7, 2277x892 21.7 / 19.3.  Calls of 12 steps
+# 4.0 / 4.5, 768x512 5.4 / 4.6; with a rim cylinder 400x300 2.7 / 13.9, 900x700
+# 7.2 / 14.9, 1500x1000 16.7 / 17.8, 2277x892 21.1 / 19.6.  Calls of 12 steps
 # replay no graph, which costs the two-step sweep's three kernels more:
-# 1500x1000 18.7 / 26.3, 2277x892 23.5 / 25.2, 2400x1200 31.3 / 28.2.
+# 1500x1000 18.3 / 28.4, 2277x892 22.7 / 25.6, 2400x1200 30.0 / 27.9.
 _PAIRS_TILED_CELLS = {True: 5 << 16, False: 1 << 21}
+# and from which on strips are, without a rim (with one wherever they pay): 2048x512
+# 10.5 / 9.0, 2048x1024 15.3 / 15.4, 4096x1024 26.6 / 26.9, 8192x2048 85 / 92; with
+# a rim cylinder 8192x2048 64.5 / 82.2, 4096x1024 21.5 / 26.8, cavity 1500x1300 13.4
+# (tiles 16.8)
+_PAIRS_STRIP_CELLS = 1 << 21
 # chunks of the strip sweep the GPU holds at once
 _STRIP_SLOTS = {8: 768, 4: 1536}
 # the strip sweep's tiles recompute most of their cells: a lattice with more
@@ -837,10 +847,9 @@ class D2Q9Engine:
     and FP32 storage when the two population buffers exceed
     ``TWO_STEP_MIN_BYTES`` and they cover the lattice (the results are
     bitwise those of single steps), for 16-bit storage only when asked (its
-    intermediate step stays in FP32, which changes the rounding).  FP64 and
-    FP32 lattices large enough for the strip sweep take that instead, and small
-    16-bit ones the tiled sweep, to the same bits (``_choose_sweep``).
-    Otherwise steps go through the strip sweep
+    intermediate step stays in FP32, which changes the rounding).  Lattices
+    large enough for the strip sweep take that instead, and small 16-bit ones
+    the tiled sweep, to the same bits (``_choose_sweep``).  Otherwise steps go through the strip sweep
     on large lattices (d2q9_strip_steps) and the tiled sweep on others
     (d2q9_tiled_steps), several steps per launch and bitwise single steps in
     every storage form, or through single sweeps where the case cannot be
@@ -991,6 +1000,7 @@ class D2Q9Engine:
             two_step = self._two_step_moving and (self._codes is None or
                                                   self._rimless())
         self._two_step_req = bool(two_step)
+        self._deep_split = None
         self._choose_sweep()
         self.two_step = False
         self._setup_two_step()
@@ -1037,7 +1047,8 @@ class D2Q9Engine:
         self.two_step = False
         if not self._two_step_req:
             return
-        d = self.tables.deep_split(int(self.lib.d2q9_deep_rows()))
+        d = self._deep_tiles()
+        self._deep_split = None
         if d.n_deep == 0:
             return
         self.n_deep = d.n_deep
@@ -1109,38 +1120,56 @@ class D2Q9Engine:
         sweep were asked for.
 
         The two-step sweep keeps lattices that ask for it and are too small
-        for strips or, in 16-bit storage, too large for tiles, and those
-        without tables.  us per
-        step two-step / strips, without a rim: FP64 MRT 2048x1024 32.8 / 32.2,
-        4096x1024 59.5 / 55.5, 8192x2048 235 / 191, FP32 2048x1024 16.2 / 12.0,
-        4096x1024 34.6 / 25.4; with one (two more kernels, a fork and a join):
-        FP64 3001x1333 65 / 36, 1371x1362 36 / 20, FP32 22 / 9.  In 16-bit
-        storage the sweep decides what is rounded: the two-step sweep every
-        second step (in the rim every step), which the tiled one can do too
-        and the strips cannot."""
-        self._split = None
+        for strips (in 16-bit storage, and too large for tiles), and those
+        without tables.  us per step two-step / strips, without a rim: FP64 MRT
+        2048x1024 32.8 / 32.2, 4096x1024 59.5 / 55.5, 8192x2048 235 / 191, FP32
+        2048x1024 16.2 / 12.0, 4096x1024 34.6 / 25.4; with one (two more
+        kernels, a fork and a join): FP64 3001x1333 65 / 36, 1371x1362 36 / 20,
+        FP32 22 / 9.  In 16-bit storage all of them then round what the
+        two-step sweep does (``_set_rounding``), and the strips' chunks
+        (``_pair_strips``) keep to its deep tiles."""
+        half = self.raw_dtype.itemsize == 2
+        self._split, self._pair_strips = None, False
         if self._codes is not None:
             shape = [ctypes.c_int32() for _ in range(3)]
             nt.check(self.lib.d2q9_strip_shape(
                 *[ctypes.byref(v) for v in shape]), "d2q9_strip_shape")
             self._strip_shape = tuple(v.value for v in shape)
-            bits = 8 * self.raw_dtype.itemsize
-            rounds = bits == 16
-            split = None
-            if self.nx * -(-self.ny // self._strip_shape[1]) >= strip_least(
-                    bits == 64, rounds):
-                split = self.tables.strip_split(
-                    *self._strip_shape, functools.partial(
-                        strip_rows, double=bits == 64, rounds=rounds,
-                        most=32 if bits == 32 and self.forcing is None
-                        else 160))
-            if split is not None and split[2] <= _STRIP_TILE_SHARE:
-                self._split = split
-        half = self.raw_dtype.itemsize == 2
+            if half and self._two_step_req and self._deep_tiles().n_deep:
+                if (self.nx * self.ny > _PAIRS_STRIP_CELLS or
+                        not self._rimless()):
+                    self._split = self._strip_lists_of(
+                        False, self._deep_tiles().covered)
+                self._pair_strips = self._split is not None
+            else:
+                self._split = self._strip_lists_of(half)
         self._several = not self._two_step_req or (
-            self._codes is not None and
+            self._pair_strips or self._codes is not None and
             self.nx * self.ny <= _PAIRS_TILED_CELLS[self._rimless()] if half
             else self._split is not None)
+
+    def _strip_lists_of(self, rounds, deep=None):
+        """Chunks and tiles of the strip sweep (see ``strip_split``), or None
+        where it does not pay; ``rounds``: every step is rounded."""
+        bits = 8 * self.raw_dtype.itemsize
+        if self.nx * -(-self.ny // self._strip_shape[1]) < strip_least(
+                bits == 64, rounds):
+            return None
+        split = self.tables.strip_split(
+            *self._strip_shape, functools.partial(
+                strip_rows, double=bits == 64, rounds=rounds,
+                most=32 if bits == 32 and self.forcing is None else 160),
+            deep)
+        if split is None or split[2] > _STRIP_TILE_SHARE:
+            return None
+        return split
+
+    def _deep_tiles(self):
+        """The deep tiles of the two-step sweep for the present tile rows."""
+        if self._deep_split is None:
+            self._deep_split = self.tables.deep_split(
+                int(self.lib.d2q9_deep_rows()))
+        return self._deep_split
 
     def _setup_tiled(self):
         """Tables of the tiled sweep on the device, where the lattice takes
@@ -1213,7 +1242,10 @@ class D2Q9Engine:
         self.strips = None
         split = self._split
         if rows is not None:
-            split = self.tables.strip_split(*self._strip_shape, rows)
+            self._pair_strips = self._pairs()
+            split = self.tables.strip_split(
+                *self._strip_shape, rows,
+                self._covered if self._pair_strips else None)
         if self.tiled is None or split is None:
             return
         with torch.cuda.stream(self.stream):
@@ -1293,6 +1325,10 @@ class D2Q9Engine:
             self._setup_two_step()
         if self.tiled is not None and self.raw_dtype.itemsize == 2:
             self._set_rounding(self.tiled, self.tables.special_codes()[0])
+            if self._pair_strips:
+                self._split = self._strip_lists_of(False, self._covered)
+                self._pair_strips = self._split is not None
+                self._setup_strips()
 
     # ---- layout helpers -------------------------------------------------
     def _upload_plane(self, pad, dtype, count=1):
@@ -1372,8 +1408,8 @@ class D2Q9Engine:
             return "two-step"
         if self.tiled is None:
             return "single"
-        return ("strips" if self.strips is not None and not self.tiled.pairs
-                else "tiled")
+        return ("strips" if self.strips is not None and
+                (self._pair_strips or not self.tiled.pairs) else "tiled")
 
     @property
     def runs_pairs(self):

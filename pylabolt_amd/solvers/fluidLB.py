@@ -66,9 +66,9 @@ class Solver:
     how tiles holding solid cells are swept (``solid_tiles``: "sweep",
     "cells" or "auto"; None picks per storage form) and whether pairs of
     steps run as one sweep over the deep interior (``two_step``; None: not in
-    16-bit storage).  FP64 and FP32 lattices large enough for the strip sweep
-    take that whatever ``two_step`` says, and smaller ones are faster without
-    it.  Every choice gives bitwise the same results, but for ``two_step`` in
+    16-bit storage).  Lattices for which another sweep is as good take that
+    instead, to the same bits; FP64 and FP32 ones too small for strips are faster
+    without it.  Every choice gives bitwise the same results, but for ``two_step`` in
     16-bit storage, whose intermediate step stays in FP32.
     """
 

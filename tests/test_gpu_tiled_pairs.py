@@ -1,5 +1,5 @@
-"""The tiled sweep with the two-step sweep's roundings (16-bit lattices asked
-for two steps per sweep) against that sweep, bit for bit."""
+"""The tiled and strip sweeps with the two-step sweep's roundings (16-bit
+lattices asked for two steps per sweep) against that sweep, bit for bit."""
 import numpy as np
 import pytest
 
@@ -38,6 +38,7 @@ def _pair(monkeypatch, sim, storage):
     for cells in (1 << 30, 0):   # below which tiles run
         monkeypatch.setattr(engine, "_PAIRS_TILED_CELLS",
                             {True: cells, False: cells})
+        monkeypatch.setattr(engine, "strip_rows", lambda *a, **k: None)
         s = Solver(simulation=sim(), storage=storage, verbose=False,
                    graph_steps=4, two_step=True)
         f = s.state.fields
@@ -94,16 +95,67 @@ def test_other_tile_rows_move_the_rim(monkeypatch):
             _equal(a, b, (rows, n))
 
 
-def test_strips_refuse_pairs():
-    s = Solver(simulation=cases.lid_driven_cavity(1500, 1300),
-               storage="f16dev", verbose=False, two_step=True)
+STRIPS = {
+    "channel": lambda: _forced(72, 256),
+    "channel_shifted": lambda: _forced(80, 128, "BGK", "guo_linear"),
+    "cavity": lambda: cases.lid_driven_cavity(150, 512),
+    # zero-gradient walls in deep tiles, a solid, pressure ends; a part of a
+    # block at the high side; sides periodic in y
+    "cylinder": lambda: cases.cylinder(200, 384, diameter=20, xc=60),
+    "cylinder_part": lambda: cases.cylinder(160, 450, diameter=20, xc=50),
+    "box": lambda: _box(150, 512, (20.0, 10.0)),
+}
+
+
+@pytest.mark.parametrize("storage", ["f16dev", "bf16dev"])
+@pytest.mark.parametrize("rows", [9, 40])
+@pytest.mark.parametrize("name", list(STRIPS))
+def test_strips_equal_the_two_step_sweep(monkeypatch, name, rows, storage):
+    a, b = _pair(monkeypatch, STRIPS[name], storage)
+    a._setup_strips(rows)
+    assert a.sweep == "strips" and a.strips.n_chunks > 0
+    assert a.strips.n_tiles > 0 or a.tiled.pairs == 1
+    # launches of 4, 2 and 3, a step left over, whole launches
+    for n in (1, 4, 2, 3, 9, 15, 8):
+        a.advance(n)
+        b.advance(n)
+        _equal(a, b, (name, rows, storage, n))
+
+
+@pytest.mark.parametrize("sim,storage,sweep", [
+    (lambda: cases.lid_driven_cavity(1500, 1300), "f16dev", "strips"),
+    (lambda: cases.cylinder(1400, 2000, diameter=64), "bf16dev", "strips"),
+    (lambda: cases.poiseuille_channel(3000, 1024), "f16dev", "strips"),
+    (lambda: cases.poiseuille_channel(1500, 1024), "f16dev", "two-step"),
+    (lambda: cases.cylinder(2277, 892, diameter=64), "bf16dev", "tiled")])
+def test_large_lattices(monkeypatch, sim, storage, sweep):
+    """The sweep a large lattice takes, its moments and populations."""
+    out = []
+    for held in (False, True):
+        if held:
+            monkeypatch.setattr(engine, "_PAIRS_TILED_CELLS",
+                                {True: 0, False: 0})
+            monkeypatch.setattr(engine, "strip_rows", lambda *a, **k: None)
+        s = Solver(simulation=sim(), storage=storage, verbose=False,
+                   two_step=True)
+        s.set_backend()
+        out.append(s.engine)
+    a, b = out
+    assert a.sweep == sweep and b.sweep == "two-step"
+    for n in (6, 9):
+        a.advance(n)
+        b.advance(n)
+        _equal(a, b, (sweep, n))
+
+
+def test_bad_pairs_are_refused():
+    s = Solver(simulation=cases.lid_driven_cavity(60, 300), storage="f16dev",
+               verbose=False, two_step=True)
     s.set_backend()
     e = s.engine
-    e.tiled.pairs = 1
-    assert e.lib.d2q9_strip_steps(
-        e._Lp, e._tiled_p, e._strip_p, nt.ptr(e.f[0]), nt.ptr(e.f[1]),
-        nt.ptr(e.mom[0]), nt.ptr(e.mom[1]), 4, 0, e._stream_ptr) == -3
-    e.tiled.pairs = 3
-    assert e.lib.d2q9_tiled_steps(
-        e._Lp, e._tiled_p, nt.ptr(e.f[0]), nt.ptr(e.f[1]), nt.ptr(e.mom[0]),
-        nt.ptr(e.mom[1]), 4, 0, 0, None, 0, e._stream_ptr) == -1
+    for pairs, steps in ((3, 4), (-1, 4), (1, 1)):
+        e.tiled.pairs, e.tiled.steps = pairs, steps
+        assert e.lib.d2q9_tiled_steps(
+            e._Lp, e._tiled_p, nt.ptr(e.f[0]), nt.ptr(e.f[1]),
+            nt.ptr(e.mom[0]), nt.ptr(e.mom[1]), 4, 0, 0, None, 0,
+            e._stream_ptr) == -1

@@ -732,11 +732,11 @@ _SINGLE_FUSED_CELLS = {8: 1 << 20, 4: 1 << 18}
 # replay no graph, which costs the two-step sweep's three kernels more:
 # 1500x1000 18.3 / 28.4, 2277x892 22.7 / 25.6, 2400x1200 30.0 / 27.9.
 _PAIRS_TILED_CELLS = {True: 5 << 16, False: 1 << 21}
-# and from which on strips are, without a rim (with one wherever they pay): 2048x512
-# 10.5 / 9.0, 2048x1024 15.3 / 15.4, 4096x1024 26.6 / 26.9, 8192x2048 85 / 92; with
-# a rim cylinder 8192x2048 64.5 / 82.2, 4096x1024 21.5 / 26.8, cavity 1500x1300 13.4
-# (tiles 16.8)
-_PAIRS_STRIP_CELLS = 1 << 21
+# and above which strips are, without a rim (with one wherever they pay): 2048x512
+# 10.5 / 9.0, 2048x1024 15.3 / 15.4, 4096x1024 26.6 / 26.9 (calls of 20 steps 26.8 /
+# 26.5), 8192x2048 85 / 92; with a rim cylinder 8192x2048 64.5 / 82.2, 4096x1024
+# 21.5 / 26.8, cavity 1500x1300 13.4 (tiles 16.8)
+_PAIRS_STRIP_CELLS = 1 << 22
 # chunks of the strip sweep the GPU holds at once
 _STRIP_SLOTS = {8: 768, 4: 1536}
 # the strip sweep's tiles recompute most of their cells: a lattice with more

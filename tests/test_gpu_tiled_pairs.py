@@ -125,7 +125,7 @@ def test_strips_equal_the_two_step_sweep(monkeypatch, name, rows, storage):
 @pytest.mark.parametrize("sim,storage,sweep", [
     (lambda: cases.lid_driven_cavity(1500, 1300), "f16dev", "strips"),
     (lambda: cases.cylinder(1400, 2000, diameter=64), "bf16dev", "strips"),
-    (lambda: cases.poiseuille_channel(3000, 1024), "f16dev", "strips"),
+    (lambda: cases.poiseuille_channel(5000, 1024), "f16dev", "strips"),
     (lambda: cases.poiseuille_channel(1500, 1024), "f16dev", "two-step"),
     (lambda: cases.cylinder(2277, 892, diameter=64), "bf16dev", "tiled")])
 def test_large_lattices(monkeypatch, sim, storage, sweep):

@@ -83,8 +83,12 @@ def test_region_shapes(monkeypatch, name, shape):
         _equal(a, b, (name, shape, n))
 
 
-def test_other_tile_rows_move_the_rim(monkeypatch):
+@pytest.mark.parametrize("strips", [False, True])
+def test_other_tile_rows_move_the_rim(monkeypatch, strips):
     a, b = _pair(monkeypatch, lambda: _forced(70, 256), "f16dev")
+    if strips:
+        a._setup_strips(9)
+        assert a.sweep == "strips"
     for rows, pairs in ((4, 2), (2, 1)):
         a.set_tile_rows(rows)
         b.set_tile_rows(rows)

@@ -732,10 +732,10 @@ _SINGLE_FUSED_CELLS = {8: 1 << 20, 4: 1 << 18}
 # replay no graph, which costs the two-step sweep's three kernels more:
 # 1500x1000 18.3 / 28.4, 2277x892 22.7 / 25.6, 2400x1200 30.0 / 27.9.
 _PAIRS_TILED_CELLS = {True: 5 << 16, False: 1 << 21}
-# and above which strips are, without a rim (with one wherever they pay): 2048x512
-# 10.5 / 9.0, 2048x1024 15.3 / 15.4, 4096x1024 26.6 / 26.9 (calls of 20 steps 26.8 /
-# 26.5), 8192x2048 85 / 92; with a rim cylinder 8192x2048 64.5 / 82.2, 4096x1024
-# 21.5 / 26.8, cavity 1500x1300 13.4 (tiles 16.8)
+# and above which strips are, without a rim (with one wherever they pay):
+# 2048x512 10.5 / 9.0, 2048x1024 15.3 / 15.4, 4096x1024 26.6 / 26.9 (calls of 20
+# steps 26.8 / 26.5), 8192x2048 85 / 92; with a rim cylinder 8192x2048 64.5 /
+# 82.2, 4096x1024 21.5 / 26.8, cavity 1500x1300 13.4 (tiles 16.8)
 _PAIRS_STRIP_CELLS = 1 << 22
 # chunks of the strip sweep the GPU holds at once
 _STRIP_SLOTS = {8: 768, 4: 1536}
@@ -849,11 +849,11 @@ class D2Q9Engine:
     bitwise those of single steps), for 16-bit storage only when asked (its
     intermediate step stays in FP32, which changes the rounding).  Lattices
     large enough for the strip sweep take that instead, and small 16-bit ones
-    the tiled sweep, to the same bits (``_choose_sweep``).  Otherwise steps go through the strip sweep
-    on large lattices (d2q9_strip_steps) and the tiled sweep on others
-    (d2q9_tiled_steps), several steps per launch and bitwise single steps in
-    every storage form, or through single sweeps where the case cannot be
-    expressed in their tables or a solid moves.  ``sweep`` names the one that
+    the tiled sweep, to the same bits (``_choose_sweep``).  Otherwise steps go
+    through the strip sweep on large lattices (d2q9_strip_steps) and the tiled
+    sweep on others (d2q9_tiled_steps), several steps per launch and bitwise
+    single steps in every storage form, or through single sweeps where the
+    case cannot be expressed in their tables or a solid moves.  ``sweep`` names the one that
     runs; the attribute ``two_step`` says that the two-step sweep was chosen
     and deep tiles fit, also where the strips then take its place.
     """
